@@ -272,6 +272,8 @@ constexpr uint32_t kLeavesPerWave = SVDAG_LEAVES_PER_WAVE;
 constexpr uint32_t kLeafLanes = 64u / kLeavesPerWave; // lanes per leaf
 constexpr uint32_t kLeafWordsPerLane = (18u + kLeafLanes - 1u) / kLeafLanes; // a record has at most 18 words
 
+__device__ inline void dedup_clear(const WsDev& ws, uint32_t count, uint32_t tid, uint32_t stride);
+
 template <bool kMulti>
 __global__ void __launch_bounds__(256) svo_leaf_level(WsDev ws, DagDev dag, const EditorDev* eds)
 {
@@ -282,6 +284,8 @@ __global__ void __launch_bounds__(256) svo_leaf_level(WsDev ws, DagDev dag, cons
     const LevelDesc me = ws.lvl[dag.leafLevel];
     const uint32_t wavesPerBlock = blockDim.x / 64u;
     const uint32_t count = min(me.count, ws.capLeaf);
+    // The merge starts at this level: an empty dedup table for it.
+    dedup_clear(ws, count, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x);
     for (uint32_t i0 = (blockIdx.x * wavesPerBlock + wv) * kLeavesPerWave; i0 < count;
          i0 += gridDim.x * wavesPerBlock * kLeavesPerWave) {
         const uint32_t i = i0 + seg;
@@ -384,6 +388,23 @@ __global__ void __launch_bounds__(256) svo_leaf_level(WsDev ws, DagDev dag, cons
                 }
             }
         }
+        // Full leaf: all voxels set, every material word the first voxel's
+        // material repeated (leaf_is_full).
+        if (__ballot(mask == ~0ull) != 0ull) {
+            const uint32_t m0 = (uint32_t)__shfl((int)word[2u / kLeafLanes], (int)(seg * kLeafLanes + 2u % kLeafLanes), 64)
+                                & ((1u << dag.M) - 1u);
+            const uint32_t repw = dag.M == 4 ? m0 * 0x11111111u : m0 * 0x01010101u;
+            const uint32_t matWords = (64u * dag.M) / 32u;
+            bool off = mask != ~0ull;
+#pragma unroll
+            for (uint32_t k = 0; k < kLeafWordsPerLane; ++k) {
+                const uint32_t q = s + kLeafLanes * k;
+                off |= q >= 2u && q < 2u + matWords && word[k] != repw;
+            }
+            const uint64_t offs = __ballot(off);
+            if (valid && s == 0u && ((offs >> (kLeafLanes * seg)) & ((1ull << kLeafLanes) - 1ull)) == 0ull)
+                set_flag(kMulti ? &ws.edFull[ws.editOf[w] * kMaxLevels + dag.leafLevel] : &ws.lvl[dag.leafLevel].fullCount);
+        }
         const uint64_t diff = __ballot(differ);
         const bool unchanged = cmp && ((diff >> (kLeafLanes * seg)) & ((1ull << kLeafLanes) - 1ull)) == 0ull;
         if (valid && s == 0u) {
@@ -398,235 +419,427 @@ __global__ void __launch_bounds__(256) svo_leaf_level(WsDev ws, DagDev dag, cons
     }
 }
 
-// Bottom-up, per level: clear the level's dedup table; map SVO children to
-// DAG handles and drop empty ones (updateChildPointers,
-// my_gpu_hash_dag_edits.cu:44-95); flag full items when the level below had
-// any (discover_fully_filled, 96-150, gated at 337).  kMulti: the gate and
-// the full-item counts are per edit, and items of an edit that made no leaf
-// are emptied (that edit is dropped as a whole, :651).
+// The tables' descriptors in LDS: a lane's probe then waits for its record,
+// not for its record and then a descriptor.
+__device__ inline void tables_stage(TableDev* sTab, const DagDev& dag)
+{
+    const uint32_t* src = reinterpret_cast<const uint32_t*>(dag.tables);
+    uint32_t* dst = reinterpret_cast<uint32_t*>(sTab);
+    for (uint32_t i = threadIdx.x; i < dag.numTables * (sizeof(TableDev) / 4u); i += blockDim.x)
+        dst[i] = src[i];
+}
+
+__device__ inline void dedup_clear(const WsDev& ws, uint32_t count, uint32_t tid, uint32_t stride)
+{
+    const uint32_t cap = dedup_cap(count, ws.dedupCap);
+    ulonglong2* d = reinterpret_cast<ulonglong2*>(ws.dedup); // caps are even
+    for (uint32_t i = tid; i < cap / 2u; i += stride)
+        d[i] = make_ulonglong2(0ull, 0ull);
+}
+
+// Bottom-up, per level above the leaves: map SVO children to DAG handles and
+// drop empty ones (updateChildPointers, my_gpu_hash_dag_edits.cu:44-95); flag
+// full items when the level below had any (discover_fully_filled, 96-150,
+// gated at 337).  kMulti: the gate and the full-item counts are per edit, and
+// items of an edit that made no leaf are emptied (that edit is dropped as a
+// whole, :651).  The children's representatives, then their handles, are
+// loaded together: two dependent round trips for the item, not two per child.
+template <bool kMulti>
+__device__ inline void prepare_item(const WsDev& ws, const DagDev& dag, uint32_t L, uint32_t w, bool gateAll,
+                                    uint32_t childStart)
+{
+    uint32_t* rec = ws.nodes + (size_t)w * kNodeStride;
+    uint32_t r[kNodeStride];
+    lane_rec_load<(int)kNodeStride>(r, rec);
+    const uint32_t e = kMulti ? ws.editOf[w] : 0u;
+    const uint32_t mask = r[0] & 0xFFu;
+    if (mask == 0)
+        return;
+    const bool gate = kMulti ? ws.edFull[e * kMaxLevels + L + 1] != 0 : gateAll;
+    if (kMulti && ws.edCount[e * kMaxLevels + dag.leafLevel] == 0) {
+        rec[0] = 0u;
+        return;
+    }
+    const bool leafChildren = L + 1 == dag.leafLevel;
+    const uint32_t imask = header_payload(r[0], dag.M) & 0xFFu;
+    uint32_t rep[8], created[8], bit[8];
+    uint32_t m = mask;
+#pragma unroll
+    for (uint32_t k = 0; k < 8; ++k) {
+        bit[k] = m & (0u - m);
+        m ^= bit[k];
+        rep[k] = (imask & bit[k]) ? ws.rep[childStart + r[1 + k]] : kSentinel;
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < 8; ++k) {
+        created[k] = 0u;
+        if (imask & bit[k]) {
+            r[1 + k] = kSentinel;
+            if (rep[k] != kSentinel) {
+                r[1 + k] = ws.handle[rep[k]];
+                created[k] = ws.created[rep[k]]; // 1: inserted by this merge (2: unchanged leaf)
+            }
+        }
+    }
+    uint32_t newMask = 0, newChild = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < 8; ++k) {
+        newChild |= created[k] & 1u;
+        if (bit[k] && r[1 + k] != kSentinel)
+            newMask |= bit[k];
+    }
+    bool full = false;
+    uint32_t fm = 0;
+    if (gate && newMask == 0xFFu) {
+        // Full children of one material are usually one shared item.
+        full = true;
+#pragma unroll
+        for (uint32_t j = 0; j < 8; ++j) {
+            if (!full || (j > 0 && r[1 + j] == r[1]))
+                continue;
+            uint32_t cm = 0;
+            const bool f = leafChildren ? leaf_is_full(dag_leaf_ptr(dag, r[1 + j]), dag.M, cm)
+                                        : header_full(dag_node_ptr(dag, r[1 + j])[0], dag.M, cm);
+            if (j == 0)
+                fm = cm;
+            full = f && cm == fm;
+        }
+    }
+    r[0] = full ? header_make_full(0xFFu, fm, dag.M) : header_make(newMask, 0u, dag.M);
+    r[9] = newChild; // outside the item's words: equal items agree on it
+    if (newMask == mask) {
+        uint2* out = reinterpret_cast<uint2*>(rec);
+#pragma unroll
+        for (uint32_t k = 0; k < kNodeStride / 2u; ++k)
+            out[k] = make_uint2(r[2 * k], r[2 * k + 1]);
+    } else {
+        uint32_t n = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < 8; ++k)
+            if (bit[k] && r[1 + k] != kSentinel)
+                rec[1 + n++] = r[1 + k];
+        for (; n < 8; ++n)
+            rec[1 + n] = 0u;
+        rec[0] = r[0];
+        rec[9] = r[9];
+    }
+    if (full)
+        set_flag(kMulti ? &ws.edFull[e * kMaxLevels + L] : &ws.lvl[L].fullCount);
+}
+
 template <bool kMulti>
 __global__ void __launch_bounds__(256) merge_prepare(WsDev ws, DagDev dag, uint32_t L)
 {
     if (merge_skipped(ws, dag))
         return;
     const LevelDesc me = ws.lvl[L];
-    const uint32_t cap = dedup_cap(me.count, ws.dedupCap);
-    const uint32_t tid = blockIdx.x * blockDim.x + threadIdx.x;
+    const LevelDesc below = ws.lvl[L + 1];
     const uint32_t stride = gridDim.x * blockDim.x;
-    for (uint32_t i = tid; i < cap; i += stride)
-        ws.dedup[i] = 0ull;
-    if (L == dag.leafLevel) {
-        for (uint32_t i = tid; i < me.count; i += stride) {
-            uint32_t m;
-            if (leaf_is_full(ws.leaves + (size_t)i * ws.leafStride, dag.M, m))
-                set_flag(kMulti ? &ws.edFull[ws.editOf[me.start + i] * kMaxLevels + L] : &ws.lvl[L].fullCount);
-        }
-        return;
-    }
-    const bool gateAll = ws.lvl[L + 1].fullCount != 0;
-    const uint32_t childStart = ws.lvl[L + 1].start;
-    const bool leafChildren = L + 1 == dag.leafLevel;
-    for (uint32_t i = tid; i < me.count; i += stride) {
-        uint32_t* rec = ws.nodes + (size_t)(me.start + i) * kNodeStride;
-        const uint32_t e = kMulti ? ws.editOf[me.start + i] : 0u;
-        const bool gate = kMulti ? ws.edFull[e * kMaxLevels + L + 1] != 0 : gateAll;
-        const uint32_t hdr = rec[0];
-        const uint32_t mask = hdr & 0xFFu;
-        if (mask == 0)
-            continue;
-        if (kMulti && ws.edCount[e * kMaxLevels + dag.leafLevel] == 0) {
-            rec[0] = 0u;
-            continue;
-        }
-        const uint32_t imask = header_payload(hdr, dag.M) & 0xFFu;
-        uint32_t out[8];
-        uint32_t n = 0, newMask = 0, k = 0, newChild = 0;
-        for (uint32_t c = 0; c < 8; ++c) {
-            if (!((mask >> c) & 1u))
-                continue;
-            uint32_t h = rec[1 + k++];
-            if ((imask >> c) & 1u) {
-                const uint32_t r = ws.rep[childStart + h];
-                h = (r == kSentinel) ? kSentinel : ws.handle[r];
-                if (r != kSentinel)
-                    newChild |= ws.created[r] & 1u; // 1: inserted by this merge (2: unchanged leaf)
-            }
-            if (h != kSentinel) {
-                out[n++] = h;
-                newMask |= 1u << c;
-            }
-        }
-        bool full = false;
-        uint32_t fm = 0;
-        if (gate && newMask == 0xFFu) {
-            full = true;
-            for (uint32_t j = 0; j < 8 && full; ++j) {
-                uint32_t m = 0;
-                const bool f = leafChildren ? leaf_is_full(dag_leaf_ptr(dag, out[j]), dag.M, m)
-                                            : header_full(dag_node_ptr(dag, out[j])[0], dag.M, m);
-                if (j == 0)
-                    fm = m;
-                full = f && m == fm;
-            }
-        }
-        rec[0] = full ? header_make_full(0xFFu, fm, dag.M) : header_make(newMask, 0u, dag.M);
-        for (uint32_t j = 0; j < 8; ++j)
-            rec[1 + j] = j < n ? out[j] : 0u;
-        rec[9] = newChild; // outside the item's words: equal items agree on it
-        if (full)
-            set_flag(kMulti ? &ws.edFull[e * kMaxLevels + L] : &ws.lvl[L].fullCount);
-    }
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < me.count; i += stride)
+        prepare_item<kMulti>(ws, dag, L, me.start + i, below.fullCount != 0, below.start);
 }
 
 // Per level: collapse equal SVO items onto one representative through a
 // transient open-addressing table of (hash, index) keys -- contents are
 // compared in place, so no slot ever waits on another writer -- and look
 // each representative up in the DAG (insertDuplicates / findUnique1 /
-// findUnique2, my_gpu_hash_dag_edits.cu:164-246).
-template <int G>
-__global__ void __launch_bounds__(256) merge_dedup_find(WsDev ws, DagDev dag, uint32_t L)
+// findUnique2, my_gpu_hash_dag_edits.cu:164-246).  MW: words of a record
+// (the node stride, or the leaf stride).
+//
+// Bound: the dependent trips of one item (record, dedup slot, line, compare),
+// about 2 us each.  One lane per item puts a whole level in flight at once,
+// where 16 lanes per item took it in ten rounds: the leaf level of a 16-edit
+// wave at depth 15 went from 64 to 27 us, the deepest level of a depth-15
+// terrain build from 11 to 2.2 ms.  Its duplicates are in flight at once too
+// (a filled box makes tens of thousands of equal leaves) and would queue on
+// one word of the table before the first of them shows there (that level then
+// took 93 us): each block collapses its own items in LDS first, and only one
+// of each content goes to the table.
+constexpr uint32_t kMergeBlock = 256;
+
+// Lanes of a wave each item of a level gets (log2): the most, up to maxLanes,
+// that keeps the level within kMergeSpread blocks.  Only the first of them
+// works: a wave's time is its longest chain walk plus every slab allocation
+// of its lanes, so small levels are spread over more waves (a level of 1000
+// nodes inserts in 13 us at 16 lanes each, 27 us at one).  Spread further, a
+// level's blocks cost more than its waves gain: 256 edits at depth 15 took
+// 14.2-14.4 ms at 512 blocks, 14.4-14.5 at 2048, 15.3 with the whole grid.
+constexpr uint32_t kMergeSpread = 512;
+__device__ inline uint32_t merge_lanes_log2(uint32_t count, uint32_t maxLanes)
+{
+    const uint32_t most = min(gridDim.x, kMergeSpread) * kMergeBlock;
+    uint32_t lg = 0;
+    while ((2u << lg) <= maxLanes && ((uint64_t)count << (lg + 1u)) <= (uint64_t)most)
+        ++lg;
+    return lg;
+}
+
+template <bool kLeaf, int MW>
+__global__ void __launch_bounds__(kMergeBlock) merge_dedup_find(WsDev ws, DagDev dag, uint32_t L, uint32_t maxLanes)
 {
     if (merge_skipped(ws, dag))
         return;
+    __shared__ TableDev sTab[kRefTables];
+    __shared__ uint32_t sFirst[2 * kMergeBlock]; // 1 + the block's first item of a content, by hash
+    __shared__ uint32_t sHash[kMergeBlock], sRep[kMergeBlock];
     const LevelDesc me = ws.lvl[L];
-    const bool isLeaf = L == dag.leafLevel;
+    const uint32_t lg = merge_lanes_log2(me.count, maxLanes);
+    const uint32_t perBlock = kMergeBlock >> lg;
+    if (blockIdx.x * perBlock >= me.count)
+        return;
+    tables_stage(sTab, dag);
     const uint32_t capMask = dedup_cap(me.count, ws.dedupCap) - 1u;
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t gl = lane & (G - 1);
-    const uint32_t gbase = lane & ~(uint32_t)(G - 1);
-    const uint32_t groupsPerBlock = blockDim.x / G;
-    for (uint32_t i = blockIdx.x * groupsPerBlock + threadIdx.x / G; i < me.count; i += gridDim.x * groupsPerBlock) {
+    const uint32_t t = threadIdx.x >> lg;
+    const bool works = (threadIdx.x & ((1u << lg) - 1u)) == 0u;
+    for (uint32_t i0 = blockIdx.x * perBlock; i0 < me.count; i0 += gridDim.x * perBlock) {
+        const uint32_t i = i0 + t;
         const uint32_t w = me.start + i;
-        if (isLeaf && ws.created[w] == 2u)
-            continue; // unchanged leaf: rep and handle were set by svo_leaf_level
-        const uint32_t* rec = isLeaf ? ws.leaves + (size_t)i * ws.leafStride : ws.nodes + (size_t)w * kNodeStride;
-        const uint32_t w0 = rec[0], w1 = rec[1];
-        const bool empty = isLeaf ? (w0 == 0u && w1 == 0u) : ((w0 & 0xFFu) == 0u);
-        if (empty) {
-            if (gl == 0)
+        // unchanged leaf: rep and handle were set by svo_leaf_level
+        bool active = works && i < me.count && !(kLeaf && ws.created[w] == 2u);
+        uint32_t n[MW];
+        uint32_t s = 0, h = 0;
+        if (active) {
+            lane_rec_load<MW>(n, kLeaf ? ws.leaves + (size_t)i * MW : ws.nodes + (size_t)w * kNodeStride);
+            const bool empty = kLeaf ? (n[0] == 0u && n[1] == 0u) : ((n[0] & 0xFFu) == 0u);
+            if (empty) {
                 ws.rep[w] = kSentinel;
-            continue;
-        }
-        const uint32_t s = isLeaf ? leaf_size_from_words(w0, w1, dag.M) : node_size_from_header(w0);
-        Needle<G> n;
-        needle_load(n, rec, s, gl);
-        const uint32_t h = needle_hash(n, s, gl);
-        const unsigned long long key = ((unsigned long long)h << 32) | (unsigned long long)(w + 1u);
-        uint32_t p = mix32(h) & capMask;
-        uint32_t rep = w;
-        while (true) {
-            // Equal items share a slot: read first, so duplicates (common
-            // surface patterns occur thousands of times) resolve without
-            // queueing on one atomic; only an empty slot is claimed by CAS.
-            unsigned long long v = 0;
-            if (gl == 0) {
-                v = ld_filter64(&ws.dedup[p]);
-                if (v == 0ull)
-                    v = atomicCAS(&ws.dedup[p], 0ull, key);
+                active = false;
+            } else {
+                s = kLeaf ? leaf_size_from_words(n[0], n[1], dag.M) : node_size_from_header(n[0]);
+                h = lane_hash<MW>(n, s);
             }
-            const uint32_t vlo = group_bcast<G>((uint32_t)v, 0);
-            const uint32_t vhi = group_bcast<G>((uint32_t)(v >> 32), 0);
-            if (vlo == 0u && vhi == 0u)
-                break;
-            if (vhi == h) {
-                const uint32_t j = vlo - 1u;
-                const uint32_t* other = isLeaf ? ws.leaves + (size_t)(j - me.start) * ws.leafStride
-                                               : ws.nodes + (size_t)j * kNodeStride;
-                const bool eq = needle_equal_lane(n, other, s, gl);
-                if (group_ballot<G>(!eq, gbase) == 0) {
-                    rep = j;
+        }
+        // The item equals item j of the level (of this block or another).
+        auto same = [&](uint32_t j) {
+            uint32_t o[MW];
+            lane_rec_load<MW>(o, kLeaf ? ws.leaves + (size_t)j * MW : ws.nodes + (size_t)(me.start + j) * kNodeStride);
+            bool eq = true;
+#pragma unroll
+            for (int k = 0; k < MW; ++k)
+                eq &= (uint32_t)k >= s || o[k] == n[k];
+            return eq;
+        };
+        sFirst[threadIdx.x] = 0u;
+        sFirst[threadIdx.x + kMergeBlock] = 0u;
+        if (works)
+            sHash[t] = h;
+        __syncthreads();
+        const uint32_t mixed = mix32(h);
+        uint32_t first = t;
+        if (active) {
+            uint32_t p = (mixed >> 8) & (2 * kMergeBlock - 1u);
+            while (true) {
+                uint32_t v = __hip_atomic_load(&sFirst[p], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                if (v == 0u)
+                    v = atomicCAS(&sFirst[p], 0u, t + 1u);
+                if (v == 0u)
+                    break;
+                if (sHash[v - 1u] == h && same(i0 + v - 1u)) {
+                    first = v - 1u;
                     break;
                 }
+                p = (p + 1u) & (2 * kMergeBlock - 1u);
             }
-            p = (p + 1u) & capMask;
         }
-        if (gl == 0)
+        uint32_t rep = w;
+        if (active && first == t) {
+            const unsigned long long key = ((unsigned long long)h << 32) | (unsigned long long)(i + 1u);
+            uint32_t p = mixed & capMask;
+            while (true) {
+                // A cached load first; only an empty slot is claimed by CAS.
+                unsigned long long v = ld_filter64(&ws.dedup[p]);
+                if (v == 0ull)
+                    v = atomicCAS(&ws.dedup[p], 0ull, key);
+                if (v == 0ull)
+                    break;
+                if ((uint32_t)(v >> 32) == h && same((uint32_t)v - 1u)) {
+                    rep = me.start + (uint32_t)v - 1u;
+                    break;
+                }
+                p = (p + 1u) & capMask;
+            }
+            sRep[t] = rep;
+        }
+        __syncthreads();
+        if (active) {
+            if (first != t)
+                rep = sRep[first];
             ws.rep[w] = rep;
-        if (rep == w) {
-            // A node with a child this merge inserted is new: no find.
-            uint32_t r = kNotFound, hint = kNoSlab;
-            if (isLeaf || rec[9] == 0u)
-                r = table_find_group_hint<G>(dag.tables[s - 2], n, s, h, gl, gbase, hint);
-            if (gl == 0) {
-                ws.handle[w] = (r == kNotFound) ? kNotFound : (isLeaf ? leaf_handle(dag, r, s) : node_handle(r, s));
+            if (rep == w) {
+                // A node with a child this merge inserted is new: no find.
+                uint32_t r = kNotFound, hint = kNoSlab;
+                if (kLeaf || n[MW - 1] == 0u)
+                    r = lane_find_hint<MW>(sTab[s - 2], n, s, h, hint);
+                ws.handle[w] = (r == kNotFound) ? kNotFound : (kLeaf ? leaf_handle(dag, r, s) : node_handle(r, s));
                 ws.created[w] = 0;
                 ws.hint[w] = hint;
             }
         }
+        __syncthreads(); // sFirst, sHash and sRep are rewritten next iteration
     }
 }
 
 // Insert the representatives the DAG did not hold (insertUniqueInHashTableAsWarp,
 // my_gpu_hash_dag_edits.cu:248-280).  All contents are distinct, so inserts
-// never race on equal items, and no find runs in this kernel.
-template <int G>
-__global__ void __launch_bounds__(256) merge_insert(WsDev ws, DagDev dag, uint32_t L)
+// never race on equal items, and no find runs beside them except the one for
+// an equal item of another role.  Returns true when an item was inserted.
+//
+// Bound: dependent trips again (record, line, CAS, counts).  One lane per
+// item, as in the find: the leaf level of a 16-edit wave at depth 15 inserts
+// in 28 instead of 91 us, the level above in 38 instead of 92, the leaves of
+// a depth-15 terrain build in 0.36 instead of 7.3 ms.
+// The children's references are summed per block in LDS, under the child's
+// handle, and each child gets one update: a child that thousands of items
+// share would otherwise collect thousands of atomics before the first shows
+// in its count (a stream of 256 edits took 25 ms so, 15 with the sums).
+constexpr uint32_t kRefSlots = 2048; // 256 items have at most 2048 children
+template <uint32_t kSlots>
+struct BlockRefs {
+    uint32_t child[kSlots], add[kSlots];
+};
+
+__device__ inline uint32_t* child_count(const DagDev& dag, const TableDev* sTab, uint32_t c, uint8_t role)
+{
+    const bool leaf = role == kRoleParentOfLeaves;
+    const uint32_t s = leaf ? leaf_handle_size(dag, c) : node_handle_size(c);
+    return sTab[s - 2].refs + (leaf ? leaf_handle_ptr(dag, c) : node_handle_ptr(c));
+}
+
+template <uint32_t kSlots>
+__device__ inline void block_ref_add(BlockRefs<kSlots>& refs, uint32_t slotMask, const DagDev& dag,
+                                     const TableDev* sTab, uint32_t c, uint8_t role)
+{
+    uint32_t p = (c * 0x9E3779B1u) >> 21;
+    for (uint32_t tries = 0; tries < 8; ++tries) {
+        p &= slotMask;
+        uint32_t v = __hip_atomic_load(&refs.child[p], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (v == kSentinel)
+            v = atomicCAS(&refs.child[p], kSentinel, c);
+        if (v == kSentinel || v == c) {
+            atomicAdd(&refs.add[p], 1u);
+            return;
+        }
+        ++p;
+    }
+    uint32_t* cnt = child_count(dag, sTab, c, role);
+    if (ld_filter(cnt) < kStickyRefs)
+        atomicAdd(cnt, 1u);
+}
+
+template <bool kLeaf, int MW, uint32_t kSlots>
+__device__ inline bool insert_item(const WsDev& ws, const DagDev& dag, const TableDev* sTab, const LevelDesc& me,
+                                   uint32_t i, uint8_t role, BlockRefs<kSlots>& refs, uint32_t slotMask)
+{
+    const uint32_t w = me.start + i;
+    const uint32_t rep = ws.rep[w], found = ws.handle[w];
+    uint32_t hint = ws.hint[w];
+    const uint32_t old = ws.work[w].w;
+    const uint8_t created = kLeaf ? ws.created[w] : 0u;
+    // The record is read along with what decides whether it is needed.
+    uint32_t n[MW];
+    lane_rec_load<MW>(n, kLeaf ? ws.leaves + (size_t)i * MW : ws.nodes + (size_t)w * kNodeStride);
+    if (rep != w)
+        return false;
+    // A found node that lacks the role it is needed in counts as a miss
+    // (the reference-count rule in dag_internal.h).  A leaf the edit
+    // left unchanged (created 2) is the DAG's own leaf there: plain.
+    // The item the DAG holds at this position already has this position's
+    // role (unchanged leaves are that case too): no role load.
+    if (found != kNotFound) {
+        if (found == old)
+            return false;
+        if (kLeaf) {
+            if (created == 2u || sTab[leaf_handle_size(dag, found) - 2].roles[leaf_handle_ptr(dag, found)] == 0u)
+                return false;
+        } else if (sTab[node_handle_size(found) - 2].roles[node_handle_ptr(found)] & role) {
+            return false;
+        }
+    }
+    const uint32_t s = kLeaf ? leaf_size_from_words(n[0], n[1], dag.M) : node_size_from_header(n[0]);
+    const uint32_t h = lane_hash<MW>(n, s);
+    const TableDev& t = sTab[s - 2];
+    if (found != kNotFound) {
+        // An equal item stored with the right role may follow in the chain.
+        const uint32_t again = lane_find_hint<MW>(t, n, s, h, hint, kLeaf ? kRoleLeafUse : role);
+        if (again != kNotFound) {
+            ws.handle[w] = kLeaf ? leaf_handle(dag, again, s) : node_handle(again, s);
+            return false;
+        }
+    }
+    const uint32_t r = lane_insert<MW>(t, n, s, h, hint);
+    if (r == kNotFound) {
+        atomicOr(&ws.status->oom, 1u);
+        ws.handle[w] = kSentinel;
+        return false;
+    }
+    ws.handle[w] = kLeaf ? leaf_handle(dag, r, s) : node_handle(r, s);
+    ws.created[w] = 1;
+    t.roles[r] = kLeaf ? (uint8_t)0u : role;
+    if (!kLeaf) {
+#pragma unroll
+        for (uint32_t k = 0; k < 8; ++k)
+            if (k + 1u < s)
+                block_ref_add(refs, slotMask, dag, sTab, n[1 + k], role);
+    }
+    return true;
+}
+
+// Also clears the dedup table for the level above, which the next launches
+// fill.
+template <bool kLeaf, int MW>
+__global__ void __launch_bounds__(kMergeBlock) merge_insert(WsDev ws, DagDev dag, uint32_t L, uint32_t maxLanes)
 {
     if (merge_skipped(ws, dag))
         return;
     __shared__ uint32_t sInserted;
-    __shared__ RefArrays sRa;
+    __shared__ TableDev sTab[kRefTables];
+    __shared__ BlockRefs<kLeaf ? 1u : kRefSlots> sRefs;
+    const LevelDesc me = ws.lvl[L];
+    if (L > 0)
+        dedup_clear(ws, ws.lvl[L - 1].count, blockIdx.x * kMergeBlock + threadIdx.x, gridDim.x * kMergeBlock);
+    const uint32_t lg = merge_lanes_log2(me.count, maxLanes);
+    const uint32_t perBlock = kMergeBlock >> lg;
+    if (blockIdx.x * perBlock >= me.count)
+        return;
+    const uint32_t slotMask = (kRefSlots >> lg) - 1u;
     if (threadIdx.x == 0)
         sInserted = 0u;
-    ref_arrays_stage(sRa, dag);
-    __syncthreads();
-    const LevelDesc me = ws.lvl[L];
-    const bool isLeaf = L == dag.leafLevel;
-    const uint8_t role = isLeaf ? 0u : node_role(dag, L);
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t gl = lane & (G - 1);
-    const uint32_t gbase = lane & ~(uint32_t)(G - 1);
-    const uint32_t groupsPerBlock = blockDim.x / G;
-    for (uint32_t i = blockIdx.x * groupsPerBlock + threadIdx.x / G; i < me.count; i += gridDim.x * groupsPerBlock) {
-        const uint32_t w = me.start + i;
-        if (ws.rep[w] != w)
-            continue;
-        uint32_t hint = ws.hint[w];
-        const uint32_t found = ws.handle[w];
-        // A found node that lacks the role it is needed in counts as a miss
-        // (the reference-count rule in dag_internal.h).  A leaf the edit
-        // left unchanged (created 2) is the DAG's own leaf there: plain.
-        // The item the DAG holds at this position already has this position's
-        // role (unchanged leaves are that case too): no role load.
-        if (found != kNotFound) {
-            if (found == ws.work[w].w)
-                continue;
-            if (isLeaf) {
-                if (ws.created[w] == 2u
-                    || sRa.roles[leaf_handle_size(dag, found) - 2][leaf_handle_ptr(dag, found)] == 0u)
-                    continue;
-            } else if (sRa.roles[node_handle_size(found) - 2][node_handle_ptr(found)] & role) {
-                continue;
+    tables_stage(sTab, dag);
+    const uint8_t role = kLeaf ? (uint8_t)0u : node_role(dag, L);
+    for (uint32_t i0 = blockIdx.x * perBlock; i0 < me.count; i0 += gridDim.x * perBlock) {
+        if constexpr (!kLeaf)
+            for (uint32_t q = threadIdx.x; q <= slotMask; q += kMergeBlock) {
+                sRefs.child[q] = kSentinel;
+                sRefs.add[q] = 0u;
             }
-        }
-        const uint32_t* rec = isLeaf ? ws.leaves + (size_t)i * ws.leafStride : ws.nodes + (size_t)w * kNodeStride;
-        const uint32_t w0 = rec[0], w1 = rec[1];
-        const uint32_t s = isLeaf ? leaf_size_from_words(w0, w1, dag.M) : node_size_from_header(w0);
-        Needle<G> n;
-        needle_load(n, rec, s, gl);
-        const uint32_t h = needle_hash(n, s, gl);
-        if (found != kNotFound) {
-            // An equal item stored with the right role may follow in the chain.
-            const uint32_t again = table_find_group_hint<G>(dag.tables[s - 2], n, s, h, gl, gbase, hint,
-                                                            isLeaf ? kRoleLeafUse : role);
-            if (again != kNotFound) {
-                if (gl == 0)
-                    ws.handle[w] = isLeaf ? leaf_handle(dag, again, s) : node_handle(again, s);
-                continue;
+        __syncthreads();
+        const uint32_t i = i0 + (threadIdx.x >> lg);
+        const bool works = (threadIdx.x & ((1u << lg) - 1u)) == 0u;
+        const bool made = works && i < me.count && insert_item<kLeaf, MW>(ws, dag, sTab, me, i, role, sRefs, slotMask);
+        const unsigned long long b = __ballot(made);
+        if (b != 0ull && (threadIdx.x & 63u) == 0u)
+            atomicAdd(&sInserted, (uint32_t)__popcll(b));
+        __syncthreads();
+        if constexpr (!kLeaf) {
+            // Every count the thread updates is loaded before the first update.
+            constexpr uint32_t kPer = kRefSlots / kMergeBlock;
+            uint32_t* cnt[kPer];
+            uint32_t seen[kPer], add[kPer];
+#pragma unroll
+            for (uint32_t k = 0; k < kPer; ++k) {
+                const uint32_t q = k * kMergeBlock + threadIdx.x;
+                const uint32_t c = q <= slotMask ? sRefs.child[q] : kSentinel;
+                seen[k] = kStickyRefs;
+                if (c != kSentinel) {
+                    cnt[k] = child_count(dag, sTab, c, role);
+                    add[k] = sRefs.add[q];
+                    seen[k] = ld_filter(cnt[k]);
+                }
             }
-        }
-        const uint32_t r = table_insert_group<G>(dag.tables[s - 2], n, s, h, gl, gbase, hint);
-        if (r != kNotFound)
-            refs_on_insert(dag, sRa, n, s, r, role, gl);
-        if (gl == 0) {
-            if (r == kNotFound) {
-                atomicOr(&ws.status->oom, 1u);
-                ws.handle[w] = kSentinel;
-            } else {
-                ws.handle[w] = isLeaf ? leaf_handle(dag, r, s) : node_handle(r, s);
-                ws.created[w] = 1;
-                atomicAdd(&sInserted, 1u);
-            }
+#pragma unroll
+            for (uint32_t k = 0; k < kPer; ++k)
+                if (seen[k] < kStickyRefs)
+                    atomicAdd(cnt[k], add[k]);
         }
     }
     __syncthreads();
@@ -938,25 +1151,29 @@ static void launch_merge_level(svdag_ctx* ctx, const WsDev& ws, uint32_t L, uint
 {
     const DagDev& dag = ctx->dag;
     const hipStream_t st = ctx->stream;
-    merge_prepare<kMulti><<<grid_for(2 * items, 256, kCap), 256, 0, st>>>(ws, dag, L);
-    const uint32_t G = ctx->groupSize;
-    const uint32_t gridG = grid_for(items, 256 / G, kCap);
-    switch (G) {
+    const uint32_t grid = grid_for(items, 256, kCap);
+    // Small levels: several lanes per item (merge_lanes_log2).
+    const uint32_t lanes = ctx->groupSize;
+    const uint32_t gridM = std::max(grid, grid_for(items * lanes, kMergeBlock, std::min(kCap, kMergeSpread)));
+    if (L < dag.leafLevel) {
+        merge_prepare<kMulti><<<grid, 256, 0, st>>>(ws, dag, L);
+        merge_dedup_find<false, (int)kNodeStride><<<gridM, 256, 0, st>>>(ws, dag, L, lanes);
+        merge_insert<false, (int)kNodeStride><<<gridM, 256, 0, st>>>(ws, dag, L, lanes);
+        return;
+    }
+    // The leaf record's words: 2, 10 or 18 (dag.maxLeafWords).
+    switch (dag.M) {
+    case 0:
+        merge_dedup_find<true, 2><<<gridM, 256, 0, st>>>(ws, dag, L, lanes);
+        merge_insert<true, 2><<<gridM, 256, 0, st>>>(ws, dag, L, lanes);
+        break;
     case 4:
-        merge_dedup_find<4><<<gridG, 256, 0, st>>>(ws, dag, L);
-        merge_insert<4><<<gridG, 256, 0, st>>>(ws, dag, L);
-        break;
-    case 8:
-        merge_dedup_find<8><<<gridG, 256, 0, st>>>(ws, dag, L);
-        merge_insert<8><<<gridG, 256, 0, st>>>(ws, dag, L);
-        break;
-    case 32:
-        merge_dedup_find<32><<<gridG, 256, 0, st>>>(ws, dag, L);
-        merge_insert<32><<<gridG, 256, 0, st>>>(ws, dag, L);
+        merge_dedup_find<true, 10><<<gridM, 256, 0, st>>>(ws, dag, L, lanes);
+        merge_insert<true, 10><<<gridM, 256, 0, st>>>(ws, dag, L, lanes);
         break;
     default:
-        merge_dedup_find<16><<<gridG, 256, 0, st>>>(ws, dag, L);
-        merge_insert<16><<<gridG, 256, 0, st>>>(ws, dag, L);
+        merge_dedup_find<true, 18><<<gridM, 256, 0, st>>>(ws, dag, L, lanes);
+        merge_insert<true, 18><<<gridM, 256, 0, st>>>(ws, dag, L, lanes);
         break;
     }
 }

@@ -566,6 +566,148 @@ __device__ inline uint32_t table_insert_lane(const TableDev& t, const uint32_t* 
     }
 }
 
+// ---------------------------------------------------------------- one lane per item, words in registers
+// An SVO record (or leaf record) of MW words, 8-byte aligned, into registers.
+template <int MW>
+__device__ inline void lane_rec_load(uint32_t (&w)[MW], const uint32_t* rec)
+{
+    static_assert(MW % 2 == 0, "records are read in word pairs");
+    const uint2* p = reinterpret_cast<const uint2*>(rec);
+#pragma unroll
+    for (int k = 0; k < MW / 2; ++k) {
+        const uint2 v = p[k];
+        w[2 * k] = v.x;
+        w[2 * k + 1] = v.y;
+    }
+}
+template <int MW>
+__device__ inline uint32_t lane_hash(const uint32_t (&w)[MW], uint32_t s)
+{
+    uint32_t h = 0;
+#pragma unroll
+    for (int j = 0; j < MW; ++j)
+        if ((uint32_t)j < s)
+            h ^= hash_part(w[j], (uint32_t)j);
+    return h;
+}
+// The first s words of an item equal w's: all of them are loaded at once, so
+// a compare costs one round trip.
+template <int MW>
+__device__ inline bool lane_item_equal(const uint32_t (&w)[MW], const uint32_t* item, uint32_t s)
+{
+    uint32_t v[MW];
+#pragma unroll
+    for (int k = 0; k < MW; ++k)
+        v[k] = (uint32_t)k < s ? item[k] : 0u;
+    bool eq = true;
+#pragma unroll
+    for (int k = 0; k < MW; ++k)
+        eq &= (uint32_t)k >= s || v[k] == w[k];
+    return eq;
+}
+
+// table_find_group_hint for one lane.
+template <int MW>
+__device__ inline uint32_t lane_find_hint(const TableDev& t, const uint32_t (&w)[MW], uint32_t s, uint32_t h,
+                                          uint32_t& hint, uint8_t role = 0)
+{
+    const uint32_t tag4 = make_tag(h) * 0x01010101u;
+    uint32_t slab = h % t.numBuckets;
+    hint = kNoSlab;
+    while (true) {
+        LineHead L;
+        line_head_load(L, t.lines + (size_t)slab * kLineWords, t.tagWords);
+        uint32_t cand = line_match(t, L, tag4);
+        while (cand) {
+            const uint32_t slot = __ffs(cand) - 1u;
+            cand &= cand - 1u;
+            if (lane_item_equal<MW>(w, line_item(t, slab, slot), s)) {
+                const uint32_t ptr = (slab << kSlotBits) | slot;
+                if (role == 0 || (role == kRoleLeafUse ? t.roles[ptr] == 0 : (t.roles[ptr] & role) != 0))
+                    return ptr;
+            }
+        }
+        uint32_t emp;
+        if (hint == kNoSlab && line_empty(t, L.tag, emp))
+            hint = slab;
+        if (L.next >= kPendingSlab) {
+            if (hint == kNoSlab)
+                hint = slab;
+            return kNotFound;
+        }
+        slab = L.next;
+    }
+}
+
+// table_insert_group for one lane.  Lanes of a wave insert side by side, and
+// whatever they do differently the wave does one after the other, so a step
+// is the same for all: one CAS, on a tag word (a free slot seen) or on the
+// tail's link (none), then the slabs for the links that were claimed, then
+// the next line's head.  The head is read with plain loads: tags only gain
+// slots and a link is set once while inserts run, so an old value only makes
+// the CAS fail, and the CAS brings the current one.
+template <int MW>
+__device__ inline uint32_t lane_insert(const TableDev& t, const uint32_t (&w)[MW], uint32_t s, uint32_t h,
+                                       uint32_t start = kNoSlab)
+{
+    const uint32_t tag = make_tag(h);
+    uint32_t slab = start == kNoSlab ? h % t.numBuckets : start;
+    LineHead L;
+    line_head_load(L, t.lines + (size_t)slab * kLineWords, t.tagWords);
+    while (true) {
+        uint32_t* line = t.lines + (size_t)slab * kLineWords;
+        uint32_t emp;
+        const bool room = line_empty(t, L.tag, emp);
+        if (room || L.next == kNoSlab) {
+            const uint32_t bit = room ? __ffs(emp) - 1u : 0u;
+            const uint32_t j = room ? bit >> 2 : t.tagWords;
+            uint32_t old = kNoSlab, want = kPendingSlab;
+            if (room) {
+#pragma unroll
+                for (uint32_t q = 0; q < 4; ++q)
+                    if (q == j)
+                        old = L.tag[q];
+                want = old | (tag << (8u * (bit & 3u)));
+            }
+            const uint32_t got = atomicCAS(line + j, old, want);
+            if (room) {
+                if (got == old) {
+                    uint32_t* item = line + t.tagWords + 1u + bit * s;
+#pragma unroll
+                    for (int k = 0; k < MW; ++k)
+                        if ((uint32_t)k < s)
+                            item[k] = w[k];
+                    return (slab << kSlotBits) | bit;
+                }
+#pragma unroll
+                for (uint32_t q = 0; q < 4; ++q)
+                    if (q == j)
+                        L.tag[q] = got;
+            } else if (got < kPendingSlab) {
+                L.next = got; // else: the link is still being set, ask again
+            }
+            // Claimed links get their slabs together; a new line is empty.
+            const bool mine = !room && got == kNoSlab;
+            if (__ballot(mine) != 0ull) {
+                const uint32_t id = wave_slab_alloc(t, mine);
+                if (mine) {
+                    st_relaxed(line + t.tagWords, id);
+                    if (id == kNoSlab)
+                        return kNotFound;
+                    slab = id;
+                    L = LineHead { { 0u, 0u, 0u, 0u }, kNoSlab };
+                }
+            }
+        } else if (L.next == kPendingSlab) {
+            L.next = kNoSlab; // a head read while its link was being set: the CAS asks
+        }
+        if (!room && L.next < kPendingSlab) {
+            slab = L.next;
+            line_head_load(L, t.lines + (size_t)slab * kLineWords, t.tagWords);
+        }
+    }
+}
+
 // ---------------------------------------------------------------- DAG encoding
 struct DagDev {
     const TableDev* tables;   // [numTables], index = item words - 2

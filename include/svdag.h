@@ -119,7 +119,7 @@ typedef struct {
     uint32_t material_bits;    /* 0, 4 or 8 (reference HASH_DAG_MATERIAL_BITS) */
     uint32_t load_factor;      /* percent of each bucket's head-line slots filled at expected_items (0 = 75;
                                   replaces the reference's TARGET_LOAD_FACTOR=96 items per 32-slot bucket) */
-    uint32_t group_size;       /* lanes per item in DAG find/insert: 0 = default, 1, 4, 8, 16, 32 */
+    uint32_t group_size;       /* most lanes of a wave an item of a small level gets in the merge's find / insert: 0 = default (16), 4, 8, 16, 32 */
     uint64_t expected_items;   /* expected DAG items, sizes the bucket count (0 = 1<<20) */
     uint64_t arena_slabs;      /* overflow slab reserve per table (0 = buckets/2 + 4096) */
     uint64_t workspace_items;  /* edit workspace capacity in work items (0 = 1<<22) */
@@ -262,8 +262,8 @@ int svdag_set_batch_mode(svdag_ctx* ctx, uint32_t mode);
 
 /* Autotuner (no reference counterpart; the reference fixes warp-cooperative
  * probing at compile time).  Times a sample batch under each lanes-per-item
- * choice for the merge kernels (4, 8, 16, 32) and keeps the fastest for the
- * context.  The sample runs once untimed first; after every run the root is
+ * choice for the merge kernels (4, 8, 16, 32: the most an item of a small
+ * level gets; large levels use one) and keeps the fastest for the context.  The sample runs once untimed first; after every run the root is
  * restored and a garbage collection frees what the sample inserted, so each
  * timed run inserts its items as a real edit would and the DAG's contents
  * do not change.  Like svdag_gc, this clears the undo / redo history. */

@@ -1,0 +1,57 @@
+"""The merge kernels (one lane per item, LDS collapse of duplicates, LDS sums
+of child references) at the sizes where they change behaviour: levels of less
+than a block, several blocks, chains that grow, contents that repeat."""
+import numpy as np
+import pytest
+
+import oracle_py
+import svdag_py
+
+
+def _noise(side, rng, fill, mats):
+    vox = np.full((side,) * 3, 0xFF, np.uint8)
+    pick = rng.uniform(size=(side,) * 3) < fill
+    vox[pick] = rng.choice(mats, int(pick.sum()))
+    return vox
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bits,lanes,grid_log2,pattern", [
+    (0, 4, 4, "noise"), (4, 32, 5, "noise"), (8, 0, 6, "noise"),
+    (0, 0, 6, "noise"), (4, 0, 7, "repeat"), (8, 16, 6, "repeat"), (4, 8, 2, "noise")])
+def test_merge_matches_oracle_and_counts_references(bits, lanes, grid_log2, pattern):
+    levels, side = 8, 1 << grid_log2
+    rng = np.random.default_rng(100 * bits + 10 * grid_log2 + lanes)
+    mats = [0] if bits == 0 else list(range(1, min(15, (1 << bits) - 2)))
+    if pattern == "noise":
+        vox = _noise(side, rng, 0.3, mats)
+    else:  # sixteen different bricks over and over
+        bricks = [_noise(8, rng, 0.4, mats) for _ in range(16)]
+        vox = np.empty((side,) * 3, np.uint8)
+        for x in range(0, side, 8):
+            for y in range(0, side, 8):
+                for z in range(0, side, 8):
+                    vox[x:x + 8, y:y + 8, z:z + 8] = bricks[rng.integers(16)]
+    # Tables of 64 buckets: chains grow while the level is inserted.
+    g = svdag_py.MyGPUHashDAG(levels, bits, group_size=lanes, expected_items=64, arena_slabs=1 << 17)
+    o = oracle_py.OracleDag(levels, bits)
+    print(f"[case] merge bits={bits} lanes={lanes} side={side} {pattern}", flush=True)
+    g.build_voxels(vox)
+    full = np.full((1 << levels,) * 3, 0xFF, np.uint8)
+    full[:side, :side, :side] = vox
+    oracle_py.build_dense(o, full)
+    assert g.canonical() == o.canonical()
+    edits = [(svdag_py.BOX_ADD, mats[0], (100.0, 90.0, 120.0), 37.0), (svdag_py.SPHERE_ADD, mats[-1], (60.0, 60.0, 60.0), 30.0),
+             (svdag_py.BOX_REMOVE, 0, (110.0, 90.0, 100.0), 9.0), (svdag_py.PAINT, mats[-1], (100.0, 70.0, 120.0), 25.0)]
+    g.edit_batch(edits)
+    for kind, mat, c, r in edits:
+        o.edit(kind, mat, c, r)
+    assert g.canonical() == o.canonical()
+    # A marking collection right after a counting one frees nothing: the
+    # counts the merge kept are those of the stored items.
+    counted = g.garbage_collect()
+    marked = g.garbage_collect(mark=True)
+    assert counted.marked == 0 and marked.items_freed == 0
+    assert counted.items_live == marked.items_live
+    assert g.canonical() == o.canonical()
+    g.close()
