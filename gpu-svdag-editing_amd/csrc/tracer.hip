@@ -113,8 +113,8 @@ __device__ inline uint32_t intersection_mask(uint32_t shift, uint32_t px, uint32
 //     address, child mask, children left), sized by the DAG's depth: 22 waves
 //     per CU at depth 15.  A bit per level says where children are left, so
 //     going up reads one entry, not one per level.
-//   - The item address needs the table's base only (staged in LDS); the rest
-//     of its layout follows from the item size.
+//   - An item's address takes one LDS read after its handle, and lanes at
+//     nodes and lanes at leaves load theirs together.
 // Measured against the walk with 16x16 tiles and a 20-level stack per block
 // of 256: primary 1920x1080 at depth 15 1.354 -> 0.644 ms; at depth 13 and
 // 1280x720 shadows 0.616 -> 0.298, occlusion at 3 samples 0.548 -> 0.243 ms;
@@ -122,31 +122,42 @@ __device__ inline uint32_t intersection_mask(uint32_t shift, uint32_t px, uint32
 constexpr uint32_t kTile = 8;
 constexpr uint32_t kTraceBlock = kTile * kTile;
 
+// Per item size: the address of slot 0 of line 0, and the slot bits of a
+// handle index.
 struct TraceShared {
-    const uint32_t* lines[kRefTables]; // line arrays of the tables
+    uint4 table[kRefTables];
 };
 __device__ inline void trace_stage(TraceShared& sh, const DagDev& dag)
 {
-    if (threadIdx.x < dag.numTables)
-        sh.lines[threadIdx.x] = dag.tables[threadIdx.x].lines;
+    if (threadIdx.x < dag.numTables) {
+        const TableDev& t = dag.tables[threadIdx.x];
+        const uint64_t at = (uint64_t)(uintptr_t)(t.lines + t.tagWords + 1u);
+        sh.table[threadIdx.x] = make_uint4((uint32_t)at, (uint32_t)(at >> 32), slot_code_bits(t.itemWords), 0u);
+    }
     __syncthreads();
 }
-// First item word of a line of s-word items (line_tag_words(line_slots(s)) + 1).
-__device__ inline uint32_t item_base(uint32_t s)
+// How a handle's bits split: size = minWords + (h >> 1 >> sizeShift), the
+// index below.  Nodes and leaves differ only in these numbers, so lanes that
+// reach nodes and lanes that reach leaves decode and load together.
+struct HandleBits {
+    uint32_t sizeShift, indexMask, minWords;
+};
+__device__ inline HandleBits node_bits()
 {
-    return s <= 5u ? (s <= 3u ? 7u - s : 3u) : 2u;
+    return { 31u - kNodeSizeBits, (1u << (32u - kNodeSizeBits)) - 1u, 2u };
 }
-__device__ inline const uint32_t* item_address(const TraceShared& sh, uint32_t ptr, uint32_t s)
+__device__ inline HandleBits leaf_bits(const DagDev& dag)
 {
-    return sh.lines[s - 2u] + (size_t)(ptr >> kSlotBits) * kLineWords + (item_base(s) + (ptr & (kMaxSlots - 1u)) * s);
+    return { 31u - dag.leafSizeBits, ~0u >> dag.leafSizeBits, dag.minLeafWords };
 }
-__device__ inline const uint32_t* walk_node(const TraceShared& sh, uint32_t h)
+__device__ inline const uint32_t* item_address(const TraceShared& sh, const HandleBits& hb, uint32_t h)
 {
-    return item_address(sh, node_handle_ptr(h), node_handle_size(h));
-}
-__device__ inline const uint32_t* walk_leaf(const TraceShared& sh, const DagDev& dag, uint32_t h)
-{
-    return item_address(sh, leaf_handle_ptr(dag, h), leaf_handle_size(dag, h));
+    const uint32_t s = hb.minWords + ((h >> 1) >> hb.sizeShift);
+    const uint32_t idx = h & hb.indexMask;
+    const uint4 t = sh.table[s - 2u];
+    const uint32_t slot = idx & ((1u << t.z) - 1u);
+    const uint64_t base = (uint64_t)t.x | ((uint64_t)t.y << 32);
+    return reinterpret_cast<const uint32_t*>(base + (uint64_t)(idx >> t.z) * (kLineWords * 4u) + slot * s * 4u);
 }
 
 // Child mask bit c moves to bit c ^ order: the children in visit order.
@@ -182,7 +193,8 @@ __device__ inline bool walk(const DagDev& dag, const TraceShared& sh, uint32_t r
 {
     const uint32_t levels = dag.levels, leafLevel = dag.leafLevel;
     const ChildOrder co(ray);
-    const uint32_t* node = walk_node(sh, root);
+    const HandleBits nb = node_bits(), lb = leaf_bits(dag);
+    const uint32_t* node = item_address(sh, nb, root);
     uint32_t child = node[0] & 0xFFu;
     uint32_t left = co.sort(child & intersection_mask<true, kTame>(levels, 0, 0, 0, ray));
     uint32_t level = 0, pending = 0;
@@ -220,19 +232,22 @@ __device__ inline bool walk(const DagDev& dag, const TraceShared& sh, uint32_t r
         z |= (nc & 1u) << shift;
         if (level <= leafLevel) {
             const uint32_t h = node[1 + __builtin_popcount(child & ((1u << nc) - 1u))];
-            if (level < leafLevel) {
-                node = walk_node(sh, h);
-                const uint32_t hdr = node[0];
-                child = hdr & 0xFFu;
-                if (kAny && (hdr & 0x100u))
-                    return true;
-            } else {
-                leaf = walk_leaf(sh, dag, h);
-                leafLo = leaf[0];
-                leafHi = leaf[1];
+            const bool isLeaf = level == leafLevel;
+            const HandleBits hb { isLeaf ? lb.sizeShift : nb.sizeShift, isLeaf ? lb.indexMask : nb.indexMask,
+                                  isLeaf ? lb.minWords : nb.minWords };
+            const uint32_t* item = item_address(sh, hb, h);
+            const uint32_t w0 = item[0], w1 = item[1]; // an item has at least two words
+            if (isLeaf) {
+                leaf = item;
+                leafLo = w0;
+                leafHi = w1;
                 // a bit per byte that holds a voxel
-                child = compact_bytes(~zero_bytes(leafLo) & 0x80808080u)
-                    | (compact_bytes(~zero_bytes(leafHi) & 0x80808080u) << 4);
+                child = compact_bytes(~zero_bytes(w0) & 0x80808080u) | (compact_bytes(~zero_bytes(w1) & 0x80808080u) << 4);
+            } else {
+                node = item;
+                child = w0 & 0xFFu;
+                if (kAny && (w0 & 0x100u))
+                    return true;
             }
         } else {
             child = ((nc & 4u ? leafHi : leafLo) >> (8u * (nc & 3u))) & 0xFFu;
