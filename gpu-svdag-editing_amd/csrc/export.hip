@@ -376,7 +376,7 @@ static int insert_level(svdag_ctx* ctx, const std::vector<std::vector<uint32_t>>
         SVDAG_HIP(hipMalloc(&dout, order.size() * 4));
         fr.p.push_back(dout);
         SVDAG_HIP(hipMemcpy(dw, words.data(), words.size() * 4, hipMemcpyHostToDevice));
-        SVDAG_TRY(launch_bulk(ctx->ts, dw, segs.data(), (uint32_t)segs.size(), dout, 16, insert, ctx->stream, segBuf,
+        SVDAG_TRY(launch_bulk(ctx->ts, dw, segs.data(), (uint32_t)segs.size(), dout, insert ? 16 : 1, insert, ctx->stream, segBuf,
                               nullptr));
         std::vector<uint32_t> out(order.size());
         SVDAG_HIP(hipMemcpyAsync(out.data(), dout, out.size() * 4, hipMemcpyDeviceToHost, ctx->stream));

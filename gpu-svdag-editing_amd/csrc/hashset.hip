@@ -169,9 +169,10 @@ __device__ inline uint32_t seg_of(const uint32_t* segs, uint32_t nseg, uint32_t 
     return s;
 }
 
-template <int G, bool kInsert, int MW>
-__global__ void __launch_bounds__(256) bulk_group_kernel(const TableDev* tables, uint32_t minWords, const uint32_t* words,
-                                                         const uint32_t* segs, uint32_t nseg, uint32_t total, uint32_t* out)
+template <int G, int MW>
+__global__ void __launch_bounds__(256) bulk_find_group_kernel(const TableDev* tables, uint32_t minWords,
+                                                              const uint32_t* words, const uint32_t* segs,
+                                                              uint32_t nseg, uint32_t total, uint32_t* out)
 {
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t gl = lane & (G - 1);
@@ -185,11 +186,7 @@ __global__ void __launch_bounds__(256) bulk_group_kernel(const TableDev* tables,
         Needle<G, MW> n;
         needle_load(n, words + segs[sg * 5 + 2] + (size_t)local * s, s, gl);
         const uint32_t h = needle_hash(n, s, gl);
-        uint32_t r;
-        if constexpr (kInsert)
-            r = table_insert_group<G>(t, n, s, h, gl, gbase);
-        else
-            r = table_find_group<G>(t, n, s, h, gl, gbase);
+        const uint32_t r = table_find_group<G>(t, n, s, h, gl, gbase);
         if (gl == 0)
             out[segs[sg * 5 + 3] + local] = r;
     }
@@ -244,9 +241,9 @@ __global__ void __launch_bounds__(256) bulk_find_multi_kernel(const TableDev* ta
     }
 }
 
-template <bool kInsert>
-__global__ void __launch_bounds__(256) bulk_lane_kernel(const TableDev* tables, uint32_t minWords, const uint32_t* words,
-                                                        const uint32_t* segs, uint32_t nseg, uint32_t total, uint32_t* out)
+__global__ void __launch_bounds__(256) bulk_find_lane_kernel(const TableDev* tables, uint32_t minWords,
+                                                             const uint32_t* words, const uint32_t* segs,
+                                                             uint32_t nseg, uint32_t total, uint32_t* out)
 {
     for (uint32_t idx = blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += gridDim.x * blockDim.x) {
         const uint32_t sg = seg_of(segs, nseg, idx);
@@ -257,7 +254,7 @@ __global__ void __launch_bounds__(256) bulk_lane_kernel(const TableDev* tables, 
         uint32_t h = 0;
         for (uint32_t j = 0; j < s; ++j)
             h ^= hash_part(p[j], j);
-        out[segs[sg * 5 + 3] + local] = kInsert ? table_insert_lane(t, p, s, h) : table_find_lane(t, p, s, h);
+        out[segs[sg * 5 + 3] + local] = table_find_lane(t, p, s, h);
     }
 }
 
@@ -496,6 +493,33 @@ __global__ void __launch_bounds__(256) find_lanes_seg(const TableDev* tables, co
     }
 }
 
+// Bulk insert, one lane per item, blocks assigned to segments as above.
+// Bound: an item's trips (words, line head, tag CAS), all of a wave's in
+// flight at once, and the CAS rate.  One lane per item for every variant: the
+// groups of 4 to 32 lanes used to share these trips without shortening them,
+// and held 64 / G items per wave.  2^24 items of 2-9 words at 75% fill: 6.37
+// (16 lanes each) -> 2.40 ms; 4 M items of 2-18 words: 2.5 -> 0.73 ms.  What
+// bounds it now is the allocation counter of the overflow lines.
+template <int MW>
+__global__ void __launch_bounds__(256) insert_lanes_seg(const TableDev* tables, const uint32_t* words, LaneSegs a,
+                                                        uint32_t* out)
+{
+    uint32_t sg = 0;
+    while (sg + 1 < a.n && blockIdx.x >= a.blockStart[sg + 1])
+        ++sg;
+    const uint32_t s = a.s[sg];
+    const TableDev t = tables[s - a.minWords];
+    const uint32_t idx = (blockIdx.x - a.blockStart[sg]) * 256u + threadIdx.x;
+    if (idx >= a.count[sg])
+        return;
+    const uint32_t* nd = words + a.wordOff[sg] + (size_t)idx * s;
+    uint32_t w[MW];
+#pragma unroll
+    for (int j = 0; j < MW; ++j)
+        w[j] = (uint32_t)j < s ? nd[j] : 0u;
+    out[a.outOff[sg] + idx] = lane_insert<MW>(t, w, s, lane_hash<MW>(w, s));
+}
+
 // Copy the words of n items (pointers already validated on the host).
 __global__ void gather_items(TableDev t, const uint32_t* ptrs, uint32_t n, uint32_t* out)
 {
@@ -592,6 +616,25 @@ static int launch_binned(const TableSet& ts, const uint32_t* words, const svdag_
     return SVDAG_OK;
 }
 
+// Segments as kernel arguments, perBlock items to a block.
+static LaneSegs lane_segs(const TableSet& ts, const svdag_segment* segs, uint32_t n, uint32_t perBlock)
+{
+    LaneSegs a {};
+    a.n = n;
+    a.minWords = ts.minWords;
+    uint64_t blocks = 0;
+    for (uint32_t i = 0; i < n; ++i) {
+        a.s[i] = segs[i].item_words;
+        a.count[i] = segs[i].count;
+        a.wordOff[i] = segs[i].word_offset;
+        a.outOff[i] = segs[i].out_offset;
+        a.blockStart[i] = (uint32_t)blocks;
+        blocks += ((uint64_t)segs[i].count + perBlock - 1) / perBlock;
+    }
+    a.blockStart[n] = (uint32_t)blocks;
+    return a;
+}
+
 int launch_bulk(const TableSet& ts,const uint32_t* words, const svdag_segment* segs, uint32_t nseg, uint32_t* out,
                 int variant, bool insert, hipStream_t stream, uint32_t* segBuf, BinScratch* bins, hipEvent_t ev0,
                 hipEvent_t ev1)
@@ -628,9 +671,9 @@ int launch_bulk(const TableSet& ts,const uint32_t* words, const svdag_segment* s
         set_error("too many items");
         return SVDAG_E_INVALID;
     }
-    // The segment-uniform lane variants (1, 2, 3) take their segments as
-    // kernel arguments; the others read them from segBuf.
-    if (!(variant >= 1 && variant <= 3))
+    // Inserts and the segment-uniform lane variants (1, 2, 3) take their
+    // segments as kernel arguments; the others read them from segBuf.
+    if (!insert && !(variant >= 1 && variant <= 3))
         SVDAG_HIP(hipMemcpyAsync(segBuf, host, nseg * 5 * 4, hipMemcpyHostToDevice, stream));
     const uint32_t n = (uint32_t)total;
     if (n == 0)
@@ -653,27 +696,16 @@ int launch_bulk(const TableSet& ts,const uint32_t* words, const svdag_segment* s
             return SVDAG_E_INVALID;
         }
         const int npl = variant == 1 ? 1 : (variant == 2 ? 2 : 4);
-        LaneSegs a {};
-        a.n = nseg;
-        a.minWords = ts.minWords;
-        uint64_t blocks = 0;
-        for (uint32_t i = 0; i < nseg; ++i) {
-            a.s[i] = segs[i].item_words;
-            a.count[i] = segs[i].count;
-            a.wordOff[i] = segs[i].word_offset;
-            a.outOff[i] = segs[i].out_offset;
-            a.blockStart[i] = (uint32_t)blocks;
-            blocks += ((uint64_t)segs[i].count + 256u * npl - 1) / (256u * npl);
-        }
-        a.blockStart[nseg] = (uint32_t)blocks;
+        const LaneSegs a = lane_segs(ts, segs, nseg, 256u * npl);
+        const uint32_t blocks = a.blockStart[nseg];
         if (ev0)
             SVDAG_HIP(hipEventRecord(ev0, stream));
         const bool narrowItems = ts.maxWords <= 10;
 #define SVDAG_LANE_SEG(NPL)                                                                                  \
         if (narrowItems)                                                                                     \
-            find_lanes_seg<NPL, 10><<<(uint32_t)blocks, block, 0, stream>>>(ts.devTables, words, a, out);    \
+            find_lanes_seg<NPL, 10><<<blocks, block, 0, stream>>>(ts.devTables, words, a, out);    \
         else                                                                                                 \
-            find_lanes_seg<NPL, 18><<<(uint32_t)blocks, block, 0, stream>>>(ts.devTables, words, a, out);
+            find_lanes_seg<NPL, 18><<<blocks, block, 0, stream>>>(ts.devTables, words, a, out);
         if (npl == 1) {
             SVDAG_LANE_SEG(1)
         } else if (npl == 2) {
@@ -687,29 +719,42 @@ int launch_bulk(const TableSet& ts,const uint32_t* words, const svdag_segment* s
         SVDAG_HIP(hipGetLastError());
         return SVDAG_OK;
     }
+    if (insert && (variant == 204 || variant == 404 || variant == 208 || variant == 408)) {
+        set_error("multi-needle variants are find-only");
+        return SVDAG_E_INVALID;
+    }
     if (ev0)
         SVDAG_HIP(hipEventRecord(ev0, stream));
     // Items of at most 10 words need fewer needle registers per lane.
     const bool narrow = ts.maxWords <= 10;
+    if (insert && (variant == 0 || variant == 4 || variant == 8 || variant == 16 || variant == 32)) {
+        for (uint32_t i0 = 0; i0 < nseg; i0 += kMaxLaneSegs) {
+            const LaneSegs a = lane_segs(ts, segs + i0, std::min(nseg - i0, kMaxLaneSegs), 256u);
+            const uint32_t grid = a.blockStart[a.n];
+            if (grid == 0)
+                continue;
+            if (narrow)
+                insert_lanes_seg<10><<<grid, block, 0, stream>>>(ts.devTables, words, a, out);
+            else
+                insert_lanes_seg<18><<<grid, block, 0, stream>>>(ts.devTables, words, a, out);
+        }
+        if (ev1)
+            SVDAG_HIP(hipEventRecord(ev1, stream));
+        SVDAG_HIP(hipGetLastError());
+        return SVDAG_OK;
+    }
     switch (variant) {
     case 0: {
         const uint32_t grid = grid_for(n, block, 1u << 16);
-        if (insert)
-            bulk_lane_kernel<true><<<grid, block, 0, stream>>>(ts.devTables, ts.minWords, words, segBuf, nseg, n, out);
-        else
-            bulk_lane_kernel<false><<<grid, block, 0, stream>>>(ts.devTables, ts.minWords, words, segBuf, nseg, n, out);
+        bulk_find_lane_kernel<<<grid, block, 0, stream>>>(ts.devTables, ts.minWords, words, segBuf, nseg, n, out);
         break;
     }
-#define SVDAG_BULK_LAUNCH(G, INS, MW) \
-    bulk_group_kernel<G, INS, MW><<<grid, block, 0, stream>>>(ts.devTables, ts.minWords, words, segBuf, nseg, n, out)
+#define SVDAG_BULK_LAUNCH(G, MW) \
+    bulk_find_group_kernel<G, MW><<<grid, block, 0, stream>>>(ts.devTables, ts.minWords, words, segBuf, nseg, n, out)
 #define SVDAG_BULK_CASE(G)                                                                                              \
     case G: {                                                                                                           \
         const uint32_t grid = grid_for((uint64_t)n * G, block, 1u << 16);                                               \
-        if (insert) {                                                                                                   \
-            if (narrow) SVDAG_BULK_LAUNCH(G, true, 10); else SVDAG_BULK_LAUNCH(G, true, 18);                            \
-        } else {                                                                                                        \
-            if (narrow) SVDAG_BULK_LAUNCH(G, false, 10); else SVDAG_BULK_LAUNCH(G, false, 18);                          \
-        }                                                                                                               \
+        if (narrow) SVDAG_BULK_LAUNCH(G, 10); else SVDAG_BULK_LAUNCH(G, 18);                                            \
         break;                                                                                                          \
     }
         SVDAG_BULK_CASE(4)
@@ -720,10 +765,6 @@ int launch_bulk(const TableSet& ts,const uint32_t* words, const svdag_segment* s
 #undef SVDAG_BULK_LAUNCH
 #define SVDAG_MULTI_CASE(V, G, N)                                                                                       \
     case V: {                                                                                                           \
-        if (insert) {                                                                                                   \
-            set_error("multi-needle variants are find-only");                                                           \
-            return SVDAG_E_INVALID;                                                                                     \
-        }                                                                                                               \
         const uint32_t grid = grid_for(((uint64_t)n + N - 1) / N * G, block, 1u << 16);                                 \
         if (narrow)                                                                                                     \
             bulk_find_multi_kernel<G, N, 10><<<grid, block, 0, stream>>>(ts.devTables, ts.minWords, words, segBuf, nseg, n, out); \

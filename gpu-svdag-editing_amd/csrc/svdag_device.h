@@ -163,7 +163,11 @@ __device__ inline uint32_t slab_alloc_lanes(const TableDev& t, unsigned long lon
     int top = 0;
     uint32_t base = 0;
     if (__lane_id() == leader) {
-        top = atomicSub(&a->freeCount, (int)k);
+        // Tables without reference counts never free a slab.  (Loading the
+        // count first instead costs more than the pop it saves: every growing
+        // chain of the table updates that line.)
+        if (t.refs)
+            top = atomicSub(&a->freeCount, (int)k);
         const uint32_t avail = top <= 0 ? 0u : ((uint32_t)top < k ? (uint32_t)top : k);
         if (avail < k)
             base = atomicAdd(&a->fresh, k - avail);
@@ -658,7 +662,14 @@ __device__ inline uint32_t lane_insert(const TableDev& t, const uint32_t (&w)[MW
         uint32_t* line = t.lines + (size_t)slab * kLineWords;
         uint32_t emp;
         const bool room = line_empty(t, L.tag, emp);
-        if (room || L.next == kNoSlab) {
+        if (L.next == kPendingSlab)
+            L.next = kNoSlab; // a head read while its link was being set: the CAS asks
+        // Chains grow once the wave has nothing else to do, so that its new
+        // slabs come from one allocation: the table's counter is one word
+        // that all waves queue on (about 13 ns each).
+        const bool grow = !room && L.next == kNoSlab;
+        const bool others = __ballot(!grow) != 0ull;
+        if (room || (grow && !others)) {
             const uint32_t bit = room ? __ffs(emp) - 1u : 0u;
             const uint32_t j = room ? bit >> 2 : t.tagWords;
             uint32_t old = kNoSlab, want = kPendingSlab;
@@ -698,8 +709,6 @@ __device__ inline uint32_t lane_insert(const TableDev& t, const uint32_t (&w)[MW
                     L = LineHead { { 0u, 0u, 0u, 0u }, kNoSlab };
                 }
             }
-        } else if (L.next == kPendingSlab) {
-            L.next = kNoSlab; // a head read while its link was being set: the CAS asks
         }
         if (!room && L.next < kPendingSlab) {
             slab = L.next;

@@ -72,7 +72,8 @@ typedef struct {
 } svdag_segment;
 
 /* Variant of a bulk operation: 0 = one lane per item (cf. add/find),
- * 4/8/16/32 = that many lanes of a wave64 per item (cf. addAsWarp/findAsWarp),
+ * 4/8/16/32 = that many lanes of a wave64 per item (cf. findAsWarp; inserts
+ * take these too and run one lane per item, which is faster throughout),
  * 1/2/3 = find only, one lane per item with blocks assigned to segments and
  * 1/2/4 finds per lane in flight (at most 32 segments),
  * N*100 + G (204, 404, 208, 408) = find only, G lanes per group with N
