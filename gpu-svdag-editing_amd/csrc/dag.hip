@@ -11,7 +11,7 @@
 // read.  Work items of all levels live in one array (level L+1 starts where
 // level L ends); the SVO node of work item w is nodes[w], the SVO leaf of
 // leaf work item i is leaves[i].
-#include "dag_internal.h"
+#include "merge_device.h"
 #include <algorithm>
 #include <chrono>
 #include <cmath>
@@ -419,16 +419,6 @@ __global__ void __launch_bounds__(256) svo_leaf_level(WsDev ws, DagDev dag, cons
     }
 }
 
-// The tables' descriptors in LDS: a lane's probe then waits for its record,
-// not for its record and then a descriptor.
-__device__ inline void tables_stage(TableDev* sTab, const DagDev& dag)
-{
-    const uint32_t* src = reinterpret_cast<const uint32_t*>(dag.tables);
-    uint32_t* dst = reinterpret_cast<uint32_t*>(sTab);
-    for (uint32_t i = threadIdx.x; i < dag.numTables * (sizeof(TableDev) / 4u); i += blockDim.x)
-        dst[i] = src[i];
-}
-
 __device__ inline void dedup_clear(const WsDev& ws, uint32_t count, uint32_t tid, uint32_t stride)
 {
     const uint32_t cap = dedup_cap(count, ws.dedupCap);
@@ -444,86 +434,126 @@ __device__ inline void dedup_clear(const WsDev& ws, uint32_t count, uint32_t tid
 // items of an edit that made no leaf are emptied (that edit is dropped as a
 // whole, :651).  The children's representatives, then their handles, are
 // loaded together: two dependent round trips for the item, not two per child.
-template <bool kMulti>
-__device__ inline void prepare_item(const WsDev& ws, const DagDev& dag, uint32_t L, uint32_t w, bool gateAll,
-                                    uint32_t childStart)
+struct NodeItem {
+    uint32_t r[kNodeStride]; // the record: header, children, "has a new child"
+    uint32_t oldMask;        // the record's child mask before empty children were dropped
+    bool full;
+};
+// below(r, bit, imask, newChild): replaces the interior children of r (items of
+// the level below) by their handles, kSentinel for empty ones, and says
+// whether this merge inserted one.  dropped: the item's edit made no leaf.
+// Returns false for an item that was empty already.
+template <bool kMulti, typename Below>
+__device__ inline bool resolve_item(const DagDev& dag, uint32_t L, bool dropped, bool gate, NodeItem& it, Below&& below)
 {
-    uint32_t* rec = ws.nodes + (size_t)w * kNodeStride;
-    uint32_t r[kNodeStride];
-    lane_rec_load<(int)kNodeStride>(r, rec);
-    const uint32_t e = kMulti ? ws.editOf[w] : 0u;
+    uint32_t (&r)[kNodeStride] = it.r;
     const uint32_t mask = r[0] & 0xFFu;
+    it.oldMask = mask;
+    it.full = false;
     if (mask == 0)
-        return;
-    const bool gate = kMulti ? ws.edFull[e * kMaxLevels + L + 1] != 0 : gateAll;
-    if (kMulti && ws.edCount[e * kMaxLevels + dag.leafLevel] == 0) {
-        rec[0] = 0u;
-        return;
+        return false;
+    if (kMulti && dropped) {
+        r[0] = 0u;
+        return true;
     }
     const bool leafChildren = L + 1 == dag.leafLevel;
     const uint32_t imask = header_payload(r[0], dag.M) & 0xFFu;
-    uint32_t rep[8], created[8], bit[8];
+    uint32_t bit[8], newMask = 0, newChild = 0;
     uint32_t m = mask;
 #pragma unroll
     for (uint32_t k = 0; k < 8; ++k) {
         bit[k] = m & (0u - m);
         m ^= bit[k];
-        rep[k] = (imask & bit[k]) ? ws.rep[childStart + r[1 + k]] : kSentinel;
     }
+    below(r, bit, imask, newChild);
 #pragma unroll
-    for (uint32_t k = 0; k < 8; ++k) {
-        created[k] = 0u;
-        if (imask & bit[k]) {
-            r[1 + k] = kSentinel;
-            if (rep[k] != kSentinel) {
-                r[1 + k] = ws.handle[rep[k]];
-                created[k] = ws.created[rep[k]]; // 1: inserted by this merge (2: unchanged leaf)
-            }
-        }
-    }
-    uint32_t newMask = 0, newChild = 0;
-#pragma unroll
-    for (uint32_t k = 0; k < 8; ++k) {
-        newChild |= created[k] & 1u;
+    for (uint32_t k = 0; k < 8; ++k)
         if (bit[k] && r[1 + k] != kSentinel)
             newMask |= bit[k];
-    }
-    bool full = false;
     uint32_t fm = 0;
     if (gate && newMask == 0xFFu) {
         // Full children of one material are usually one shared item.
-        full = true;
+        it.full = true;
 #pragma unroll
         for (uint32_t j = 0; j < 8; ++j) {
-            if (!full || (j > 0 && r[1 + j] == r[1]))
+            if (!it.full || (j > 0 && r[1 + j] == r[1]))
                 continue;
             uint32_t cm = 0;
             const bool f = leafChildren ? leaf_is_full(dag_leaf_ptr(dag, r[1 + j]), dag.M, cm)
                                         : header_full(dag_node_ptr(dag, r[1 + j])[0], dag.M, cm);
             if (j == 0)
                 fm = cm;
-            full = f && cm == fm;
+            it.full = f && cm == fm;
         }
     }
-    r[0] = full ? header_make_full(0xFFu, fm, dag.M) : header_make(newMask, 0u, dag.M);
+    r[0] = it.full ? header_make_full(0xFFu, fm, dag.M) : header_make(newMask, 0u, dag.M);
     r[9] = newChild; // outside the item's words: equal items agree on it
-    if (newMask == mask) {
+    return true;
+}
+
+// The children's results from the workspace: representatives, then their
+// handles, each loaded together.
+struct BelowWs {
+    const WsDev& ws;
+    uint32_t childStart;
+    __device__ void operator()(uint32_t (&r)[kNodeStride], const uint32_t (&bit)[8], uint32_t imask,
+                               uint32_t& newChild) const
+    {
+        uint32_t rep[8], created[8];
+#pragma unroll
+        for (uint32_t k = 0; k < 8; ++k)
+            rep[k] = (imask & bit[k]) ? ws.rep[childStart + r[1 + k]] : kSentinel;
+#pragma unroll
+        for (uint32_t k = 0; k < 8; ++k) {
+            created[k] = 0u;
+            if (imask & bit[k]) {
+                r[1 + k] = kSentinel;
+                if (rep[k] != kSentinel) {
+                    r[1 + k] = ws.handle[rep[k]];
+                    created[k] = ws.created[rep[k]]; // 1: inserted by this merge (2: unchanged leaf)
+                }
+            }
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < 8; ++k)
+            newChild |= created[k] & 1u;
+    }
+};
+
+template <bool kMulti>
+__device__ inline void prepare_item(const WsDev& ws, const DagDev& dag, uint32_t L, uint32_t w, bool gateAll,
+                                    uint32_t childStart)
+{
+    uint32_t* rec = ws.nodes + (size_t)w * kNodeStride;
+    NodeItem it;
+    lane_rec_load<(int)kNodeStride>(it.r, rec);
+    const uint32_t e = kMulti ? ws.editOf[w] : 0u;
+    const bool gate = kMulti ? ws.edFull[e * kMaxLevels + L + 1] != 0 : gateAll;
+    const bool dropped = kMulti && ws.edCount[e * kMaxLevels + dag.leafLevel] == 0;
+    if (!resolve_item<kMulti>(dag, L, dropped, gate, it, BelowWs { ws, childStart }))
+        return;
+    if ((it.r[0] & 0xFFu) == it.oldMask) {
         uint2* out = reinterpret_cast<uint2*>(rec);
 #pragma unroll
         for (uint32_t k = 0; k < kNodeStride / 2u; ++k)
-            out[k] = make_uint2(r[2 * k], r[2 * k + 1]);
+            out[k] = make_uint2(it.r[2 * k], it.r[2 * k + 1]);
+    } else if ((it.r[0] & 0xFFu) == 0u) {
+        rec[0] = it.r[0];
+        rec[9] = it.r[9];
     } else {
-        uint32_t n = 0;
+        uint32_t n = 0, m = it.oldMask;
 #pragma unroll
-        for (uint32_t k = 0; k < 8; ++k)
-            if (bit[k] && r[1 + k] != kSentinel)
-                rec[1 + n++] = r[1 + k];
+        for (uint32_t k = 0; k < 8; ++k) {
+            if (m && it.r[1 + k] != kSentinel)
+                rec[1 + n++] = it.r[1 + k];
+            m &= m - 1u;
+        }
         for (; n < 8; ++n)
             rec[1 + n] = 0u;
-        rec[0] = r[0];
-        rec[9] = r[9];
+        rec[0] = it.r[0];
+        rec[9] = it.r[9];
     }
-    if (full)
+    if (it.full)
         set_flag(kMulti ? &ws.edFull[e * kMaxLevels + L] : &ws.lvl[L].fullCount);
 }
 
@@ -565,33 +595,32 @@ constexpr uint32_t kMergeBlock = 256;
 // level's blocks cost more than its waves gain: 256 edits at depth 15 took
 // 14.2-14.4 ms at 512 blocks, 14.4-14.5 at 2048, 15.3 with the whole grid.
 constexpr uint32_t kMergeSpread = 512;
-__device__ inline uint32_t merge_lanes_log2(uint32_t count, uint32_t maxLanes)
+__device__ inline uint32_t merge_lanes_log2(uint32_t count, uint32_t maxLanes, uint32_t most)
 {
-    const uint32_t most = min(gridDim.x, kMergeSpread) * kMergeBlock;
     uint32_t lg = 0;
     while ((2u << lg) <= maxLanes && ((uint64_t)count << (lg + 1u)) <= (uint64_t)most)
         ++lg;
     return lg;
 }
 
-template <bool kLeaf, int MW>
-__global__ void __launch_bounds__(kMergeBlock) merge_dedup_find(WsDev ws, DagDev dag, uint32_t L, uint32_t maxLanes)
+template <uint32_t kBlock>
+struct DedupShared {
+    uint32_t first[2 * kBlock]; // 1 + the block's first item of a content, by hash
+    uint32_t hash[kBlock], rep[kBlock];
+};
+// This block's part (of `blocks`) of a level.
+template <bool kLeaf, int MW, uint32_t kBlock>
+__device__ inline void dedup_find_block(const WsDev& ws, const DagDev& dag, const TableDev* sTab, const LevelDesc& me,
+                                        uint32_t lg, uint32_t block, uint32_t blocks, DedupShared<kBlock>& sh)
 {
-    if (merge_skipped(ws, dag))
-        return;
-    __shared__ TableDev sTab[kRefTables];
-    __shared__ uint32_t sFirst[2 * kMergeBlock]; // 1 + the block's first item of a content, by hash
-    __shared__ uint32_t sHash[kMergeBlock], sRep[kMergeBlock];
-    const LevelDesc me = ws.lvl[L];
-    const uint32_t lg = merge_lanes_log2(me.count, maxLanes);
-    const uint32_t perBlock = kMergeBlock >> lg;
-    if (blockIdx.x * perBlock >= me.count)
-        return;
-    tables_stage(sTab, dag);
+    uint32_t (&sFirst)[2 * kBlock] = sh.first;
+    uint32_t (&sHash)[kBlock] = sh.hash;
+    uint32_t (&sRep)[kBlock] = sh.rep;
+    const uint32_t perBlock = kBlock >> lg;
     const uint32_t capMask = dedup_cap(me.count, ws.dedupCap) - 1u;
     const uint32_t t = threadIdx.x >> lg;
     const bool works = (threadIdx.x & ((1u << lg) - 1u)) == 0u;
-    for (uint32_t i0 = blockIdx.x * perBlock; i0 < me.count; i0 += gridDim.x * perBlock) {
+    for (uint32_t i0 = block * perBlock; i0 < me.count; i0 += blocks * perBlock) {
         const uint32_t i = i0 + t;
         const uint32_t w = me.start + i;
         // unchanged leaf: rep and handle were set by svo_leaf_level
@@ -620,14 +649,14 @@ __global__ void __launch_bounds__(kMergeBlock) merge_dedup_find(WsDev ws, DagDev
             return eq;
         };
         sFirst[threadIdx.x] = 0u;
-        sFirst[threadIdx.x + kMergeBlock] = 0u;
+        sFirst[threadIdx.x + kBlock] = 0u;
         if (works)
             sHash[t] = h;
         __syncthreads();
         const uint32_t mixed = mix32(h);
         uint32_t first = t;
         if (active) {
-            uint32_t p = (mixed >> 8) & (2 * kMergeBlock - 1u);
+            uint32_t p = (mixed >> 8) & (2 * kBlock - 1u);
             while (true) {
                 uint32_t v = __hip_atomic_load(&sFirst[p], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                 if (v == 0u)
@@ -638,7 +667,7 @@ __global__ void __launch_bounds__(kMergeBlock) merge_dedup_find(WsDev ws, DagDev
                     first = v - 1u;
                     break;
                 }
-                p = (p + 1u) & (2 * kMergeBlock - 1u);
+                p = (p + 1u) & (2 * kBlock - 1u);
             }
         }
         uint32_t rep = w;
@@ -668,8 +697,9 @@ __global__ void __launch_bounds__(kMergeBlock) merge_dedup_find(WsDev ws, DagDev
             if (rep == w) {
                 // A node with a child this merge inserted is new: no find.
                 uint32_t r = kNotFound, hint = kNoSlab;
+                LineHead head;
                 if (kLeaf || n[MW - 1] == 0u)
-                    r = lane_find_hint<MW>(sTab[s - 2], n, s, h, hint);
+                    r = lane_find_hint<MW>(sTab[s - 2], n, s, h, hint, head);
                 ws.handle[w] = (r == kNotFound) ? kNotFound : (kLeaf ? leaf_handle(dag, r, s) : node_handle(r, s));
                 ws.created[w] = 0;
                 ws.hint[w] = hint;
@@ -677,6 +707,21 @@ __global__ void __launch_bounds__(kMergeBlock) merge_dedup_find(WsDev ws, DagDev
         }
         __syncthreads(); // sFirst, sHash and sRep are rewritten next iteration
     }
+}
+
+template <bool kLeaf, int MW>
+__global__ void __launch_bounds__(kMergeBlock) merge_dedup_find(WsDev ws, DagDev dag, uint32_t L, uint32_t maxLanes)
+{
+    if (merge_skipped(ws, dag))
+        return;
+    __shared__ TableDev sTab[kRefTables];
+    __shared__ DedupShared<kMergeBlock> sh;
+    const LevelDesc me = ws.lvl[L];
+    const uint32_t lg = merge_lanes_log2(me.count, maxLanes, min(gridDim.x, kMergeSpread) * kMergeBlock);
+    if (blockIdx.x * (kMergeBlock >> lg) >= me.count)
+        return;
+    tables_stage(sTab, dag);
+    dedup_find_block<kLeaf, MW, kMergeBlock>(ws, dag, sTab, me, lg, blockIdx.x, gridDim.x, sh);
 }
 
 // Insert the representatives the DAG did not hold (insertUniqueInHashTableAsWarp,
@@ -692,40 +737,6 @@ __global__ void __launch_bounds__(kMergeBlock) merge_dedup_find(WsDev ws, DagDev
 // handle, and each child gets one update: a child that thousands of items
 // share would otherwise collect thousands of atomics before the first shows
 // in its count (a stream of 256 edits took 25 ms so, 15 with the sums).
-constexpr uint32_t kRefSlots = 2048; // 256 items have at most 2048 children
-template <uint32_t kSlots>
-struct BlockRefs {
-    uint32_t child[kSlots], add[kSlots];
-};
-
-__device__ inline uint32_t* child_count(const DagDev& dag, const TableDev* sTab, uint32_t c, uint8_t role)
-{
-    const bool leaf = role == kRoleParentOfLeaves;
-    const uint32_t s = leaf ? leaf_handle_size(dag, c) : node_handle_size(c);
-    return sTab[s - 2].refs + (leaf ? leaf_handle_ptr(dag, c) : node_handle_ptr(c));
-}
-
-template <uint32_t kSlots>
-__device__ inline void block_ref_add(BlockRefs<kSlots>& refs, uint32_t slotMask, const DagDev& dag,
-                                     const TableDev* sTab, uint32_t c, uint8_t role)
-{
-    uint32_t p = (c * 0x9E3779B1u) >> 21;
-    for (uint32_t tries = 0; tries < 8; ++tries) {
-        p &= slotMask;
-        uint32_t v = __hip_atomic_load(&refs.child[p], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        if (v == kSentinel)
-            v = atomicCAS(&refs.child[p], kSentinel, c);
-        if (v == kSentinel || v == c) {
-            atomicAdd(&refs.add[p], 1u);
-            return;
-        }
-        ++p;
-    }
-    uint32_t* cnt = child_count(dag, sTab, c, role);
-    if (ld_filter(cnt) < kStickyRefs)
-        atomicAdd(cnt, 1u);
-}
-
 template <bool kLeaf, int MW, uint32_t kSlots>
 __device__ inline bool insert_item(const WsDev& ws, const DagDev& dag, const TableDev* sTab, const LevelDesc& me,
                                    uint32_t i, uint8_t role, BlockRefs<kSlots>& refs, uint32_t slotMask)
@@ -760,7 +771,8 @@ __device__ inline bool insert_item(const WsDev& ws, const DagDev& dag, const Tab
     const TableDev& t = sTab[s - 2];
     if (found != kNotFound) {
         // An equal item stored with the right role may follow in the chain.
-        const uint32_t again = lane_find_hint<MW>(t, n, s, h, hint, kLeaf ? kRoleLeafUse : role);
+        LineHead head;
+        const uint32_t again = lane_find_hint<MW>(t, n, s, h, hint, head, kLeaf ? kRoleLeafUse : role);
         if (again != kNotFound) {
             ws.handle[w] = kLeaf ? leaf_handle(dag, again, s) : node_handle(again, s);
             return false;
@@ -784,31 +796,18 @@ __device__ inline bool insert_item(const WsDev& ws, const DagDev& dag, const Tab
     return true;
 }
 
-// Also clears the dedup table for the level above, which the next launches
-// fill.
-template <bool kLeaf, int MW>
-__global__ void __launch_bounds__(kMergeBlock) merge_insert(WsDev ws, DagDev dag, uint32_t L, uint32_t maxLanes)
+// This block's part (of `blocks`) of a level.
+template <bool kLeaf, int MW, uint32_t kBlock, uint32_t kSlots>
+__device__ inline void insert_block(const WsDev& ws, const DagDev& dag, const TableDev* sTab, const LevelDesc& me,
+                                    uint32_t L, uint32_t lg, uint32_t block, uint32_t blocks,
+                                    BlockRefs<kSlots>& sRefs, uint32_t& sInserted)
 {
-    if (merge_skipped(ws, dag))
-        return;
-    __shared__ uint32_t sInserted;
-    __shared__ TableDev sTab[kRefTables];
-    __shared__ BlockRefs<kLeaf ? 1u : kRefSlots> sRefs;
-    const LevelDesc me = ws.lvl[L];
-    if (L > 0)
-        dedup_clear(ws, ws.lvl[L - 1].count, blockIdx.x * kMergeBlock + threadIdx.x, gridDim.x * kMergeBlock);
-    const uint32_t lg = merge_lanes_log2(me.count, maxLanes);
-    const uint32_t perBlock = kMergeBlock >> lg;
-    if (blockIdx.x * perBlock >= me.count)
-        return;
-    const uint32_t slotMask = (kRefSlots >> lg) - 1u;
-    if (threadIdx.x == 0)
-        sInserted = 0u;
-    tables_stage(sTab, dag);
+    const uint32_t perBlock = kBlock >> lg;
+    const uint32_t slotMask = min(kRefSlots, 8u * perBlock) - 1u;
     const uint8_t role = kLeaf ? (uint8_t)0u : node_role(dag, L);
-    for (uint32_t i0 = blockIdx.x * perBlock; i0 < me.count; i0 += gridDim.x * perBlock) {
+    for (uint32_t i0 = block * perBlock; i0 < me.count; i0 += blocks * perBlock) {
         if constexpr (!kLeaf)
-            for (uint32_t q = threadIdx.x; q <= slotMask; q += kMergeBlock) {
+            for (uint32_t q = threadIdx.x; q <= slotMask; q += kBlock) {
                 sRefs.child[q] = kSentinel;
                 sRefs.add[q] = 0u;
             }
@@ -822,12 +821,12 @@ __global__ void __launch_bounds__(kMergeBlock) merge_insert(WsDev ws, DagDev dag
         __syncthreads();
         if constexpr (!kLeaf) {
             // Every count the thread updates is loaded before the first update.
-            constexpr uint32_t kPer = kRefSlots / kMergeBlock;
+            constexpr uint32_t kPer = kSlots / kBlock;
             uint32_t* cnt[kPer];
             uint32_t seen[kPer], add[kPer];
 #pragma unroll
             for (uint32_t k = 0; k < kPer; ++k) {
-                const uint32_t q = k * kMergeBlock + threadIdx.x;
+                const uint32_t q = k * kBlock + threadIdx.x;
                 const uint32_t c = q <= slotMask ? sRefs.child[q] : kSentinel;
                 seen[k] = kStickyRefs;
                 if (c != kSentinel) {
@@ -842,9 +841,197 @@ __global__ void __launch_bounds__(kMergeBlock) merge_insert(WsDev ws, DagDev dag
                     atomicAdd(cnt[k], add[k]);
         }
     }
+}
+
+// Also clears the dedup table for the level above, which the next launches
+// fill.
+template <bool kLeaf, int MW>
+__global__ void __launch_bounds__(kMergeBlock) merge_insert(WsDev ws, DagDev dag, uint32_t L, uint32_t maxLanes)
+{
+    if (merge_skipped(ws, dag))
+        return;
+    __shared__ uint32_t sInserted;
+    __shared__ TableDev sTab[kRefTables];
+    __shared__ BlockRefs<kLeaf ? 1u : kRefSlots> sRefs;
+    const LevelDesc me = ws.lvl[L];
+    if (L > 0)
+        dedup_clear(ws, ws.lvl[L - 1].count, blockIdx.x * kMergeBlock + threadIdx.x, gridDim.x * kMergeBlock);
+    const uint32_t lg = merge_lanes_log2(me.count, maxLanes, min(gridDim.x, kMergeSpread) * kMergeBlock);
+    if (blockIdx.x * (kMergeBlock >> lg) >= me.count)
+        return;
+    if (threadIdx.x == 0)
+        sInserted = 0u;
+    tables_stage(sTab, dag);
+    insert_block<kLeaf, MW, kMergeBlock>(ws, dag, sTab, me, L, lg, blockIdx.x, gridDim.x, sRefs, sInserted);
     __syncthreads();
     if (threadIdx.x == 0 && sInserted)
         atomicAdd(dag.stored, (unsigned long long)sInserted);
+}
+
+// The children's results from LDS.
+struct BelowSmall {
+    const SmallShared<kSmallBlock>& sh;
+    uint32_t parity;
+    __device__ void operator()(uint32_t (&r)[kNodeStride], const uint32_t (&bit)[8], uint32_t imask,
+                               uint32_t& newChild) const
+    {
+#pragma unroll
+        for (uint32_t k = 0; k < 8; ++k)
+            if (imask & bit[k]) {
+                const uint32_t rep = sh.rep[parity][r[1 + k]];
+                r[1 + k] = rep == kSentinel ? kSentinel : sh.handle[parity][rep];
+                newChild |= rep == kSentinel ? 0u : sh.created[parity][rep];
+            }
+    }
+};
+
+// Levels first .. last (upwards), none a leaf level.  Levels of more items
+// than threads go through the workspace, in this block too.  What a level
+// needs from the SVO build (records, edits, leaf counts) is loaded while the
+// level below is in its find and insert.
+template <bool kMulti>
+__global__ void __launch_bounds__(kSmallBlock) merge_small(WsDev ws, DagDev dag, uint32_t first, uint32_t last,
+                                                           uint32_t maxLanes)
+{
+    if (merge_skipped(ws, dag))
+        return;
+    __shared__ TableDev sTab[kRefTables];
+    __shared__ SmallShared<kSmallBlock> sh;
+    __shared__ LevelDesc sLvl[kMaxLevels];
+    // Full items of the level below, by edit & 255 (a wave's edits are at most
+    // 256 consecutive ones).
+    __shared__ uint32_t sFull[2][kMulti ? 256 : 1];
+    if (threadIdx.x == 0)
+        sh.inserted = sh.oom = 0u;
+    if (threadIdx.x < kMaxLevels)
+        sLvl[threadIdx.x] = ws.lvl[threadIdx.x];
+    for (uint32_t q = threadIdx.x; q < 2u * (kMulti ? 256u : 1u); q += kSmallBlock)
+        (&sFull[0][0])[q] = 0u;
+    tables_stage(sTab, dag);
+    __syncthreads();
+    struct Ahead {
+        uint32_t r[kNodeStride], e, leaves;
+    };
+    auto lanes = [&](uint32_t L) { return merge_lanes_log2(sLvl[L].count, maxLanes, kSmallBlock); };
+    auto item_of = [&](uint32_t L, uint32_t& w) {
+        const uint32_t lg = lanes(L), slot = threadIdx.x >> lg;
+        w = sLvl[L].start + slot;
+        return sLvl[L].count <= kSmallBlock && (threadIdx.x & ((1u << lg) - 1u)) == 0u && slot < sLvl[L].count;
+    };
+    auto load = [&](uint32_t L, Ahead& a) {
+#pragma unroll
+        for (uint32_t k = 0; k < kNodeStride; ++k)
+            a.r[k] = 0u;
+        a.e = 0u;
+        uint32_t w;
+        if (item_of(L, w)) {
+            lane_rec_load<(int)kNodeStride>(a.r, ws.nodes + (size_t)w * kNodeStride);
+            if (kMulti)
+                a.e = ws.editOf[w];
+        }
+    };
+    auto load_leaves = [&](uint32_t L, Ahead& a) {
+        uint32_t w;
+        a.leaves = kMulti && item_of(L, w) ? ws.edCount[a.e * kMaxLevels + dag.leafLevel] : 1u;
+    };
+    bool belowSmall = false;
+    Ahead next;
+    load(first, next);
+    load_leaves(first, next);
+    for (int L = (int)first; L >= (int)last; --L) {
+        const LevelDesc me = sLvl[L];
+        const uint32_t below = sLvl[L + 1].start;
+        const uint32_t parity = (uint32_t)L & 1u;
+        const bool more = L > (int)last;
+        if (me.count > kSmallBlock) {
+            const bool gate = kMulti || ws.lvl[L + 1].fullCount != 0;
+            for (uint32_t i = threadIdx.x; i < me.count; i += kSmallBlock)
+                prepare_item<kMulti>(ws, dag, (uint32_t)L, me.start + i, gate, below);
+            dedup_clear(ws, me.count, threadIdx.x, kSmallBlock);
+            for (uint32_t q = threadIdx.x; q < 2u * (kMulti ? 256u : 1u); q += kSmallBlock)
+                (&sFull[0][0])[q] = 0u;
+            __syncthreads();
+            DedupShared<kSmallBlock>& ds = *reinterpret_cast<DedupShared<kSmallBlock>*>(&sh.word[0][0]);
+            dedup_find_block<false, (int)kNodeStride, kSmallBlock>(ws, dag, sTab, me, 0u, 0u, 1u, ds);
+            __syncthreads();
+            insert_block<false, (int)kNodeStride, kSmallBlock>(ws, dag, sTab, me, (uint32_t)L, 0u, 0u, 1u,
+                                                               sh.refs[parity], sh.inserted);
+            __syncthreads();
+            belowSmall = false;
+            if (more) {
+                load((uint32_t)L - 1u, next);
+                load_leaves((uint32_t)L - 1u, next);
+            }
+            continue;
+        }
+        const uint32_t lg = lanes((uint32_t)L);
+        const uint32_t slot = threadIdx.x >> lg;
+        const bool works = (threadIdx.x & ((1u << lg) - 1u)) == 0u;
+        const bool active = works && slot < me.count;
+        const uint32_t w = me.start + slot;
+        const Ahead cur = next;
+        if (more)
+            load((uint32_t)L - 1u, next);
+        NodeItem it;
+#pragma unroll
+        for (uint32_t k = 0; k < kNodeStride; ++k)
+            it.r[k] = cur.r[k];
+        it.full = false;
+        if (active) {
+            const uint32_t e = cur.e;
+            if (belowSmall)
+                resolve_item<kMulti>(dag, (uint32_t)L, cur.leaves == 0u, sFull[parity ^ 1u][kMulti ? e & 255u : 0u] != 0, it,
+                                     BelowSmall { sh, parity ^ 1u });
+            else
+                resolve_item<kMulti>(dag, (uint32_t)L, cur.leaves == 0u,
+                                     (kMulti ? ws.edFull[e * kMaxLevels + L + 1] : ws.lvl[L + 1].fullCount) != 0, it,
+                                     BelowWs { ws, below });
+            if ((it.r[0] & 0xFFu) != it.oldMask) { // close the gaps of dropped children
+                uint32_t out[8], n = 0, m = it.oldMask;
+#pragma unroll
+                for (uint32_t k = 0; k < 8; ++k)
+                    out[k] = 0u;
+#pragma unroll
+                for (uint32_t k = 0; k < 8; ++k) {
+                    if (m && it.r[1 + k] != kSentinel) {
+#pragma unroll
+                        for (uint32_t q = 0; q < 8; ++q)
+                            if (q == n)
+                                out[q] = it.r[1 + k];
+                        ++n;
+                    }
+                    m &= m - 1u;
+                }
+#pragma unroll
+                for (uint32_t k = 0; k < 8; ++k)
+                    it.r[1 + k] = out[k];
+            }
+        }
+        if (it.full) {
+            sFull[parity][kMulti ? cur.e & 255u : 0u] = 1u;
+            set_flag(kMulti ? &ws.edFull[cur.e * kMaxLevels + L] : &ws.lvl[L].fullCount); // for the spine, or a large level
+        }
+        small_find_insert(dag, sTab, it.r, slot, works, active, node_role(dag, (uint32_t)L), parity, sh, [&] {
+            if (more)
+                load_leaves((uint32_t)L - 1u, next);
+            if (threadIdx.x < (kMulti ? 256u : 1u)) // read above, set by the next level
+                sFull[parity ^ 1u][threadIdx.x] = 0u;
+        });
+        if (active) { // what the spine and edit_finish read
+            const uint32_t rep = sh.rep[parity][slot];
+            ws.rep[w] = rep == kSentinel ? kSentinel : me.start + rep;
+            ws.handle[w] = sh.handle[parity][slot];
+            ws.created[w] = sh.created[parity][slot];
+        }
+        belowSmall = true;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        if (sh.oom)
+            atomicOr(&ws.status->oom, 1u);
+        if (sh.inserted)
+            atomicAdd(dag.stored, (unsigned long long)sh.inserted);
+    }
 }
 
 // Publish the new root (my_gpu_hash_dag_edits.cu:626) unless the merge was
@@ -1178,6 +1365,24 @@ static void launch_merge_level(svdag_ctx* ctx, const WsDev& ws, uint32_t L, uint
     }
 }
 
+// Levels leafLevel .. top: the large ones one after the other over the grid,
+// the small ones above them in one block.  The line is drawn on the host's
+// bound of a level's items (about twice what it holds): one block takes 9-15
+// us a level up to there, three launches 25; at a bound of 8192 it takes
+// longer than they do (256 edits at depth 15: 13.6 ms at 512 to 4096, 14.5 at
+// 8192 and with launches only).
+constexpr uint64_t kSmallLevel = 2048;
+template <bool kMulti>
+static void launch_merge_levels(svdag_ctx* ctx, const WsDev& ws, uint32_t top, const uint64_t* items, uint32_t kCap)
+{
+    const DagDev& dag = ctx->dag;
+    int L = (int)dag.leafLevel;
+    for (; L >= (int)top && (L == (int)dag.leafLevel || items[L] > kSmallLevel); --L)
+        launch_merge_level<kMulti>(ctx, ws, (uint32_t)L, items[L], kCap);
+    if (L >= (int)top)
+        merge_small<kMulti><<<1, kSmallBlock, 0, ctx->stream>>>(ws, dag, (uint32_t)L, top, ctx->groupSize);
+}
+
 // Enqueue one edit: ed is the host copy (for grid sizing), edDev the same
 // editor in device memory, ws the workspace view whose status / level table
 // slots this edit uses.
@@ -1189,17 +1394,13 @@ int launch_edit(svdag_ctx* ctx, const EditorDev& ed, const EditorDev* edDev, con
     const uint32_t kCap = ctx->maxBlocks;
     edit_begin<<<1, 64, 0, st>>>(ws, ctx->dRoot, ed.kind == EK_COPY ? 1u : 0u,
                                  ed.kind == EK_DENSE || ed.kind == EK_TERRAIN ? 1u : 0u);
-    for (uint32_t L = 0; L < dag.leafLevel; ++L) {
-        const uint64_t items = std::min<uint64_t>(level_bound(ctx, b, L), ws.capWork);
-        svo_inner_level<false><<<grid_for(items, 32, kCap), 256, 0, st>>>(ws, dag, edDev, L);
-    }
-    {
-        const uint64_t items = std::min<uint64_t>(level_bound(ctx, b, dag.leafLevel), ws.capLeaf);
-        svo_leaf_level<false><<<grid_for(items, 4 * kLeavesPerWave, kCap), 256, 0, st>>>(ws, dag, edDev);
-    }
-    for (int L = (int)dag.leafLevel; L >= 0; --L)
-        launch_merge_level<false>(ctx, ws, (uint32_t)L, std::min<uint64_t>(level_bound(ctx, b, (uint32_t)L), ws.capWork),
-                                  kCap);
+    uint64_t items[kMaxLevels] {};
+    for (uint32_t L = 0; L <= dag.leafLevel; ++L)
+        items[L] = std::min<uint64_t>(level_bound(ctx, b, L), L == dag.leafLevel ? ws.capLeaf : ws.capWork);
+    for (uint32_t L = 0; L < dag.leafLevel; ++L)
+        svo_inner_level<false><<<grid_for(items[L], 32, kCap), 256, 0, st>>>(ws, dag, edDev, L);
+    svo_leaf_level<false><<<grid_for(items[dag.leafLevel], 4 * kLeavesPerWave, kCap), 256, 0, st>>>(ws, dag, edDev);
+    launch_merge_levels<false>(ctx, ws, 0, items, kCap);
     edit_finish<<<1, 64, 0, st>>>(ws, dag, ctx->dRoot);
     SVDAG_HIP(hipGetLastError());
     return SVDAG_OK;
@@ -1210,21 +1411,20 @@ int launch_joint_levels(svdag_ctx* ctx, const WsDev& ws, const EditorDev* eds, u
 {
     const DagDev& dag = ctx->dag;
     const hipStream_t st = ctx->stream;
+    uint64_t items[kMaxLevels] {};
+    for (uint32_t L = S; L <= dag.leafLevel; ++L)
+        items[L] = std::min<uint64_t>(levelItems[L], L == dag.leafLevel ? ws.capLeaf : ws.capWork);
     if (part != 2) {
         for (uint32_t L = S; L < dag.leafLevel; ++L)
-            svo_inner_level<true><<<grid_for(std::min<uint64_t>(levelItems[L], ws.capWork), 32, kCap), 256, 0, st>>>(
-                ws, dag, eds, L);
-        svo_leaf_level<true><<<grid_for(std::min<uint64_t>(levelItems[dag.leafLevel], ws.capLeaf),
-                                        4 * kLeavesPerWave, kCap),
-                               256, 0, st>>>(ws, dag, eds);
+            svo_inner_level<true><<<grid_for(items[L], 32, kCap), 256, 0, st>>>(ws, dag, eds, L);
+        svo_leaf_level<true><<<grid_for(items[dag.leafLevel], 4 * kLeavesPerWave, kCap), 256, 0, st>>>(ws, dag, eds);
     }
     // The build above only reads items the root reaches; the merge below
     // finds and inserts, so it waits for whatever mergeAfter marks.
     if (mergeAfter)
         SVDAG_HIP(hipStreamWaitEvent(st, mergeAfter, 0));
     if (part != 1)
-        for (int L = (int)dag.leafLevel; L >= (int)S; --L)
-            launch_merge_level<true>(ctx, ws, (uint32_t)L, std::min<uint64_t>(levelItems[L], ws.capWork), kCap);
+        launch_merge_levels<true>(ctx, ws, S, items, kCap);
     SVDAG_HIP(hipGetLastError());
     return SVDAG_OK;
 }

@@ -31,7 +31,7 @@
 // Copy edits read the live DAG outside their own region and run on their
 // own, as does an edit the spine cannot take (more than eight items on a
 // level, which the choice of S rules out).
-#include "dag_internal.h"
+#include "merge_device.h"
 #include <algorithm>
 #include <cstring>
 
@@ -123,20 +123,18 @@ __global__ void __launch_bounds__(256) fused_seed(WsDev ws, DagDev dag, const Ed
 // wave to the sequential spine.
 constexpr uint32_t kParEdits = 64;
 constexpr uint32_t kParItems = kParEdits * kSpineItems;
-constexpr uint32_t kParThreads = 1024;
+constexpr uint32_t kParThreads = kSmallBlock;
 
 struct SpineItem {
     uint32_t x, y, z, orig; // position at its level; its handle in the wave's input DAG
     uint32_t sub;           // children this edit subdivides
     uint32_t dep;           // paint: children whose decision read their state (empty or not)
     uint32_t ref[8];        // per subdivided child: its item one level down, or its seed work item at S
-    uint32_t handle, created;
     uint32_t och[8];        // its children in the wave's input DAG (kSentinel: none)
 };
 struct SpineScratch {
     SpineItem item[kParEdits][kMaxLevels][kSpineItems];
     uint32_t cnt[kParEdits][kMaxLevels];
-    uint32_t full[kParEdits][kMaxLevels];
 };
 
 size_t spine_scratch_bytes()
@@ -159,18 +157,16 @@ __global__ void __launch_bounds__(kParThreads) fused_spine_par(WsDev ws, DagDev 
                                                                uint32_t* rootPtr, EditStatus* status,
                                                                LevelDesc* levels)
 {
-    __shared__ uint32_t sPos[kParItems][3];
-    __shared__ uint32_t sRec[kParItems][kNodeStride];
-    __shared__ uint32_t sNew[kParItems], sRep[kParItems], sResH[kParItems], sResC[kParItems];
-    __shared__ uint32_t sRepList[kParItems], sSubCnt[kParItems];
+    __shared__ uint32_t sPos[kParItems][3], sSubCnt[kParItems];
     __shared__ uint32_t sSub[kParItems], sChildNew[kParItems], sChildH[kParItems][8];
-    __shared__ uint32_t sHash[2 * kParItems], sPosHash[2 * kParItems], sPosOf[kParItems], sPrev[kParItems];
+    __shared__ uint32_t sPosHash[2 * kParItems], sPosOf[kParItems], sPrev[kParItems];
     __shared__ unsigned long long sPosEdits[kParItems];
-    __shared__ uint32_t sFullCnt[kParEdits], sDropped[kParEdits];
-    __shared__ uint32_t sOk, sBad, sOom, sNumReps;
-    __shared__ RefArrays sRa;
+    __shared__ uint32_t sFullCnt[2][kParEdits], sDropped[kParEdits]; // full items by level parity
+    __shared__ uint32_t sOk, sBad;
+    __shared__ TableDev sTab[kRefTables];
+    __shared__ SmallShared<kParItems> sh;
     const uint32_t t = threadIdx.x;
-    ref_arrays_stage(sRa, dag); // read after the barriers below
+    tables_stage(sTab, dag); // read after the barriers below
     const uint2 wv = f.waves[*f.waveIdx];
     const uint32_t K = wv.y - wv.x, S = f.S;
     const uint32_t leafLevel = dag.leafLevel;
@@ -185,7 +181,8 @@ __global__ void __launch_bounds__(kParThreads) fused_spine_par(WsDev ws, DagDev 
         }
         sOk = ok;
         sBad = 0u;
-        sOom = 0u;
+        sh.oom = 0u;
+        sh.inserted = 0u;
     }
     __syncthreads();
     if (!sOk)
@@ -297,10 +294,38 @@ __global__ void __launch_bounds__(kParThreads) fused_spine_par(WsDev ws, DagDev 
     }
 
     // ---- bottom-up: levels S-1 .. 0, every edit's nodes of a level at once.
-    const uint32_t lane = t & 63u, gl = t & 7u, gbase = lane & ~7u;
+    // An item of the SVO does not change any more, so the next level's is
+    // loaded while this one is found and inserted.
+    const uint32_t idx = t; // (edit k, item i) = (t / 8, t % 8)
+    struct Ahead {
+        uint32_t cnt, x, y, z, sub, dep, ref[8], och[8];
+    };
+    auto load = [&](uint32_t l, Ahead& a) {
+        a.cnt = k < K ? sc.cnt[k][l] : 0u;
+        const SpineItem& it = sc.item[k < K ? k : 0u][l][i];
+        a.x = it.x;
+        a.y = it.y;
+        a.z = it.z;
+        a.sub = it.sub;
+        a.dep = it.dep;
+#pragma unroll
+        for (uint32_t c = 0; c < 8; ++c) {
+            a.ref[c] = it.ref[c];
+            a.och[c] = it.och[c];
+        }
+    };
+    const bool paint = k < K && eds[wv.x + k].kind == EK_PAINT;
+    if (t < kParEdits)
+        sFullCnt[S & 1u][t] = t < K ? ws.edFull[(wv.x + t) * kMaxLevels + S] : 0u;
+    Ahead next;
+    load(S - 1u, next);
     for (int l = (int)S - 1; l >= 0; --l) {
-        const bool active = k < K && i < sc.cnt[k][l] && !sDropped[k];
-        const uint32_t idx = k * kSpineItems + i;
+        const Ahead it = next;
+        if (l > 0)
+            load((uint32_t)l - 1u, next);
+        const uint32_t parity = (uint32_t)l & 1u;
+        const bool here = k < K && i < it.cnt;
+        const bool active = here && !sDropped[k];
         const bool childLevelS = (uint32_t)l + 1 == S;
         const bool leafChildren = (uint32_t)l + 1 == leafLevel;
         // Stage the level in LDS: positions, and the subdivided children with
@@ -308,43 +333,40 @@ __global__ void __launch_bounds__(kParThreads) fused_spine_par(WsDev ws, DagDev 
         // it stages no subdivided children.
         if (t < kParItems) {
             uint32_t subm = 0, newm = 0;
-            if (k < K && i < sc.cnt[k][l]) {
-                const SpineItem& it = sc.item[k][l][i];
+            sPos[t][0] = kSentinel;
+            if (here) {
                 sPos[t][0] = it.x;
                 sPos[t][1] = it.y;
                 sPos[t][2] = it.z;
-                if (!sDropped[k]) {
-                    subm = it.sub;
-                    for (uint32_t c = 0; c < 8; ++c) {
-                        if (!((subm >> c) & 1u))
-                            continue;
-                        uint32_t cr = 0;
-                        if (childLevelS) {
-                            sChildH[t][c] = joint_handle(ws, it.ref[c], cr);
-                        } else {
-                            const SpineItem& ch = sc.item[k][l + 1][it.ref[c]];
-                            sChildH[t][c] = ch.handle;
-                            cr = ch.created;
-                        }
-                        newm |= cr << c;
+            }
+            if (active) {
+                subm = it.sub;
+                uint32_t rep[8];
+#pragma unroll
+                for (uint32_t c = 0; c < 8; ++c)
+                    rep[c] = !((subm >> c) & 1u) ? kSentinel
+                        : childLevelS ? ws.rep[it.ref[c]] : sh.rep[parity ^ 1u][k * kSpineItems + it.ref[c]];
+#pragma unroll
+                for (uint32_t c = 0; c < 8; ++c) {
+                    if (!((subm >> c) & 1u))
+                        continue;
+                    uint32_t h = kSentinel, cr = 0;
+                    if (rep[c] != kSentinel) {
+                        h = childLevelS ? ws.handle[rep[c]] : sh.handle[parity ^ 1u][rep[c]];
+                        cr = childLevelS ? ws.created[rep[c]] & 1u : sh.created[parity ^ 1u][rep[c]];
                     }
+                    sChildH[t][c] = h;
+                    newm |= cr << c;
                 }
-            } else {
-                sPos[t][0] = kSentinel;
             }
             sSub[t] = subm;
             sChildNew[t] = newm;
-        }
-        for (uint32_t h = t; h < 2 * kParItems; h += blockDim.x) {
-            sHash[h] = 0u;
-            sPosHash[h] = 0u;
-        }
-        if (t < kParItems)
             sPosEdits[t] = 0ull;
+        }
+        for (uint32_t h = t; h < 2 * kParItems; h += blockDim.x)
+            sPosHash[h] = 0u;
         if (t < kParEdits)
-            sFullCnt[t] = 0u;
-        if (t == 0)
-            sNumReps = 0u;
+            sFullCnt[parity][t] = 0u;
         __syncthreads();
         // Group the level's items by position: the first item to claim a
         // position names it, and collects the set of edits with an item there.
@@ -390,59 +412,61 @@ __global__ void __launch_bounds__(kParThreads) fused_spine_par(WsDev ws, DagDev 
             sPrev[t] = prev;
         }
         __syncthreads();
-        bool empty = true;
+        uint32_t rec[kNodeStride];
+#pragma unroll
+        for (uint32_t w = 0; w < kNodeStride; ++w)
+            rec[w] = 0u;
         if (active) {
-            const SpineItem& it = sc.item[k][l][i];
             const uint32_t mySub = sSub[idx];
             uint32_t ver[8];
+#pragma unroll
             for (uint32_t c = 0; c < 8; ++c)
-                ver[c] = ((mySub >> c) & 1u) ? sChildH[idx][c] : kSentinel;
+                ver[c] = ((mySub >> c) & 1u) ? sChildH[idx][c] : it.och[c];
             // A child this edit leaves alone is the version the latest earlier
             // edit rebuilt, else the input DAG's: walk the position's
             // predecessors until every such child has its version.
-            uint32_t left = ~mySub & 0xFFu, from = 0u;
+            uint32_t left = ~mySub & 0xFFu;
             for (uint32_t o = sPrev[idx]; left != 0u && o != kSentinel; o = sPrev[o]) {
                 const uint32_t hit = sSub[o] & left;
+#pragma unroll
                 for (uint32_t c = 0; c < 8; ++c)
                     if ((hit >> c) & 1u)
                         ver[c] = sChildH[o][c];
                 left &= ~hit;
-                from |= hit;
             }
-            from |= mySub;
-            uint32_t outH[8], nOut = 0, newMask = 0;
-            const uint32_t newChild = sChildNew[idx] != 0u ? 1u : 0u;
+            uint32_t n = 0, newMask = 0;
+#pragma unroll
             for (uint32_t c = 0; c < 8; ++c) {
-                const uint32_t h = ((from >> c) & 1u) ? ver[c] : it.och[c];
-                if (h != kSentinel) {
-                    outH[nOut++] = h;
-                    newMask |= 1u << c;
-                }
+                if (ver[c] == kSentinel)
+                    continue;
+#pragma unroll
+                for (uint32_t q = 0; q <= c; ++q)
+                    if (q == n)
+                        rec[1 + q] = ver[c];
+                ++n;
+                newMask |= 1u << c;
             }
             // Discovery, gated on this edit's full items one level down.
-            const uint32_t prevFull = childLevelS ? ws.edFull[(wv.x + k) * kMaxLevels + S] : sc.full[k][l + 1];
             bool full = false;
             uint32_t fm = 0;
-            if (prevFull != 0u && newMask == 0xFFu) {
+            if (sFullCnt[parity ^ 1u][k] != 0u && newMask == 0xFFu) {
                 full = true;
-                for (uint32_t j = 0; j < 8 && full; ++j) {
+#pragma unroll
+                for (uint32_t j = 0; j < 8; ++j) {
+                    if (!full || (j > 0 && rec[1 + j] == rec[1]))
+                        continue;
                     uint32_t m = 0;
-                    const bool fj = leafChildren ? leaf_is_full(dag_leaf_ptr(dag, outH[j]), dag.M, m)
-                                                 : header_full(dag_node_ptr(dag, outH[j])[0], dag.M, m);
+                    const bool fj = leafChildren ? leaf_is_full(dag_leaf_ptr(dag, rec[1 + j]), dag.M, m)
+                                                 : header_full(dag_node_ptr(dag, rec[1 + j])[0], dag.M, m);
                     if (j == 0)
                         fm = m;
                     full = fj && m == fm;
                 }
             }
-            empty = newMask == 0u;
-            uint32_t* rec = sRec[idx];
             rec[0] = full ? header_make_full(0xFFu, fm, dag.M) : header_make(newMask, 0u, dag.M);
-            for (uint32_t j = 0; j < 8; ++j)
-                rec[1 + j] = j < nOut ? outH[j] : 0u;
-            rec[9] = 0u;
-            sNew[idx] = newChild;
+            rec[9] = sChildNew[idx] != 0u ? 1u : 0u;
             if (full)
-                atomicAdd(&sFullCnt[k], 1u);
+                atomicAdd(&sFullCnt[parity][k], 1u);
         }
         // A paint item decided its state-dependent children on the input
         // DAG's state; the edits before it in the wave may have made such a
@@ -452,122 +476,39 @@ __global__ void __launch_bounds__(kParThreads) fused_spine_par(WsDev ws, DagDev 
         // the current state.  Nothing of the wave is published before the
         // last level, and what was inserted below is what the sequential
         // spine builds again and finds.
-        if (k < K && i < sc.cnt[k][l] && eds[wv.x + k].kind == EK_PAINT) {
-            const SpineItem& it = sc.item[k][l][i];
+        if (here && paint) {
             uint32_t need = it.dep, prior[8];
+#pragma unroll
             for (uint32_t c = 0; c < 8; ++c)
                 prior[c] = it.och[c];
             for (uint32_t o = sPrev[idx]; need != 0u && o != kSentinel; o = sPrev[o]) {
                 const uint32_t hit = sSub[o] & need;
+#pragma unroll
                 for (uint32_t c = 0; c < 8; ++c)
                     if ((hit >> c) & 1u)
                         prior[c] = sChildH[o][c];
                 need &= ~hit;
             }
+#pragma unroll
             for (uint32_t c = 0; c < 8; ++c)
                 if (((it.dep >> c) & 1u) && (prior[c] == kSentinel) != (it.och[c] == kSentinel))
                     atomicOr(&sBad, 1u);
         }
         __syncthreads();
         if (sBad)
-            return; // the sequential spine takes the wave
-        // In-level dedup over every edit's nodes: the first claimant of a
-        // content is its representative.
-        if (active && !empty) {
-            const uint32_t* rec = sRec[idx];
-            uint32_t hh = 0;
-            for (uint32_t w = 0; w < kNodeStride; ++w)
-                hh = mix32(hh ^ (rec[w] + w * 0x9E3779B9u));
-            uint32_t p = hh & (2 * kParItems - 1u);
-            uint32_t rep = idx;
-            while (true) {
-                uint32_t v = sHash[p];
-                if (v == 0u) {
-                    v = atomicCAS(&sHash[p], 0u, idx + 1u);
-                    if (v == 0u)
-                        break;
-                }
-                bool eq = true;
-                for (uint32_t w = 0; w < kNodeStride && eq; ++w)
-                    eq = sRec[v - 1u][w] == rec[w];
-                if (eq) {
-                    rep = v - 1u;
-                    break;
-                }
-                p = (p + 1u) & (2 * kParItems - 1u);
-            }
-            sRep[idx] = rep;
-            if (rep == idx)
-                sRepList[atomicAdd(&sNumReps, 1u)] = idx;
-        } else if (t < kParItems) {
-            sRep[t] = kSentinel;
-        }
-        if (t < kParEdits && t < K)
-            sc.full[t][l] = sFullCnt[t];
-        __syncthreads();
-        // DAG finds of the representatives, eight lanes each, then the
-        // inserts of those not found.  Finds and inserts never run at once:
-        // an insert claims its slot's tag before writing the item, so a
-        // concurrent find could otherwise match a half-written slot.
-        const uint32_t nReps = sNumReps;
-        for (uint32_t r = t >> 3; r < nReps; r += kParThreads / 8u) {
-            const uint32_t ri = sRepList[r];
-            const uint32_t* rec = sRec[ri];
-            const uint32_t s = node_size_from_header(rec[0]);
-            Needle<8> nd;
-            needle_load(nd, rec, s, gl);
-            const uint32_t hsh = needle_hash(nd, s, gl);
-            uint32_t res = kNotFound, hint = kNoSlab;
-            if (sNew[ri] == 0u)
-                res = table_find_group_hint<8>(dag.tables[s - 2], nd, s, hsh, gl, gbase, hint,
-                                               node_role(dag, (uint32_t)l));
-            if (gl == 0) {
-                sResH[ri] = res == kNotFound ? hint : node_handle(res, s);
-                sResC[ri] = res == kNotFound ? 2u : 0u; // 2: to insert, from the line in sResH
-            }
-        }
-        __syncthreads();
-        for (uint32_t r = t >> 3; r < nReps; r += kParThreads / 8u) {
-            const uint32_t ri = sRepList[r];
-            if (sResC[ri] != 2u)
-                continue; // uniform over the eight lanes of the item
-            const uint32_t* rec = sRec[ri];
-            const uint32_t s = node_size_from_header(rec[0]);
-            Needle<8> nd;
-            needle_load(nd, rec, s, gl);
-            const uint32_t hsh = needle_hash(nd, s, gl);
-            const uint32_t res = table_insert_group<8>(dag.tables[s - 2], nd, s, hsh, gl, gbase, sResH[ri]);
-            if (res != kNotFound) {
-                refs_on_insert(dag, sRa, nd, s, res, node_role(dag, (uint32_t)l), gl);
-                if (gl == 0)
-                    atomicAdd(dag.stored, 1ull);
-            }
-            // Every lane has read sResH above; the group's lanes are in
-            // lockstep within the wave, so lane 0 may overwrite it.
-            if (gl == 0) {
-                if (res == kNotFound) {
-                    sOom = 1u;
-                    sResH[ri] = kSentinel;
-                } else {
-                    sResH[ri] = node_handle(res, s);
-                }
-                sResC[ri] = 1u;
-            }
-        }
-        __syncthreads();
-        if (active) {
-            SpineItem& it = sc.item[k][l][i];
-            const uint32_t rep = sRep[idx];
-            it.handle = rep == kSentinel ? kSentinel : sResH[rep];
-            it.created = rep == kSentinel ? 0u : sResC[rep];
-        }
-        __syncthreads();
-        if (sOom)
+            break; // the sequential spine takes the wave
+        small_find_insert(dag, sTab, rec, idx, t < kParItems, active, node_role(dag, (uint32_t)l), parity, sh, [] {});
+        if (sh.oom)
             break;
     }
+    __syncthreads();
+    if (t == 0 && sh.inserted)
+        atomicAdd(dag.stored, (unsigned long long)sh.inserted);
+    if (sBad)
+        return;
 
     // ---- per-edit results, in edit order.
-    if (sOom) {
+    if (sh.oom) {
         if (t == 0) {
             EditStatus st {};
             st.oom = 1u;
@@ -593,7 +534,8 @@ __global__ void __launch_bounds__(kParThreads) fused_spine_par(WsDev ws, DagDev 
             if (!sDropped[e]) {
                 st.applied = 1u;
                 st.leafCount = ws.edCount[(wv.x + e) * kMaxLevels + leafLevel];
-                root = sc.item[e][0][0].handle;
+                const uint32_t rep = sh.rep[0][e * kSpineItems];
+                root = rep == kSentinel ? kSentinel : sh.handle[0][rep];
             }
             st.rootAfter = root;
             status[wv.x + e] = st;

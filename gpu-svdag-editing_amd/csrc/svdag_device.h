@@ -610,10 +610,11 @@ __device__ inline bool lane_item_equal(const uint32_t (&w)[MW], const uint32_t* 
     return eq;
 }
 
-// table_find_group_hint for one lane.
+// table_find_group_hint for one lane.  head: the hint line's head as the find
+// saw it.
 template <int MW>
 __device__ inline uint32_t lane_find_hint(const TableDev& t, const uint32_t (&w)[MW], uint32_t s, uint32_t h,
-                                          uint32_t& hint, uint8_t role = 0)
+                                          uint32_t& hint, LineHead& head, uint8_t role = 0)
 {
     const uint32_t tag4 = make_tag(h) * 0x01010101u;
     uint32_t slab = h % t.numBuckets;
@@ -625,20 +626,20 @@ __device__ inline uint32_t lane_find_hint(const TableDev& t, const uint32_t (&w)
         while (cand) {
             const uint32_t slot = __ffs(cand) - 1u;
             cand &= cand - 1u;
-            if (lane_item_equal<MW>(w, line_item(t, slab, slot), s)) {
-                const uint32_t ptr = (slab << kSlotBits) | slot;
-                if (role == 0 || (role == kRoleLeafUse ? t.roles[ptr] == 0 : (t.roles[ptr] & role) != 0))
-                    return ptr;
-            }
+            const uint32_t ptr = (slab << kSlotBits) | slot;
+            const uint8_t roles = role ? t.roles[ptr] : (uint8_t)0u; // beside the words, not after them
+            if (lane_item_equal<MW>(w, line_item(t, slab, slot), s)
+                && (role == 0 || (role == kRoleLeafUse ? roles == 0 : (roles & role) != 0)))
+                return ptr;
         }
         uint32_t emp;
-        if (hint == kNoSlab && line_empty(t, L.tag, emp))
+        const bool last = L.next >= kPendingSlab;
+        if (hint == kNoSlab && (line_empty(t, L.tag, emp) || last)) {
             hint = slab;
-        if (L.next >= kPendingSlab) {
-            if (hint == kNoSlab)
-                hint = slab;
-            return kNotFound;
+            head = L;
         }
+        if (last)
+            return kNotFound;
         slab = L.next;
     }
 }
@@ -651,13 +652,10 @@ __device__ inline uint32_t lane_find_hint(const TableDev& t, const uint32_t (&w)
 // slots and a link is set once while inserts run, so an old value only makes
 // the CAS fail, and the CAS brings the current one.
 template <int MW>
-__device__ inline uint32_t lane_insert(const TableDev& t, const uint32_t (&w)[MW], uint32_t s, uint32_t h,
-                                       uint32_t start = kNoSlab)
+__device__ inline uint32_t lane_insert_at(const TableDev& t, const uint32_t (&w)[MW], uint32_t s, uint32_t h,
+                                          uint32_t slab, LineHead L)
 {
     const uint32_t tag = make_tag(h);
-    uint32_t slab = start == kNoSlab ? h % t.numBuckets : start;
-    LineHead L;
-    line_head_load(L, t.lines + (size_t)slab * kLineWords, t.tagWords);
     while (true) {
         uint32_t* line = t.lines + (size_t)slab * kLineWords;
         uint32_t emp;
@@ -715,6 +713,17 @@ __device__ inline uint32_t lane_insert(const TableDev& t, const uint32_t (&w)[MW
             line_head_load(L, t.lines + (size_t)slab * kLineWords, t.tagWords);
         }
     }
+}
+
+// From the line a find pointed at, or the bucket's head (kNoSlab).
+template <int MW>
+__device__ inline uint32_t lane_insert(const TableDev& t, const uint32_t (&w)[MW], uint32_t s, uint32_t h,
+                                       uint32_t start = kNoSlab)
+{
+    const uint32_t slab = start == kNoSlab ? h % t.numBuckets : start;
+    LineHead L;
+    line_head_load(L, t.lines + (size_t)slab * kLineWords, t.tagWords);
+    return lane_insert_at<MW>(t, w, s, h, slab, L);
 }
 
 // ---------------------------------------------------------------- DAG encoding

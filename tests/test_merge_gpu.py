@@ -55,3 +55,38 @@ def test_merge_matches_oracle_and_counts_references(bits, lanes, grid_log2, patt
     assert counted.items_live == marked.items_live
     assert g.canonical() == o.canonical()
     g.close()
+
+
+@pytest.mark.gpu
+def test_levels_around_the_one_block_limit_match_oracle():
+    # Levels of 1025 to 2048 items among those one block takes (its threads
+    # loop there), from one copy and from a wave of paints; and a wave of one
+    # tiny edit.
+    levels, side = 8, 256
+    rng = np.random.default_rng(77)
+    vox = np.full((side,) * 3, 0xFF, np.uint8)
+    cells = [(x, y, z) for x in range(4) for y in range(2) for z in range(2)][:14]
+    for cx, cy, cz in cells:
+        c = tuple(64 * v + 8 for v in (cx, cy, cz))
+        vox[c[0]:c[0] + 48, c[1]:c[1] + 48, c[2]:c[2] + 48] = _noise(48, rng, 0.4, [1, 2, 3, 4])
+    vox[:96, 160:, 160:] = _noise(96, rng, 0.4, [5, 6])
+    g = svdag_py.MyGPUHashDAG(levels, 4)
+    o = oracle_py.OracleDag(levels, 4)
+    g.build_voxels(vox)
+    oracle_py.build_dense(o, vox)
+    paints = [(svdag_py.PAINT, 5 + i, (64.0 * cx + 32, 64.0 * cy + 32, 64.0 * cz + 32), 16.0)
+              for i, (cx, cy, cz) in enumerate(cells[:10])]
+    copy = (svdag_py.COPY, 0, (48.0, 208.0, 208.0), 44.0, (48.0, 208.0, 208.0), (180.0, 180.0, 70.0))
+    tiny = (svdag_py.SPHERE_ADD, 7, (200.0, 20.0, 20.0), 0.4)
+    big = [(svdag_py.PAINT, 15, (64.0 * cx + 32, 64.0 * cy + 32, 64.0 * cz + 32), 23.0) for cx, cy, cz in cells]
+    per_level = []
+    for batch in (paints, [copy], [tiny], big):
+        stats, _ = g.edit_batch(batch)
+        per_level.append(np.sum([list(s.svo_items) for s in stats], axis=0))
+        for e in batch:
+            o.edit(*e)
+        assert g.canonical() == o.canonical()
+    assert any(((n > 1024) & (n <= 2048)).any() for n in per_level)
+    st = g.garbage_collect()
+    assert st.marked == 0 and g.garbage_collect(mark=True).items_freed == 0
+    g.close()
