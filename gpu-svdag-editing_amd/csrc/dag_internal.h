@@ -112,8 +112,8 @@ __device__ inline uint8_t node_role(const DagDev& dag, uint32_t L)
 // (LDS): one dependent load less per count or role access.
 constexpr uint32_t kRefTables = 20; // item sizes 2 .. 18 words use 17
 struct RefArrays {
-    uint32_t* refs[kRefTables];
-    uint8_t* roles[kRefTables];
+    DevPtr<uint32_t> refs[kRefTables];
+    DevPtr<uint8_t> roles[kRefTables];
 };
 __device__ inline void ref_arrays_stage(RefArrays& r, const DagDev& dag)
 {

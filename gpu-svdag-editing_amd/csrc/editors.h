@@ -60,8 +60,8 @@ struct EditorDev {
     // hmax holds levels 1..D only (level 0's maxima are hmin's heights) and is
     // indexed by pyrOffset[k] - pyrOffset[1].
     uint32_t levels;
-    const int32_t* hmin;
-    const int32_t* hmax;
+    DevPtr<const int32_t> hmin;
+    DevPtr<const int32_t> hmax;
     uint64_t pyrOffset[kMaxLevels];
     // terrain height bands: cubes of 2^bandLog2 voxels hold one material
     // (band_material); banded == 0 gives every voxel `material`
@@ -72,7 +72,7 @@ struct EditorDev {
     uint32_t tileMin[2], tileMax[2];
     // dense grid of side 2^denseLog2 at the origin: pyramid level k holds
     // (side >> k)^3 codes indexed (x * s + y) * s + z (pyrOffset as above)
-    const uint16_t* dense;
+    DevPtr<const uint16_t> dense;
     uint32_t denseLog2;
 };
 

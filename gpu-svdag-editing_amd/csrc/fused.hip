@@ -341,23 +341,40 @@ __global__ void __launch_bounds__(kParThreads) fused_spine_par(WsDev ws, DagDev 
             }
             if (active) {
                 subm = it.sub;
-                uint32_t rep[8];
-#pragma unroll
-                for (uint32_t c = 0; c < 8; ++c)
-                    rep[c] = !((subm >> c) & 1u) ? kSentinel
-                        : childLevelS ? ws.rep[it.ref[c]] : sh.rep[parity ^ 1u][k * kSpineItems + it.ref[c]];
+                uint32_t rep[8], h[8], cr[8];
 #pragma unroll
                 for (uint32_t c = 0; c < 8; ++c) {
-                    if (!((subm >> c) & 1u))
-                        continue;
-                    uint32_t h = kSentinel, cr = 0;
-                    if (rep[c] != kSentinel) {
-                        h = childLevelS ? ws.handle[rep[c]] : sh.handle[parity ^ 1u][rep[c]];
-                        cr = childLevelS ? ws.created[rep[c]] & 1u : sh.created[parity ^ 1u][rep[c]];
-                    }
-                    sChildH[t][c] = h;
-                    newm |= cr << c;
+                    rep[c] = h[c] = kSentinel;
+                    cr[c] = 0u;
                 }
+                if (childLevelS) {
+#pragma unroll
+                    for (uint32_t c = 0; c < 8; ++c)
+                        if ((subm >> c) & 1u)
+                            rep[c] = ws.rep[it.ref[c]];
+#pragma unroll
+                    for (uint32_t c = 0; c < 8; ++c)
+                        if (rep[c] != kSentinel) {
+                            h[c] = ws.handle[rep[c]];
+                            cr[c] = ws.created[rep[c]] & 1u;
+                        }
+                } else {
+#pragma unroll
+                    for (uint32_t c = 0; c < 8; ++c)
+                        if ((subm >> c) & 1u) {
+                            rep[c] = sh.rep[parity ^ 1u][k * kSpineItems + it.ref[c]];
+                            if (rep[c] != kSentinel) {
+                                h[c] = sh.handle[parity ^ 1u][rep[c]];
+                                cr[c] = sh.created[parity ^ 1u][rep[c]];
+                            }
+                        }
+                }
+#pragma unroll
+                for (uint32_t c = 0; c < 8; ++c)
+                    if ((subm >> c) & 1u) {
+                        sChildH[t][c] = h[c];
+                        newm |= cr[c] << c;
+                    }
             }
             sSub[t] = subm;
             sChildNew[t] = newm;

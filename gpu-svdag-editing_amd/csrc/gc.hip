@@ -42,9 +42,9 @@ struct GcCounters {
 constexpr uint32_t kGcMaxTables = 20; // item sizes 2 .. 18 words use 17
 struct GcTables {
     TableDev t[kGcMaxTables];
-    uint8_t* visit[kGcMaxTables];
-    uint8_t* hasChain[kGcMaxTables]; // per-bucket "has overflow lines" bytes, or nullptr: walk every bucket
-    uint32_t* touched[kGcMaxTables]; // per-bucket bits: listed for the chain pass (zero between collections)
+    DevPtr<uint8_t> visit[kGcMaxTables];
+    DevPtr<uint8_t> hasChain[kGcMaxTables]; // per-bucket "has overflow lines" bytes, or nullptr: walk every bucket
+    DevPtr<uint32_t> touched[kGcMaxTables]; // per-bucket bits: listed for the chain pass (zero between collections)
 };
 
 // Clears the visit bytes of the lines handed out so far (16 bytes a line).
@@ -58,7 +58,7 @@ __global__ void __launch_bounds__(256) gc_clear_visits(GcTables a)
     if (blockIdx.x == 0 && threadIdx.x == 0 && t.alloc->freeCount < 0)
         t.alloc->freeCount = 0;
     uint4* v = reinterpret_cast<uint4*>(visit);
-    uint4* r = reinterpret_cast<uint4*>(t.roles);
+    uint4* r = reinterpret_cast<uint4*>((uint8_t*)t.roles);
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < fresh; i += (uint64_t)gridDim.x * blockDim.x) {
         v[i] = make_uint4(0u, 0u, 0u, 0u);
         r[i] = make_uint4(0u, 0u, 0u, 0u); // the mark sets the roles items are reached in
@@ -68,13 +68,13 @@ __global__ void __launch_bounds__(256) gc_clear_visits(GcTables a)
 // Visit (item, level): true if the caller is to expand the item at L (the
 // first visitor, or one of several simultaneous first visitors).  A stale
 // cached byte can only read as an earlier level, which also means "expand".
-__device__ inline uint8_t* gc_visit_byte(const DagDev& dag, uint8_t* const* visit, uint32_t h, bool leaf)
+__device__ inline uint8_t* gc_visit_byte(const DagDev& dag, const DevPtr<uint8_t>* visit, uint32_t h, bool leaf)
 {
     const uint32_t s = leaf ? leaf_handle_size(dag, h) : node_handle_size(h);
     const uint32_t ptr = leaf ? leaf_handle_ptr(dag, h) : node_handle_ptr(h); // slab * 16 + slot
     return &visit[s - 2][ptr];
 }
-__device__ inline bool gc_visit(const DagDev& dag, uint8_t* const* visit, uint32_t h, uint32_t L, bool leaf)
+__device__ inline bool gc_visit(const DagDev& dag, const DevPtr<uint8_t>* visit, uint32_t h, uint32_t L, bool leaf)
 {
     uint8_t* b = gc_visit_byte(dag, visit, h, leaf);
     const uint8_t lv = (uint8_t)(L + 1u);
@@ -84,7 +84,7 @@ __device__ inline bool gc_visit(const DagDev& dag, uint8_t* const* visit, uint32
     return true;
 }
 
-__global__ void gc_seed(DagDev dag, uint8_t* const* visit, const uint32_t* root, uint32_t* front, GcCounters* ctr)
+__global__ void gc_seed(DagDev dag, const DevPtr<uint8_t>* visit, const uint32_t* root, uint32_t* front, GcCounters* ctr)
 {
     if (threadIdx.x != 0 || blockIdx.x != 0)
         return;
@@ -130,7 +130,7 @@ __device__ inline void gc_flush_stage(uint32_t* sStage, uint32_t& sFill, uint32_
     __syncthreads();
 }
 
-__global__ void __launch_bounds__(256) gc_mark_level(DagDev dag, uint8_t* const* visit, uint32_t L,
+__global__ void __launch_bounds__(256) gc_mark_level(DagDev dag, const DevPtr<uint8_t>* visit, uint32_t L,
                                                      const uint32_t* in, uint32_t* out, uint32_t outCap,
                                                      GcCounters* ctr)
 {
@@ -318,7 +318,7 @@ __global__ void __launch_bounds__(256) gc_refs_clear(GcTables a, GcCounters* ctr
         return;
     const TableDev& t = a.t[blockIdx.y];
     const uint32_t fresh = min(t.alloc->fresh, t.slabCap);
-    uint4* r = reinterpret_cast<uint4*>(t.refs); // 64 bytes a line
+    uint4* r = reinterpret_cast<uint4*>((uint32_t*)t.refs); // 64 bytes a line
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < (uint64_t)fresh * 4u;
          i += (uint64_t)gridDim.x * blockDim.x)
         r[i] = make_uint4(0u, 0u, 0u, 0u);
@@ -334,7 +334,7 @@ __global__ void __launch_bounds__(256) gc_refs_count(DagDev dag, GcTables a, GcC
     for (uint32_t slab = blockIdx.x * blockDim.x + threadIdx.x; slab < fresh; slab += gridDim.x * blockDim.x) {
         const uint32_t* line = t.lines + (size_t)slab * kLineWords;
         const uint4 tv = *reinterpret_cast<const uint4*>(line);
-        const uint4 rv = reinterpret_cast<const uint4*>(t.roles)[slab];
+        const uint4 rv = reinterpret_cast<const uint4*>((const uint8_t*)t.roles)[slab];
         const uint32_t tw[4] = { tv.x, tv.y, tv.z, tv.w }, rw[4] = { rv.x, rv.y, rv.z, rv.w };
         for (uint32_t slot = 0; slot < t.slots; ++slot) {
             const uint32_t sh = 8u * (slot & 3u);
@@ -856,9 +856,9 @@ static int gc_mark_sweep(svdag_ctx* ctx, svdag_gc_stats* stats)
         for (size_t i = 0; i < nt; ++i)
             SVDAG_HIP(hipMemsetAsync(ctx->gcTouched[i], 0, (ctx->ts.tables[i].numBuckets + 31u) / 32u * 4, st));
         gc_clear_visits<<<dim3(grid_for(maxCap, 256, 1024), (uint32_t)nt), 256, 0, st>>>(a);
-        gc_seed<<<1, 64, 0, st>>>(dag, ctx->dGcMasks, ctx->dRoot, ctx->gcFront[0], ctr);
+        gc_seed<<<1, 64, 0, st>>>(dag, reinterpret_cast<const DevPtr<uint8_t>*>(ctx->dGcMasks), ctx->dRoot, ctx->gcFront[0], ctr);
         for (uint32_t L = 0; L < dag.leafLevel; ++L)
-            gc_mark_level<<<4096, 256, 0, st>>>(dag, ctx->dGcMasks, L, ctx->gcFront[L & 1],
+            gc_mark_level<<<4096, 256, 0, st>>>(dag, reinterpret_cast<const DevPtr<uint8_t>*>(ctx->dGcMasks), L, ctx->gcFront[L & 1],
                                                  ctx->gcFront[(L + 1) & 1], (uint32_t)cap, ctr);
         gc_sweep_lines<<<dim3(grid_for(maxCap, 256, 1024), (uint32_t)nt), 256, 0, st>>>(a, ctr);
         gc_sweep_chains<<<dim3(grid_for(maxBuckets, 256, 1024), (uint32_t)nt), 256, 0, st>>>(a, ctr);

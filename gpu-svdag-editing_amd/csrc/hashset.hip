@@ -50,12 +50,12 @@ int table_alloc(HostTable& t, uint32_t itemWords, uint32_t numBuckets, uint32_t 
     d.slabCap = slabCap;
     d.slots = line_slots(itemWords);
     d.tagWords = line_tag_words(d.slots);
-    SVDAG_HIP(hipMalloc(&d.lines, (size_t)slabCap * kLineWords * 4));
-    SVDAG_HIP(hipMalloc(&d.freeList, (size_t)slabCap * 4));
-    SVDAG_HIP(hipMalloc(&d.alloc, sizeof(AllocState)));
+    SVDAG_HIP(hipMalloc(d.lines.slot(), (size_t)slabCap * kLineWords * 4));
+    SVDAG_HIP(hipMalloc(d.freeList.slot(), (size_t)slabCap * 4));
+    SVDAG_HIP(hipMalloc(d.alloc.slot(), sizeof(AllocState)));
     if (withRefs) {
-        SVDAG_HIP(hipMalloc(&d.refs, (size_t)slabCap * kMaxSlots * 4));
-        SVDAG_HIP(hipMalloc(&d.roles, (size_t)slabCap * kMaxSlots));
+        SVDAG_HIP(hipMalloc(d.refs.slot(), (size_t)slabCap * kMaxSlots * 4));
+        SVDAG_HIP(hipMalloc(d.roles.slot(), (size_t)slabCap * kMaxSlots));
         SVDAG_HIP(hipMemsetAsync(d.refs, 0, (size_t)slabCap * kMaxSlots * 4, stream));
         SVDAG_HIP(hipMemsetAsync(d.roles, 0, (size_t)slabCap * kMaxSlots, stream));
     }

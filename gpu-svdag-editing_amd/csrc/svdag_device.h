@@ -103,14 +103,32 @@ struct AllocState {
     uint32_t pad;
 };
 
+// A pointer to device memory kept in memory (a descriptor, LDS).  The compiler
+// knows the address space of kernel arguments only; through a plain pointer
+// that it loads, every access is a flat one, which counts against the LDS
+// counter too and so is waited for at each barrier and LDS read.
+template <typename T>
+struct DevPtr {
+    __attribute__((address_space(1))) T* p;
+    __host__ __device__ operator T*() const { return (T*)p; }
+    __host__ __device__ DevPtr& operator=(T* q)
+    {
+        p = (__attribute__((address_space(1))) T*)q;
+        return *this;
+    }
+    __host__ __device__ T* operator->() const { return (T*)p; }
+    __host__ void** slot() { return reinterpret_cast<void**>(this); } // for hipMalloc
+};
+using DevWords = const __attribute__((address_space(1))) uint32_t*;
+
 // Every line that is not on a chain (the arena's never-used tail and the
 // free stack) is empty: tag words 0 and next = kNoSlab.
 struct TableDev {
-    uint32_t* lines;     // [slabCap][32]: tags, next, items
-    uint32_t* freeList;  // [slabCap] free stack of slab ids
-    AllocState* alloc;
-    uint32_t* refs;      // DAG tables: [slabCap][16] stored references to each slot's item
-    uint8_t* roles;      // DAG tables: [slabCap][16] kRoleParentOf* bits of each slot's item
+    DevPtr<uint32_t> lines;     // [slabCap][32]: tags, next, items
+    DevPtr<uint32_t> freeList;  // [slabCap] free stack of slab ids
+    DevPtr<AllocState> alloc;
+    DevPtr<uint32_t> refs;      // DAG tables: [slabCap][16] stored references to each slot's item
+    DevPtr<uint8_t> roles;      // DAG tables: [slabCap][16] kRoleParentOf* bits of each slot's item
     uint32_t itemWords;
     uint32_t numBuckets;
     uint32_t slabCap;
@@ -193,7 +211,7 @@ __device__ inline uint32_t slab_alloc_lanes(const TableDev& t, unsigned long lon
 __device__ inline uint32_t wave_slab_alloc(const TableDev& t, bool need)
 {
     unsigned long long pending = __ballot(need);
-    const uint64_t mine = (uint64_t)(uintptr_t)t.alloc;
+    const uint64_t mine = (uint64_t)(uintptr_t)t.alloc.p;
     uint32_t id = kNoSlab;
     while (pending != 0ull) {
         const int first = __ffsll((long long)pending) - 1;

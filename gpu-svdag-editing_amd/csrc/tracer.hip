@@ -150,14 +150,14 @@ __device__ inline HandleBits leaf_bits(const DagDev& dag)
 {
     return { 31u - dag.leafSizeBits, ~0u >> dag.leafSizeBits, dag.minLeafWords };
 }
-__device__ inline const uint32_t* item_address(const TraceShared& sh, const HandleBits& hb, uint32_t h)
+__device__ inline DevWords item_address(const TraceShared& sh, const HandleBits& hb, uint32_t h)
 {
     const uint32_t s = hb.minWords + ((h >> 1) >> hb.sizeShift);
     const uint32_t idx = h & hb.indexMask;
     const uint4 t = sh.table[s - 2u];
     const uint32_t slot = idx & ((1u << t.z) - 1u);
     const uint64_t base = (uint64_t)t.x | ((uint64_t)t.y << 32);
-    return reinterpret_cast<const uint32_t*>(base + (uint64_t)(idx >> t.z) * (kLineWords * 4u) + slot * s * 4u);
+    return reinterpret_cast<DevWords>(base + (uint64_t)(idx >> t.z) * (kLineWords * 4u) + slot * s * 4u);
 }
 
 // Child mask bit c moves to bit c ^ order: the children in visit order.
@@ -194,12 +194,12 @@ __device__ inline bool walk(const DagDev& dag, const TraceShared& sh, uint32_t r
     const uint32_t levels = dag.levels, leafLevel = dag.leafLevel;
     const ChildOrder co(ray);
     const HandleBits nb = node_bits(), lb = leaf_bits(dag);
-    const uint32_t* node = item_address(sh, nb, root);
+    DevWords node = item_address(sh, nb, root);
     uint32_t child = node[0] & 0xFFu;
     uint32_t left = co.sort(child & intersection_mask<true, kTame>(levels, 0, 0, 0, ray));
     uint32_t level = 0, pending = 0;
     uint32_t leafLo = 0, leafHi = 0;
-    const uint32_t* leaf = nullptr;
+    DevWords leaf = nullptr;
     x = y = z = 0;
     for (;;) {
         if (!left) {
@@ -208,7 +208,7 @@ __device__ inline bool walk(const DagDev& dag, const TraceShared& sh, uint32_t r
                 return false;
             level = 31u - (uint32_t)__clz((int)pending);
             const uint2 e = stk[level * kTraceBlock];
-            node = reinterpret_cast<const uint32_t*>((uint64_t)e.x | ((uint64_t)(e.y & 0xFFFFu) << 32));
+            node = reinterpret_cast<DevWords>((uint64_t)e.x | ((uint64_t)(e.y & 0xFFFFu) << 32));
             child = (e.y >> 16) & 0xFFu;
             left = e.y >> 24;
             const uint32_t keep = ~0u << (levels - level);
@@ -235,7 +235,7 @@ __device__ inline bool walk(const DagDev& dag, const TraceShared& sh, uint32_t r
             const bool isLeaf = level == leafLevel;
             const HandleBits hb { isLeaf ? lb.sizeShift : nb.sizeShift, isLeaf ? lb.indexMask : nb.indexMask,
                                   isLeaf ? lb.minWords : nb.minWords };
-            const uint32_t* item = item_address(sh, hb, h);
+            DevWords item = item_address(sh, hb, h);
             const uint32_t w0 = item[0], w1 = item[1]; // an item has at least two words
             if (isLeaf) {
                 leaf = item;
@@ -265,7 +265,7 @@ __device__ inline bool walk(const DagDev& dag, const TraceShared& sh, uint32_t r
     }
     const uint32_t v = ((x & 1u) << 2) | ((y & 1u) << 1) | (z & 1u) | ((x & 2u) << 4) | ((y & 2u) << 3) | ((z & 2u) << 2);
     uint32_t m;
-    material = leaf_material(leaf, v, dag.M, m) ? m : kSentinel;
+    material = leaf_material((const uint32_t*)leaf, v, dag.M, m) ? m : kSentinel;
     return true;
 }
 
