@@ -40,7 +40,8 @@ enum NState : uint32_t { NS_PARTIAL = 0, NS_FILLED = 1, NS_EMPTY = 2 };
 
 constexpr uint32_t kMaxLevels = 24;
 
-struct EditorDev {
+// What the sphere, box and paint tools decide by.
+struct EditGeom {
     uint32_t kind;
     uint32_t material;
     // sphere / paint
@@ -48,6 +49,8 @@ struct EditorDev {
     float radius, r2;
     // box and copy destination bounds
     float bmin[3], bmax[3];
+};
+struct EditorDev : EditGeom {
     // copy
     float d2s[3];
     int32_t id2s[3];
@@ -87,7 +90,7 @@ struct CopyState {
 __host__ __device__ inline float fmax_ref(float a, float b) { return a > b ? a : b; }
 __host__ __device__ inline float fmin_ref(float a, float b) { return a < b ? a : b; }
 
-__host__ __device__ inline bool sphere_overlap(const EditorDev& e, const float mn[3], const float mx[3])
+__host__ __device__ inline bool sphere_overlap(const EditGeom& e, const float mn[3], const float mx[3])
 {
     float dist = e.r2;
     const float c[3] = { e.cx, e.cy, e.cz };
@@ -103,7 +106,7 @@ __host__ __device__ inline bool sphere_overlap(const EditorDev& e, const float m
     return dist > 0.0f;
 }
 
-__host__ __device__ inline bool sphere_contained(const EditorDev& e, const float mn[3], const float mx[3])
+__host__ __device__ inline bool sphere_contained(const EditGeom& e, const float mn[3], const float mx[3])
 {
     const float c[3] = { e.cx, e.cy, e.cz };
     float m[3];
@@ -156,9 +159,10 @@ __host__ __device__ inline uint32_t band_material(const EditorDev& e, uint32_t x
     return (e.material + (y >> b) + (h & 3u)) & e.materialMask;
 }
 
-// should_edit for the stateless tools (and the copy tool's voxel level).
-__device__ inline Op decide(const EditorDev& e, uint32_t x, uint32_t y, uint32_t z, uint32_t depth, NState st,
-                            uint32_t& fillMat)
+// should_edit for the sphere, box and paint tools and the copy tool's voxel
+// level.
+__device__ inline Op decide_geom(const EditGeom& e, uint32_t x, uint32_t y, uint32_t z, uint32_t depth, NState st,
+                                 uint32_t& fillMat)
 {
     float mn[3], mx[3];
     node_box(x, y, z, depth, mn, mx);
@@ -194,6 +198,16 @@ __device__ inline Op decide(const EditorDev& e, uint32_t x, uint32_t y, uint32_t
     }
     case EK_COPY:
         return box_overlap(e.bmin, e.bmax, mn, mx) ? OP_SUBDIVIDE : OP_KEEP;
+    default:
+        return OP_KEEP;
+    }
+}
+
+// should_edit for the stateless tools (and the copy tool's voxel level).
+__device__ inline Op decide(const EditorDev& e, uint32_t x, uint32_t y, uint32_t z, uint32_t depth, NState st,
+                            uint32_t& fillMat)
+{
+    switch (e.kind) {
     case EK_DENSE: {
         // A cell of one material is filled with it, an empty cell is empty,
         // a mixed cell is subdivided.  Nodes larger than the grid hold it at
@@ -240,7 +254,7 @@ __device__ inline Op decide(const EditorDev& e, uint32_t x, uint32_t y, uint32_t
         return OP_SUBDIVIDE;
     }
     default:
-        return OP_KEEP;
+        return decide_geom(e, x, y, z, depth, st, fillMat);
     }
 }
 

@@ -126,7 +126,7 @@ constexpr uint32_t kParItems = kParEdits * kSpineItems;
 constexpr uint32_t kParThreads = kSmallBlock;
 
 struct SpineItem {
-    uint32_t x, y, z, orig; // position at its level; its handle in the wave's input DAG
+    uint32_t x, y, z;       // position at its level
     uint32_t sub;           // children this edit subdivides
     uint32_t dep;           // paint: children whose decision read their state (empty or not)
     uint32_t ref[8];        // per subdivided child: its item one level down, or its seed work item at S
@@ -157,7 +157,9 @@ __global__ void __launch_bounds__(kParThreads) fused_spine_par(WsDev ws, DagDev 
                                                                uint32_t* rootPtr, EditStatus* status,
                                                                LevelDesc* levels)
 {
-    __shared__ uint32_t sPos[kParItems][3], sSubCnt[kParItems];
+    __shared__ uint32_t sPos[kParItems][3];
+    __shared__ uint4 sItem[2][kParItems]; // top-down: a level's positions and input-DAG handles, by level parity
+    __shared__ uint32_t sCnt[2][kParEdits];
     __shared__ uint32_t sSub[kParItems], sChildNew[kParItems], sChildH[kParItems][8];
     __shared__ uint32_t sPosHash[2 * kParItems], sPosOf[kParItems], sPrev[kParItems];
     __shared__ unsigned long long sPosEdits[kParItems];
@@ -173,19 +175,20 @@ __global__ void __launch_bounds__(kParThreads) fused_spine_par(WsDev ws, DagDev 
     SpineScratch& sc = *reinterpret_cast<SpineScratch*>(f.spine);
     const EditStatus joint = *ws.status;
     if (t == 0) {
-        uint32_t ok = K >= 1 && K <= kParEdits && S >= 1 && S <= leafLevel && !joint.overflow && !joint.oom;
-        for (uint32_t k = 0; ok && k < K; ++k) {
-            const uint32_t kind = eds[wv.x + k].kind;
-            ok = kind == EK_SPHERE_ADD || kind == EK_SPHERE_REMOVE || kind == EK_BOX_ADD || kind == EK_BOX_REMOVE
-                || kind == EK_PAINT;
-        }
-        sOk = ok;
+        sOk = K >= 1 && K <= kParEdits && S >= 1 && S <= leafLevel && !joint.overflow && !joint.oom;
         sBad = 0u;
         sh.oom = 0u;
         sh.inserted = 0u;
     }
     __syncthreads();
-    if (!sOk)
+    if (sOk && t < K) {
+        const uint32_t kind = eds[wv.x + t].kind;
+        if (!(kind == EK_SPHERE_ADD || kind == EK_SPHERE_REMOVE || kind == EK_BOX_ADD || kind == EK_BOX_REMOVE
+              || kind == EK_PAINT))
+            atomicOr(&sBad, 1u);
+    }
+    __syncthreads();
+    if (!sOk || sBad)
         return; // the sequential spine takes the wave
     const uint32_t root0 = *rootPtr;
     // An edit's level may end up without items (an edit off the volume
@@ -193,98 +196,100 @@ __global__ void __launch_bounds__(kParThreads) fused_spine_par(WsDev ws, DagDev 
     for (uint32_t q = t; q < K * kMaxLevels; q += blockDim.x)
         sc.cnt[q / kMaxLevels][q % kMaxLevels] = q % kMaxLevels == 0u ? 1u : 0u;
     if (t < K) {
-        SpineItem& it = sc.item[t][0][0];
-        it.x = it.y = it.z = 0u;
-        it.orig = root0;
+        sItem[0][t * kSpineItems] = make_uint4(0u, 0u, 0u, root0);
+        sCnt[0][t] = 1u;
         sDropped[t] = ws.edCount[(wv.x + t) * kMaxLevels + leafLevel] == 0u ? 1u : 0u;
     }
     __syncthreads();
 
-    // ---- top-down: every edit's spine items on levels 0 .. S-1.
-    const uint32_t k = t >> 3, i = t & 7u; // one (edit, item) pair per thread
+    // ---- top-down: every edit's spine items on levels 0 .. S-1, eight lanes
+    // per item, one per child (13 us a level with one thread per item).
     for (uint32_t l = 0; l < S; ++l) {
-        uint32_t sub = 0, dep = 0, origChild[8];
-        const bool active = k < K && i < sc.cnt[k][l];
-        if (active) {
-            SpineItem& it = sc.item[k][l][i];
-            const EditorDev& ed = eds[wv.x + k];
-            uint32_t mask = 0;
-            const uint32_t* node = nullptr;
-            if (it.orig != kSentinel) {
-                node = dag_node_ptr(dag, it.orig);
-                mask = node[0] & 0xFFu;
-            }
-            const bool paint = ed.kind == EK_PAINT;
-            for (uint32_t c = 0; c < 8; ++c) {
-                origChild[c] = ((mask >> c) & 1u) ? node[1 + __builtin_popcount(mask & ((1u << c) - 1u))] : kSentinel;
-                const uint32_t cx = (it.x << 1) | ((c >> 2) & 1u), cy = (it.y << 1) | ((c >> 1) & 1u),
-                               cz = (it.z << 1) | (c & 1u);
+        const uint32_t par = l & 1u, c = t & 7u;
+        for (uint32_t p = t >> 3; p < K * kSpineItems; p += kParThreads / 8u) {
+            const uint32_t pk = p / kSpineItems, pi = p % kSpineItems;
+            const bool active = pi < sCnt[par][pk];
+            uint32_t child = kSentinel;
+            bool sub = false, dep = false;
+            uint4 item = make_uint4(0u, 0u, 0u, kSentinel);
+            if (active) {
+                item = sItem[par][p];
+                const EditGeom ed = eds[wv.x + pk];
+                if (item.w != kSentinel) {
+                    const uint32_t* node = dag_node_ptr(dag, item.w);
+                    const uint32_t mask = node[0] & 0xFFu;
+                    if ((mask >> c) & 1u)
+                        child = node[1 + __builtin_popcount(mask & ((1u << c) - 1u))];
+                }
                 // Sphere and box decide by geometry alone above S.  Paint
                 // reads the child's state (svo_inner_level's NodeDesc), here
                 // from the wave's input DAG; the bottom-up checks that the
                 // edits before it in the wave left that state as it was.
+                const bool paint = ed.kind == EK_PAINT;
                 NState st = NS_PARTIAL;
                 uint32_t stMat = 0;
                 if (paint) {
-                    if (origChild[c] == kSentinel)
+                    if (child == kSentinel)
                         st = NS_EMPTY;
                     else if (l + 1u != leafLevel)
-                        st = header_full(dag_node_ptr(dag, origChild[c])[0], dag.M, stMat) ? NS_FILLED : NS_PARTIAL;
+                        st = header_full(dag_node_ptr(dag, child)[0], dag.M, stMat) ? NS_FILLED : NS_PARTIAL;
                 }
                 uint32_t fm = 0;
-                const Op op = decide(ed, cx, cy, cz, dag.levels - (l + 1), st, fm);
-                if (op == OP_SUBDIVIDE)
-                    sub |= 1u << c;
-                else if (!(op == OP_KEEP || (paint && op == OP_EMPTY && st == NS_EMPTY)))
+                const Op op = decide_geom(ed, (item.x << 1) | ((c >> 2) & 1u), (item.y << 1) | ((c >> 1) & 1u),
+                                          (item.z << 1) | (c & 1u), dag.levels - (l + 1), st, fm);
+                sub = op == OP_SUBDIVIDE;
+                if (!(sub || op == OP_KEEP || (paint && op == OP_EMPTY && st == NS_EMPTY)))
                     atomicOr(&sBad, 1u); // a fill above S: the sequential spine takes the wave
-                if (paint && op != OP_KEEP)
-                    dep |= 1u << c;
+                dep = paint && op != OP_KEEP;
             }
-            it.sub = sub;
-            it.dep = dep;
-            for (uint32_t c = 0; c < 8; ++c)
-                it.och[c] = origChild[c];
-        }
-        if (t < kParItems)
-            sSubCnt[t] = active ? (uint32_t)__builtin_popcount(sub) : 0u;
-        __syncthreads();
-        if (active) {
-            SpineItem& it = sc.item[k][l][i];
-            uint32_t n = 0;
-            for (uint32_t q = 0; q < i; ++q)
-                n += sSubCnt[k * kSpineItems + q];
-            const SeedDesc sd = f.seeds[wv.x + k];
-            for (uint32_t c = 0; c < 8; ++c) {
-                if (!((sub >> c) & 1u))
-                    continue;
-                const uint32_t cx = (it.x << 1) | ((c >> 2) & 1u), cy = (it.y << 1) | ((c >> 1) & 1u),
-                               cz = (it.z << 1) | (c & 1u);
-                if (l + 1 < S) {
-                    if (n < kSpineItems) {
-                        SpineItem& ch = sc.item[k][l + 1][n];
-                        ch.x = cx;
-                        ch.y = cy;
-                        ch.z = cz;
-                        ch.orig = origChild[c];
-                    } else {
-                        atomicOr(&sBad, 1u);
-                    }
-                    it.ref[c] = n++;
-                } else {
-                    const uint32_t dx = cx - sd.lo[0], dy = cy - sd.lo[1], dz = cz - sd.lo[2];
-                    const bool inRange = dx < sd.n[0] && dy < sd.n[1] && dz < sd.n[2];
-                    const uint32_t w = inRange ? f.seedWork[(wv.x + k) * 8 + ((dx << 2) | (dy << 1) | dz)] : kSentinel;
-                    if (w == kSentinel)
-                        atomicOr(&sBad, 1u);
-                    it.ref[c] = w;
+            const uint32_t subm = group_ballot<8>(sub, t & 56u), depm = group_ballot<8>(dep, t & 56u);
+            sChildH[p][c] = child;
+            if (c == 0)
+                sSub[p] = subm;
+            if (active) {
+                SpineItem& it = sc.item[pk][l][pi];
+                it.och[c] = child;
+                if (c == 0) {
+                    it.x = item.x;
+                    it.y = item.y;
+                    it.z = item.z;
+                    it.sub = subm;
+                    it.dep = depm;
                 }
             }
-            if (i == 0 && l + 1 < S) {
-                uint32_t tot = 0;
-                for (uint32_t q = 0; q < kSpineItems; ++q)
-                    tot += sSubCnt[k * kSpineItems + q];
-                sc.cnt[k][l + 1] = tot < kSpineItems ? tot : kSpineItems;
-                if (tot > kSpineItems)
+        }
+        __syncthreads();
+        for (uint32_t p = t >> 3; p < K * kSpineItems; p += kParThreads / 8u) {
+            const uint32_t pk = p / kSpineItems, pi = p % kSpineItems;
+            uint32_t before = 0, total = 0;
+            for (uint32_t q = 0; q < kSpineItems; ++q) {
+                const uint32_t n = (uint32_t)__builtin_popcount(sSub[pk * kSpineItems + q]);
+                before += q < pi ? n : 0u;
+                total += n;
+            }
+            const uint32_t subm = sSub[p];
+            if ((subm >> c) & 1u) {
+                const uint4 item = sItem[par][p];
+                const uint32_t cx = (item.x << 1) | ((c >> 2) & 1u), cy = (item.y << 1) | ((c >> 1) & 1u),
+                               cz = (item.z << 1) | (c & 1u);
+                uint32_t ref = before + (uint32_t)__builtin_popcount(subm & ((1u << c) - 1u));
+                if (l + 1 < S) {
+                    if (ref < kSpineItems)
+                        sItem[par ^ 1u][pk * kSpineItems + ref] = make_uint4(cx, cy, cz, sChildH[p][c]);
+                } else {
+                    const SeedDesc sd = f.seeds[wv.x + pk];
+                    const uint32_t dx = cx - sd.lo[0], dy = cy - sd.lo[1], dz = cz - sd.lo[2];
+                    const bool inRange = dx < sd.n[0] && dy < sd.n[1] && dz < sd.n[2];
+                    ref = inRange ? f.seedWork[(wv.x + pk) * 8 + ((dx << 2) | (dy << 1) | dz)] : kSentinel;
+                    if (ref == kSentinel)
+                        atomicOr(&sBad, 1u);
+                }
+                sc.item[pk][l][pi].ref[c] = ref;
+            }
+            if (pi == 0 && c == 0 && l + 1 < S) {
+                sCnt[par ^ 1u][pk] = total < kSpineItems ? total : kSpineItems;
+                sc.cnt[pk][l + 1] = total < kSpineItems ? total : kSpineItems;
+                if (total > kSpineItems)
                     atomicOr(&sBad, 1u);
             }
         }
@@ -292,6 +297,7 @@ __global__ void __launch_bounds__(kParThreads) fused_spine_par(WsDev ws, DagDev 
         if (sBad)
             return; // nothing written outside the scratch: the sequential spine takes the wave
     }
+    const uint32_t k = t >> 3, i = t & 7u; // one (edit, item) pair per thread from here on
 
     // ---- bottom-up: levels S-1 .. 0, every edit's nodes of a level at once.
     // An item of the SVO does not change any more, so the next level's is

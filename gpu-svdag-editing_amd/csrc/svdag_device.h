@@ -170,8 +170,8 @@ __device__ inline unsigned long long lanes_below()
     return l ? (~0ull >> (64u - l)) : 0ull;
 }
 
-// Slabs for the lanes of mask m, all of one table: one atomic on the
-// free-stack count and at most one on the bump counter.
+// Slabs for the lanes of mask m (each lane's own), all of one table: one
+// atomic on the free-stack count and at most one on the bump counter.
 __device__ inline uint32_t slab_alloc_lanes(const TableDev& t, unsigned long long m)
 {
     const uint32_t k = (uint32_t)__popcll(m);
@@ -205,14 +205,14 @@ __device__ inline uint32_t slab_alloc_lanes(const TableDev& t, unsigned long lon
 
 // A slab for every active lane that passes need = true, from that lane's
 // table.  Lanes of one wave may insert into different tables (items of
-// different sizes), so requests are served one table at a time, each with
-// one aggregated allocation.  Lanes passing false get kNoSlab; kNoSlab with
-// oom set when the arena is exhausted.
+// different sizes): the lanes of each table are gathered first, then all
+// tables allocate at once, each with one aggregated allocation.  Lanes
+// passing false get kNoSlab; kNoSlab with oom set when the arena is exhausted.
 __device__ inline uint32_t wave_slab_alloc(const TableDev& t, bool need)
 {
     unsigned long long pending = __ballot(need);
     const uint64_t mine = (uint64_t)(uintptr_t)t.alloc.p;
-    uint32_t id = kNoSlab;
+    unsigned long long together = 0ull;
     while (pending != 0ull) {
         const int first = __ffsll((long long)pending) - 1;
         const uint32_t lo = (uint32_t)__shfl((int)(uint32_t)mine, first, 64);
@@ -221,9 +221,9 @@ __device__ inline uint32_t wave_slab_alloc(const TableDev& t, bool need)
         const unsigned long long m = __ballot(take);
         pending &= ~m;
         if (take)
-            id = slab_alloc_lanes(t, m);
+            together = m;
     }
-    return id;
+    return need ? slab_alloc_lanes(t, together) : kNoSlab;
 }
 
 // Push the slabs of the active lanes passing give = true (one atomic per
