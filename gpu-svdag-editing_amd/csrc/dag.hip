@@ -139,13 +139,59 @@ __global__ void edit_begin(WsDev ws, const uint32_t* root, uint32_t isCopy, uint
 // per-edit counts of a fused wave go through an LDS histogram (the edits of
 // a wave are at most 256 consecutive indices, so e & 255 is a unique key)
 // flushed once per block.
-template <bool kMulti>
-__global__ void __launch_bounds__(256) svo_inner_level(WsDev ws, DagDev dag, const EditorDev* eds, uint32_t L)
+// Work items of a wave64 block share one reservation on the level's counter,
+// one word that every block queues on (about 13 ns each): blocks of 1024
+// threads take 128 items at a time, and the grid is capped at the thread count
+// that blocks of 256 had.  The deepest level of a 16-edit wave at depth 15 takes
+// 23 us, 60 with blocks of 256; a copy's levels take 8-19 us, 6-34 before its
+// source lists were kept as candidate bits until a child's slot is known.
+constexpr uint32_t kSvoBlock = 1024;
+
+__device__ inline CopyParent copy_parent(const WsDev& ws, uint32_t w, int k)
 {
-    __shared__ uint32_t waveTotal[4];
+    const uint4 v = reinterpret_cast<const uint4*>(ws.state + w)[k];
+    return CopyParent { v.x, v.y, v.z, v.w };
+}
+// Entries behind the list's end are not read.
+__device__ inline void end_copy_list(CopyParent (&par)[8])
+{
+    bool live = true;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        live = live && par[k].h != kSentinel;
+        if (!live)
+            par[k].h = kSentinel;
+    }
+}
+// Work item g's source parents: the first eight candidates of item w's.
+__device__ inline void write_copy_list(const WsDev& ws, const TableDev* sTab, uint32_t w, uint32_t g, CopyCand cand)
+{
+    uint4* out = reinterpret_cast<uint4*>(ws.state + g);
+#pragma unroll
+    for (int n = 0; n < 8; ++n) {
+        uint4 v = make_uint4(0u, 0u, 0u, kSentinel);
+        if (cand != 0ull) {
+            const uint32_t b = (uint32_t)__ffsll((long long)cand) - 1u;
+            cand &= cand - 1ull;
+            const uint32_t c = b & 7u;
+            const CopyParent par = copy_parent(ws, w, (int)(b >> 3));
+            const uint32_t* node = staged_node(sTab, par.h);
+            const uint32_t mask = node[0] & 0xFFu;
+            v = make_uint4((par.x << 1) | ((c >> 2) & 1u), (par.y << 1) | ((c >> 1) & 1u), (par.z << 1) | (c & 1u),
+                           node[1 + __builtin_popcount(mask & ((1u << c) - 1u))]);
+        }
+        out[n] = v;
+    }
+}
+
+template <bool kMulti>
+__global__ void __launch_bounds__(kSvoBlock) svo_inner_level(WsDev ws, DagDev dag, const EditorDev* eds, uint32_t L)
+{
+    __shared__ uint32_t waveTotal[kSvoBlock / 64u];
     __shared__ uint32_t blockBase;
     __shared__ uint32_t hist[kMulti ? 256 : 1];
     __shared__ uint32_t histEdit[kMulti ? 256 : 1];
+    __shared__ TableDev sTab[kRefTables];
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wv = threadIdx.x >> 6;
     const uint32_t c = lane & 7u;
@@ -154,27 +200,30 @@ __global__ void __launch_bounds__(256) svo_inner_level(WsDev ws, DagDev dag, con
     const uint32_t childStart = me.start + me.count;
     if (blockIdx.x == 0 && threadIdx.x == 0)
         ws.lvl[L + 1].start = childStart;
-    if (kMulti) {
-        hist[threadIdx.x] = 0u;
-        __syncthreads();
-    }
-    const uint32_t childLevel = L + 1;
-    const uint32_t childDepth = dag.levels - childLevel;
-    const bool leafChildren = childLevel == dag.leafLevel;
-    const uint32_t groupsPerBlock = blockDim.x / 8u;
+    const uint32_t groupsPerBlock = kSvoBlock / 8u;
     // After an overflow the count may run past the array; the edit is
     // discarded then, but no lane may read or write beyond capWork.
     const uint32_t count = me.start >= ws.capWork ? 0u : min(me.count, ws.capWork - me.start);
+    if (blockIdx.x * groupsPerBlock >= count)
+        return;
+    tables_stage(sTab, dag);
+    if (kMulti && threadIdx.x < 256u)
+        hist[threadIdx.x] = 0u;
+    __syncthreads();
+    const uint32_t childLevel = L + 1;
+    const uint32_t childDepth = dag.levels - childLevel;
+    const bool leafChildren = childLevel == dag.leafLevel;
     for (uint32_t i0 = blockIdx.x * groupsPerBlock; i0 < count; i0 += gridDim.x * groupsPerBlock) {
         const uint32_t i = i0 + threadIdx.x / 8u;
         const bool active = i < count;
         const uint32_t w = me.start + (active ? i : 0u);
         const uint32_t e = (kMulti && active) ? ws.editOf[w] : 0u;
         const EditorDev& ed = eds[e];
+        const EditGeom geom = ed; // loaded beside the item, not where it is used
         const uint4 item = active ? ws.work[w] : make_uint4(0u, 0u, 0u, kSentinel);
         uint32_t childHandle = kSentinel;
         if (item.w != kSentinel) {
-            const uint32_t* node = dag_node_ptr(dag, item.w);
+            const uint32_t* node = staged_node(sTab, item.w);
             const uint32_t mask = node[0] & 0xFFu;
             if ((mask >> c) & 1u)
                 childHandle = node[1 + __builtin_popcount(mask & ((1u << c) - 1u))];
@@ -188,14 +237,23 @@ __global__ void __launch_bounds__(256) svo_inner_level(WsDev ws, DagDev dag, con
         // skip the child header read.
         if (childHandle == kSentinel)
             st = NS_EMPTY;
-        else if (!leafChildren && ed.kind == EK_PAINT)
-            st = header_full(dag_node_ptr(dag, childHandle)[0], dag.M, stMat) ? NS_FILLED : NS_PARTIAL;
+        else if (!leafChildren && geom.kind == EK_PAINT)
+            st = header_full(staged_node(sTab, childHandle)[0], dag.M, stMat) ? NS_FILLED : NS_PARTIAL;
         uint32_t fillMat = 0;
         Op op = OP_KEEP;
-        CopyState cs;
+        CopyCand cand = 0ull;
         if (active) {
-            if (ed.kind == EK_COPY)
-                op = decide_copy(ed, dag, cx, cy, cz, childDepth, ws.state[w], cs);
+            if (kMulti) // a wave holds sphere, box and paint edits
+                op = decide_geom(geom, cx, cy, cz, childDepth, st, fillMat);
+            else if (geom.kind == EK_COPY) {
+                CopyParent par[8];
+#pragma unroll
+                for (int k = 0; k < 8; ++k)
+                    par[k] = copy_parent(ws, w, k);
+                end_copy_list(par);
+                op = decide_copy(ed, cx, cy, cz, childDepth, par,
+                                 [&](uint32_t h) { return staged_node(sTab, h)[0]; }, cand);
+            }
             else
                 op = decide(ed, cx, cy, cz, childDepth, st, fillMat);
         }
@@ -208,7 +266,7 @@ __global__ void __launch_bounds__(256) svo_inner_level(WsDev ws, DagDev dag, con
         __syncthreads();
         if (threadIdx.x == 0) {
             uint32_t tot = 0;
-            for (uint32_t k = 0; k < blockDim.x / 64u; ++k)
+            for (uint32_t k = 0; k < kSvoBlock / 64u; ++k)
                 tot += waveTotal[k];
             blockBase = tot ? atomicAdd(&ws.lvl[L + 1].count, tot) : 0u;
         }
@@ -227,8 +285,8 @@ __global__ void __launch_bounds__(256) svo_inner_level(WsDev ws, DagDev dag, con
                 ws.work[g] = make_uint4(cx, cy, cz, childHandle);
                 if (kMulti)
                     ws.editOf[g] = e;
-                if (ed.kind == EK_COPY)
-                    ws.state[g] = cs;
+                if (!kMulti && geom.kind == EK_COPY)
+                    write_copy_list(ws, sTab, w, g, cand);
             } else {
                 atomicOr(&ws.status->overflow, 1u);
             }
@@ -256,7 +314,7 @@ __global__ void __launch_bounds__(256) svo_inner_level(WsDev ws, DagDev dag, con
     }
     if (kMulti) {
         __syncthreads();
-        const uint32_t v = hist[threadIdx.x];
+        const uint32_t v = threadIdx.x < 256u ? hist[threadIdx.x] : 0u;
         if (v)
             atomicAdd(&ws.edCount[histEdit[threadIdx.x] * kMaxLevels + L + 1], v);
     }
@@ -274,10 +332,60 @@ constexpr uint32_t kLeafWordsPerLane = (18u + kLeafLanes - 1u) / kLeafLanes; // 
 
 __device__ inline void dedup_clear(const WsDev& ws, uint32_t count, uint32_t tid, uint32_t stride);
 
+// Voxels of a leaf an edit covers, for the sphere, box and paint tools: at
+// voxel size their decisions (fill, empty or subdivide) all take the tool's
+// new value, so only the overlap counts.  Voxel v of a lane is voxel
+// v * kLeafLanes + s of the leaf; its x and y follow v, its z is the lane's.
+// The overlap's arithmetic is sphere_overlap's, whose axis terms are
+// subtracted in turn: a zero gap subtracts nothing.
+struct LeafCover {
+    uint32_t bits; // bit v: voxel v is covered
+    __device__ LeafCover(const EditGeom& g, const uint4& item, uint32_t s)
+    {
+        static_assert(kLeafLanes == 16, "voxel v of a lane: x bit 1 of v, y bit 0 of v");
+        const uint32_t x0 = (item.x << 2) | ((s >> 2) & 1u), y0 = (item.y << 2) | ((s >> 1) & 1u);
+        const uint32_t z = (item.z << 2) | (((s >> 3) & 1u) << 1) | (s & 1u);
+        bits = 0u;
+        if (g.kind == EK_BOX_ADD || g.kind == EK_BOX_REMOVE) {
+#pragma unroll
+            for (uint32_t v = 0; v < 4; ++v) {
+                const float mn[3] = { (float)(x0 + (v & 2u)), (float)(y0 + 2u * (v & 1u)), (float)z };
+                const float mx[3] = { mn[0] + 1.0f, mn[1] + 1.0f, mn[2] + 1.0f };
+                bits |= box_overlap(g.bmin, g.bmax, mn, mx) ? 1u << v : 0u;
+            }
+            return;
+        }
+        auto gap = [](float c, float mn) {
+            const float mx = mn + 1.0f;
+            return c < mn ? c - mn : (c > mx ? c - mx : 0.0f);
+        };
+        const float dz = gap(g.cz, (float)z);
+#pragma unroll
+        for (uint32_t x = 0; x < 2; ++x) {
+            const float dx = gap(g.cx, (float)(x0 + 2u * x));
+            const float tx = fmaf(-dx, dx, g.r2);
+#pragma unroll
+            for (uint32_t y = 0; y < 2; ++y) {
+                const float dy = gap(g.cy, (float)(y0 + 2u * y));
+                bits |= fmaf(-dz, dz, fmaf(-dy, dy, tx)) > 0.0f ? 1u << (2u * x + y) : 0u;
+            }
+        }
+    }
+};
+
+// Bound: the trips of a leaf (work item, then its old words and its editor's
+// geometry, then the stores) and the voxel decisions.  The sixteen lanes of a
+// leaf load its old words together and share them in LDS, and the table
+// descriptors are there too.  The leaf level of a 16-edit wave at depth 15
+// takes 52-57 us, 115 with sixteen lanes that each read and decided their own
+// voxels through the general tool code.
 template <bool kMulti>
 __global__ void __launch_bounds__(256) svo_leaf_level(WsDev ws, DagDev dag, const EditorDev* eds)
 {
     __shared__ uint32_t lds[4][kLeavesPerWave][16];
+    __shared__ uint32_t old[4][kLeavesPerWave][kLeafWordsPerLane * kLeafLanes];
+    __shared__ TableDev sTab[kRefTables];
+    __shared__ uint4 parents[kMulti ? 1 : 4][kLeavesPerWave][8]; // copy edits: a leaf's source leaves
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wv = threadIdx.x >> 6;
     const uint32_t seg = lane / kLeafLanes, s = lane % kLeafLanes;
@@ -286,26 +394,51 @@ __global__ void __launch_bounds__(256) svo_leaf_level(WsDev ws, DagDev dag, cons
     const uint32_t count = min(me.count, ws.capLeaf);
     // The merge starts at this level: an empty dedup table for it.
     dedup_clear(ws, count, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x);
+    if (blockIdx.x * wavesPerBlock * kLeavesPerWave >= count)
+        return;
+    tables_stage(sTab, dag);
+    __syncthreads();
     for (uint32_t i0 = (blockIdx.x * wavesPerBlock + wv) * kLeavesPerWave; i0 < count;
          i0 += gridDim.x * wavesPerBlock * kLeavesPerWave) {
         const uint32_t i = i0 + seg;
         const uint32_t w = me.start + i;
         const bool valid = i < count && w < ws.capWork;
-        uint32_t has4 = 0, mats[kLeavesPerWave];
+        uint32_t has4 = 0, mats[kLeavesPerWave], ow[kLeafWordsPerLane];
 #pragma unroll
         for (uint32_t v = 0; v < kLeavesPerWave; ++v)
             mats[v] = 0u;
-        uint32_t oldH = kSentinel;
-        const uint32_t* oldLeaf = nullptr;
+#pragma unroll
+        for (uint32_t k = 0; k < kLeafWordsPerLane; ++k)
+            ow[k] = 0u;
+        uint32_t oldH = kSentinel, e = 0;
+        uint4 item = make_uint4(0u, 0u, 0u, kSentinel);
+        EditGeom geom {};
         if (valid) {
-            const EditorDev& ed = eds[kMulti ? ws.editOf[w] : 0u];
-            const uint4 item = ws.work[w];
+            e = kMulti ? ws.editOf[w] : 0u;
+            item = ws.work[w];
+            geom = eds[e];
             oldH = item.w;
-            uint64_t oldBits = 0;
             if (oldH != kSentinel) {
-                oldLeaf = dag_leaf_ptr(dag, oldH);
-                oldBits = (uint64_t)oldLeaf[0] | ((uint64_t)oldLeaf[1] << 32);
+                const uint32_t* oldLeaf = staged_leaf(sTab, dag, oldH);
+                const uint32_t oldSize = leaf_handle_size(dag, oldH);
+#pragma unroll
+                for (uint32_t k = 0; k < kLeafWordsPerLane; ++k)
+                    if (s + kLeafLanes * k < oldSize)
+                        ow[k] = oldLeaf[s + kLeafLanes * k];
             }
+            if (!kMulti && geom.kind == EK_COPY && s < 8u)
+                parents[wv][seg][s] = reinterpret_cast<const uint4*>(ws.state + w)[s];
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < kLeafWordsPerLane; ++k)
+            old[wv][seg][s + kLeafLanes * k] = ow[k];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (valid) {
+            const uint32_t (&oldWords)[kLeafWordsPerLane * kLeafLanes] = old[wv][seg];
+            const uint64_t oldBits = (uint64_t)oldWords[0] | ((uint64_t)oldWords[1] << 32);
+            const bool geometric = kMulti || geom.kind <= EK_PAINT;
+            const LeafCover cover(geom, item, s);
 #pragma unroll
             for (uint32_t v = 0; v < kLeavesPerWave; ++v) {
                 const uint32_t b = v * kLeafLanes + s;
@@ -313,28 +446,38 @@ __global__ void __launch_bounds__(256) svo_leaf_level(WsDev ws, DagDev dag, cons
                 uint32_t oldMat = 0;
                 if (hasOld && dag.M) {
                     const uint32_t off = (uint32_t)__builtin_popcountll(oldBits & ((1ull << b) - 1ull)) * dag.M;
-                    oldMat = (oldLeaf[2 + (off >> 5)] >> (off & 31u)) & ((1u << dag.M) - 1u);
+                    oldMat = (oldWords[2 + (off >> 5)] >> (off & 31u)) & ((1u << dag.M) - 1u);
                 }
-                const uint32_t vx = (item.x << 2) | (((b >> 5) & 1u) << 1) | ((b >> 2) & 1u);
-                const uint32_t vy = (item.y << 2) | (((b >> 4) & 1u) << 1) | ((b >> 1) & 1u);
-                const uint32_t vz = (item.z << 2) | (((b >> 3) & 1u) << 1) | (b & 1u);
-                uint32_t fm;
-                const Op op = decide(ed, vx, vy, vz, 0, hasOld ? NS_FILLED : NS_EMPTY, fm);
-                bool has = false;
-                uint32_t mat = 0;
-                if (ed.kind == EK_DENSE || ed.kind == EK_TERRAIN) {
-                    // a set voxel of the grid or below the surface, with its own material;
-                    // a tiled terrain keeps voxels outside its tile
-                    has = op == OP_FILL || (op == OP_KEEP && hasOld);
-                    mat = op == OP_FILL ? fm : oldMat;
-                } else if (op == OP_FILL || op == OP_SUBDIVIDE) {
-                    if (ed.kind == EK_COPY)
-                        has = copy_value(ed, dag, vx, vy, vz, ws.state[w], hasOld, oldMat, mat);
-                    else
-                        has = new_value(ed, hasOld, oldMat, mat);
-                } else if (op == OP_KEEP) {
-                    has = hasOld;
-                    mat = oldMat;
+                bool has = hasOld;
+                uint32_t mat = oldMat;
+                if (geometric) {
+                    if ((cover.bits >> v) & 1u) {
+                        has = geom.kind == EK_SPHERE_ADD || geom.kind == EK_BOX_ADD || (geom.kind == EK_PAINT && hasOld);
+                        mat = has ? geom.material : 0u;
+                    }
+                } else {
+                    const EditorDev& ed = eds[e];
+                    const uint32_t vx = (item.x << 2) | (((b >> 5) & 1u) << 1) | ((b >> 2) & 1u);
+                    const uint32_t vy = (item.y << 2) | (((b >> 4) & 1u) << 1) | ((b >> 1) & 1u);
+                    const uint32_t vz = (item.z << 2) | (((b >> 3) & 1u) << 1) | (b & 1u);
+                    uint32_t fm;
+                    const Op op = decide(ed, vx, vy, vz, 0, hasOld ? NS_FILLED : NS_EMPTY, fm);
+                    if (ed.kind != EK_COPY) {
+                        // a set voxel of the grid or below the surface, with its own material;
+                        // a tiled terrain keeps voxels outside its tile
+                        has = op == OP_FILL || (op == OP_KEEP && hasOld);
+                        mat = op == OP_FILL ? fm : oldMat;
+                    } else if (op == OP_SUBDIVIDE) {
+                        CopyParent par[8];
+#pragma unroll
+                        for (int k = 0; k < 8; ++k) {
+                            const uint4 q = parents[kMulti ? 0 : wv][seg][k];
+                            par[k] = CopyParent { q.x, q.y, q.z, q.w };
+                        }
+                        mat = 0;
+                        has = copy_value(ed, dag, vx, vy, vz, par, [&](uint32_t h) { return staged_leaf(sTab, dag, h); },
+                                         hasOld, oldMat, mat);
+                    }
                 }
                 has4 |= (has ? 1u : 0u) << v;
                 mats[v] = mat;
@@ -383,7 +526,7 @@ __global__ void __launch_bounds__(256) svo_leaf_level(WsDev ws, DagDev dag, cons
 #pragma unroll
                 for (uint32_t k = 0; k < kLeafWordsPerLane; ++k) {
                     const uint32_t q = s + kLeafLanes * k;
-                    if (q < newSize && oldLeaf[q] != word[k])
+                    if (q < newSize && ow[k] != word[k])
                         differ = true;
                 }
             }
@@ -403,7 +546,7 @@ __global__ void __launch_bounds__(256) svo_leaf_level(WsDev ws, DagDev dag, cons
             }
             const uint64_t offs = __ballot(off);
             if (valid && s == 0u && ((offs >> (kLeafLanes * seg)) & ((1ull << kLeafLanes) - 1ull)) == 0ull)
-                set_flag(kMulti ? &ws.edFull[ws.editOf[w] * kMaxLevels + dag.leafLevel] : &ws.lvl[dag.leafLevel].fullCount);
+                set_flag(kMulti ? &ws.edFull[e * kMaxLevels + dag.leafLevel] : &ws.lvl[dag.leafLevel].fullCount);
         }
         const uint64_t diff = __ballot(differ);
         const bool unchanged = cmp && ((diff >> (kLeafLanes * seg)) & ((1ull << kLeafLanes) - 1ull)) == 0ull;
@@ -1398,7 +1541,7 @@ int launch_edit(svdag_ctx* ctx, const EditorDev& ed, const EditorDev* edDev, con
     for (uint32_t L = 0; L <= dag.leafLevel; ++L)
         items[L] = std::min<uint64_t>(level_bound(ctx, b, L), L == dag.leafLevel ? ws.capLeaf : ws.capWork);
     for (uint32_t L = 0; L < dag.leafLevel; ++L)
-        svo_inner_level<false><<<grid_for(items[L], 32, kCap), 256, 0, st>>>(ws, dag, edDev, L);
+        svo_inner_level<false><<<grid_for(items[L], kSvoBlock / 8u, std::max(1u, kCap / 4u)), kSvoBlock, 0, st>>>(ws, dag, edDev, L);
     svo_leaf_level<false><<<grid_for(items[dag.leafLevel], 4 * kLeavesPerWave, kCap), 256, 0, st>>>(ws, dag, edDev);
     launch_merge_levels<false>(ctx, ws, 0, items, kCap);
     edit_finish<<<1, 64, 0, st>>>(ws, dag, ctx->dRoot);
@@ -1416,7 +1559,7 @@ int launch_joint_levels(svdag_ctx* ctx, const WsDev& ws, const EditorDev* eds, u
         items[L] = std::min<uint64_t>(levelItems[L], L == dag.leafLevel ? ws.capLeaf : ws.capWork);
     if (part != 2) {
         for (uint32_t L = S; L < dag.leafLevel; ++L)
-            svo_inner_level<true><<<grid_for(items[L], 32, kCap), 256, 0, st>>>(ws, dag, eds, L);
+            svo_inner_level<true><<<grid_for(items[L], kSvoBlock / 8u, std::max(1u, kCap / 4u)), kSvoBlock, 0, st>>>(ws, dag, eds, L);
         svo_leaf_level<true><<<grid_for(items[dag.leafLevel], 4 * kLeavesPerWave, kCap), 256, 0, st>>>(ws, dag, eds);
     }
     // The build above only reads items the root reaches; the merge below

@@ -302,114 +302,98 @@ __host__ __device__ inline void rot_source(const EditorDev& e, const int64_t v[3
         s[a] = s[a] > 0 ? s[a] : 0;
 }
 
-// Rotated copy, node level.  The node's destination voxels inside the edit
-// box are an integer range; its image under rot_source (both corners mapped,
-// then ordered) is the source range, and the children of the parents'
-// source nodes that overlap it are the next parents.  Integer arithmetic
-// throughout, so every destination voxel's source lies in a collected parent.
-__device__ inline Op decide_copy_rot(const EditorDev& e, const DagDev& dag, uint32_t x, uint32_t y, uint32_t z,
-                                     uint32_t depth, const CopyState& in, CopyState& out)
+// Children of the copy tool's source parents that a node needs, 8 bits per
+// parent, in parent and child order; at most the first eight count.
+using CopyCand = unsigned long long;
+// Child mask from one pair of flags per axis: bit 0 (1) of a flag says that
+// children at the parent's low (high) half on that axis qualify.
+__device__ inline uint32_t octant_mask(uint32_t fx, uint32_t fy, uint32_t fz)
 {
-    for (int k = 0; k < 8; ++k)
-        out.p[k].h = kSentinel;
-    const uint32_t p[3] = { x, y, z };
-    int64_t lo[3], hi[3];
-    for (int a = 0; a < 3; ++a) {
-        const int64_t n0 = (int64_t)p[a] << depth;
-        const int64_t n1 = n0 + ((int64_t)1 << depth) - 1;
-        lo[a] = n0 > e.ivmin[a] ? n0 : e.ivmin[a];
-        hi[a] = n1 < e.ivmax[a] ? n1 : e.ivmax[a];
-        if (lo[a] > hi[a])
-            return OP_KEEP;
-    }
-    int64_t a0[3], a1[3], slo[3], shi[3];
-    rot_source(e, lo, a0);
-    rot_source(e, hi, a1);
-    for (int a = 0; a < 3; ++a) {
-        slo[a] = a0[a] < a1[a] ? a0[a] : a1[a];
-        shi[a] = a0[a] < a1[a] ? a1[a] : a0[a];
-    }
-    int nOut = 0;
-    for (int k = 0; k < 8; ++k) {
-        const CopyParent& par = in.p[k];
-        if (par.h == kSentinel)
-            break;
-        const uint32_t* node = dag_node_ptr(dag, par.h);
-        const uint32_t mask = node[0] & 0xFFu;
-        for (uint32_t c = 0; c < 8; ++c) {
-            if (!(mask & (1u << c)))
-                continue;
-            const uint32_t cp[3] = { (par.x << 1) | ((c >> 2) & 1u), (par.y << 1) | ((c >> 1) & 1u),
-                                     (par.z << 1) | (c & 1u) };
-            bool ov = true;
-            for (int a = 0; a < 3; ++a) {
-                const int64_t c0 = (int64_t)cp[a] << depth;
-                const int64_t c1 = c0 + ((int64_t)1 << depth) - 1;
-                ov = ov && c0 <= shi[a] && c1 >= slo[a];
-            }
-            if (ov && nOut < 8) {
-                out.p[nOut].x = cp[0];
-                out.p[nOut].y = cp[1];
-                out.p[nOut].z = cp[2];
-                out.p[nOut].h = node[1 + __builtin_popcount(mask & ((1u << c) - 1u))];
-                ++nOut;
-            }
-        }
-    }
-    return nOut == 0 ? OP_KEEP : OP_SUBDIVIDE;
+    const uint32_t mx = (fx & 1u ? 0x0Fu : 0u) | (fx & 2u ? 0xF0u : 0u);
+    const uint32_t my = (fy & 1u ? 0x33u : 0u) | (fy & 2u ? 0xCCu : 0u);
+    const uint32_t mz = (fz & 1u ? 0x55u : 0u) | (fz & 2u ? 0xAAu : 0u);
+    return mx & my & mz;
 }
 
-// Copy tool, stateful should_edit for an inner-level child at childDepth:
-// collects the source children of the parent's source nodes that overlap the
-// shifted destination region (my_gpu_dag_editors.h:173-217).
-__device__ inline Op decide_copy(const EditorDev& e, const DagDev& dag, uint32_t x, uint32_t y, uint32_t z,
-                                 uint32_t depth, const CopyState& in, CopyState& out)
+// Copy tool, stateful should_edit for an inner-level child at childDepth: the
+// source children of the parent's source nodes that overlap the shifted
+// destination region (my_gpu_dag_editors.h:173-217).  Both tests are one
+// interval per axis, so a parent's children need two of them per axis, and
+// all parents' headers (header(k)) are read at once; the children's handles
+// are read by whoever keeps the node.
+// Rotated: the node's destination voxels inside the edit box are an integer
+// range; its image under rot_source (both corners mapped, then ordered) is
+// the source range.  Integer arithmetic throughout, so every destination
+// voxel's source lies in a collected parent.
+template <typename Header>
+__device__ inline Op decide_copy(const EditorDev& e, uint32_t x, uint32_t y, uint32_t z, uint32_t depth,
+                                 const CopyParent (&in)[8], Header&& header, CopyCand& cand)
 {
-    if (e.rot)
-        return decide_copy_rot(e, dag, x, y, z, depth, in, out);
-    float mn[3], mx[3];
-    node_box(x, y, z, depth, mn, mx);
-    for (int k = 0; k < 8; ++k)
-        out.p[k].h = kSentinel;
-    if (!box_overlap(e.bmin, e.bmax, mn, mx))
-        return OP_KEEP;
-    const float size = (float)(1u << depth);
-    float smn[3], smx[3];
-    for (int a = 0; a < 3; ++a) {
-        smn[a] = fmax_ref(mn[a], e.bmin[a]) + e.d2s[a];
-        smx[a] = fmin_ref(smn[a] + size, e.bmax[a] + e.d2s[a]);
-    }
-    int nOut = 0;
-    for (int k = 0; k < 8; ++k) {
-        const CopyParent& par = in.p[k];
-        if (par.h == kSentinel)
-            break;
-        const uint32_t* node = dag_node_ptr(dag, par.h);
-        const uint32_t mask = node[0] & 0xFFu;
-        for (uint32_t c = 0; c < 8; ++c) {
-            if (!(mask & (1u << c)))
-                continue;
-            const uint32_t cx = (par.x << 1) | ((c >> 2) & 1u);
-            const uint32_t cy = (par.y << 1) | ((c >> 1) & 1u);
-            const uint32_t cz = (par.z << 1) | (c & 1u);
-            float cmn[3], cmx[3];
-            node_box(cx, cy, cz, depth, cmn, cmx);
-            if (aabb_overlap(cmn, cmx, smn, smx) && nOut < 8) {
-                out.p[nOut].x = cx;
-                out.p[nOut].y = cy;
-                out.p[nOut].z = cz;
-                out.p[nOut].h = node[1 + __builtin_popcount(mask & ((1u << c) - 1u))];
-                ++nOut;
-            }
+    cand = 0ull;
+    float mn[3], mx[3], smn[3], smx[3];
+    int64_t clo[3], chi[3]; // rotated: source children [clo, chi] per axis
+    if (e.rot) {
+        const uint32_t p[3] = { x, y, z };
+        int64_t lo[3], hi[3];
+        for (int a = 0; a < 3; ++a) {
+            const int64_t n0 = (int64_t)p[a] << depth;
+            const int64_t n1 = n0 + ((int64_t)1 << depth) - 1;
+            lo[a] = n0 > e.ivmin[a] ? n0 : e.ivmin[a];
+            hi[a] = n1 < e.ivmax[a] ? n1 : e.ivmax[a];
+            if (lo[a] > hi[a])
+                return OP_KEEP;
+        }
+        int64_t a0[3], a1[3];
+        rot_source(e, lo, a0);
+        rot_source(e, hi, a1);
+        for (int a = 0; a < 3; ++a) { // rot_source is never negative
+            clo[a] = (a0[a] < a1[a] ? a0[a] : a1[a]) >> depth;
+            chi[a] = (a0[a] < a1[a] ? a1[a] : a0[a]) >> depth;
+        }
+    } else {
+        node_box(x, y, z, depth, mn, mx);
+        if (!box_overlap(e.bmin, e.bmax, mn, mx))
+            return OP_KEEP;
+        const float size = (float)(1u << depth);
+        for (int a = 0; a < 3; ++a) {
+            smn[a] = fmax_ref(mn[a], e.bmin[a]) + e.d2s[a];
+            smx[a] = fmin_ref(smn[a] + size, e.bmax[a] + e.d2s[a]);
         }
     }
-    return nOut == 0 ? OP_KEEP : OP_SUBDIVIDE;
+    uint32_t mask[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+        mask[k] = in[k].h == kSentinel ? 0u : header(in[k].h) & 0xFFu;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        const uint32_t pp[3] = { in[k].x, in[k].y, in[k].z };
+        uint32_t f[3] = { 0u, 0u, 0u };
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+#pragma unroll
+            for (uint32_t half = 0; half < 2; ++half) {
+                const uint32_t cp = (pp[a] << 1) | half;
+                bool ok;
+                if (e.rot) {
+                    ok = (int64_t)cp >= clo[a] && (int64_t)cp <= chi[a];
+                } else { // one axis of aabb_overlap(child box, [smn, smx))
+                    const float cmn = (float)(cp << depth);
+                    const float cmx = cmn + (float)(1u << depth);
+                    ok = !(cmn >= smx[a] || cmx <= smn[a] || smn[a] >= cmx || smx[a] <= cmn);
+                }
+                f[a] |= ok ? 1u << half : 0u;
+            }
+        }
+        cand |= (CopyCand)(mask[k] & octant_mask(f[0], f[1], f[2])) << (8 * k);
+    }
+    return cand == 0ull ? OP_KEEP : OP_SUBDIVIDE;
 }
 
 // Copy tool voxel value (my_gpu_dag_editors.h:225-252): the source voxel's
 // material if set, else the old value; the source position clamps at 0.
+template <typename Leaf>
 __device__ inline bool copy_value(const EditorDev& e, const DagDev& dag, uint32_t vx, uint32_t vy, uint32_t vz,
-                                  const CopyState& st, bool hasOld, uint32_t oldMat, uint32_t& mat)
+                                  const CopyParent (&par)[8], Leaf&& leaf, bool hasOld, uint32_t oldMat, uint32_t& mat)
 {
     int32_t s[3];
     if (e.rot) {
@@ -427,20 +411,22 @@ __device__ inline bool copy_value(const EditorDev& e, const DagDev& dag, uint32_
             s[a] = s[a] > 0 ? s[a] : 0;
     }
     const uint32_t px = (uint32_t)s[0] >> 2, py = (uint32_t)s[1] >> 2, pz = (uint32_t)s[2] >> 2;
-    const CopyParent* found = nullptr;
+    // The list ends at the first kSentinel.
+    uint32_t found = kSentinel;
+    bool live = true;
+#pragma unroll
     for (int k = 0; k < 8; ++k) {
-        if (st.p[k].h == kSentinel)
-            break;
-        if (st.p[k].x == px && st.p[k].y == py && st.p[k].z == pz)
-            found = &st.p[k];
+        live = live && par[k].h != kSentinel;
+        if (live && par[k].x == px && par[k].y == py && par[k].z == pz)
+            found = par[k].h;
     }
     mat = oldMat;
-    if (!found)
+    if (found == kSentinel)
         return hasOld;
     const uint32_t bit = (((uint32_t)s[0] & 1u) << 2) | (((uint32_t)s[1] & 1u) << 1) | ((uint32_t)s[2] & 1u)
         | (((uint32_t)s[0] & 2u) << 4) | (((uint32_t)s[1] & 2u) << 3) | (((uint32_t)s[2] & 2u) << 2);
     uint32_t m;
-    if (leaf_material(dag_leaf_ptr(dag, found->h), bit, dag.M, m)) {
+    if (leaf_material(leaf(found), bit, dag.M, m)) {
         mat = m;
         return true;
     }

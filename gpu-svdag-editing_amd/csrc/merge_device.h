@@ -16,6 +16,15 @@ __device__ inline void tables_stage(TableDev* sTab, const DagDev& dag)
         dst[i] = src[i];
 }
 
+__device__ inline const uint32_t* staged_node(const TableDev* sTab, uint32_t h)
+{
+    return table_item_ptr(sTab[node_handle_size(h) - 2u], node_handle_ptr(h));
+}
+__device__ inline const uint32_t* staged_leaf(const TableDev* sTab, const DagDev& dag, uint32_t h)
+{
+    return table_item_ptr(sTab[leaf_handle_size(dag, h) - 2u], leaf_handle_ptr(dag, h));
+}
+
 // Reference counts summed per block before they reach the tables.
 constexpr uint32_t kRefSlots = 2048; // 256 items have at most 2048 children
 template <uint32_t kSlots>
