@@ -30,6 +30,18 @@ __global__ void table_init_lines(TableDev t, uint32_t first, uint32_t last)
     }
 }
 
+// The same for every table of a set (blockIdx.y), all lines.
+__global__ void tables_init_lines(const TableDev* tables)
+{
+    const TableDev t = tables[blockIdx.y];
+    const size_t n = (size_t)t.slabCap * kLineWords;
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
+        const uint32_t w = (uint32_t)(i % kLineWords);
+        if (w <= t.tagWords)
+            t.lines[i] = w == t.tagWords ? kNoSlab : 0u;
+    }
+}
+
 int table_alloc(HostTable& t, uint32_t itemWords, uint32_t numBuckets, uint32_t slabCap, hipStream_t stream,
                 bool withRefs)
 {
@@ -807,6 +819,12 @@ int require_device()
 
 struct svdag_hashset {
     TableSet ts;
+    // One allocation holds every table (see hashset_tables): 17 tables of their
+    // own lines, free lists and states cost 51 allocations and as many
+    // synchronising frees, 4.4 of the 6.0 ms that filling, probing and releasing
+    // 3 M items of 2-18 words took.
+    void* arena = nullptr;
+    AllocState* states = nullptr; // [tables], in the arena
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     hipEvent_t regionStart = nullptr, regionEnd = nullptr; // svdag_hashset_timer
@@ -865,6 +883,62 @@ int svdag_device_synchronize(void)
     return SVDAG_OK;
 }
 
+// The set's tables in one allocation: line arrays, then the allocator states
+// side by side (one copy reads them all), the descriptors and the segment
+// buffer.  A set's slabs are never freed, so there are no free lists.
+static int hashset_tables(svdag_hashset* hs, const uint32_t* buckets, const uint32_t* reserve)
+{
+    TableSet& ts = hs->ts;
+    const uint32_t n = ts.maxWords - ts.minWords + 1;
+    ts.tables.resize(n);
+    std::vector<AllocState> states(n);
+    std::vector<size_t> at(n);
+    size_t bytes = 0;
+    for (uint32_t i = 0; i < n; ++i) {
+        HostTable& t = ts.tables[i];
+        const uint32_t s = ts.minWords + i;
+        const uint32_t nb = std::max(1u, buckets[i]);
+        const uint64_t res = reserve ? reserve[i] : 0;
+        // Overflow reserve: equal-hash items (bulk multiset inserts) need a
+        // line per `slots` at worst; in a table sized for 75% of its slots
+        // about a fifth of the buckets overflow into a second line.
+        const uint32_t slots = line_slots(s);
+        uint64_t cap = (uint64_t)nb + res / slots + nb / 2 + 64;
+        cap = std::min<uint64_t>(cap, (1ull << (32 - kSlotBits)));
+        if (cap < nb) {
+            set_error("table_alloc: bad size");
+            return SVDAG_E_INVALID;
+        }
+        t.itemWords = t.dev.itemWords = s;
+        t.numBuckets = t.dev.numBuckets = nb;
+        t.slabCap = t.dev.slabCap = (uint32_t)cap;
+        t.dev.slots = slots;
+        t.dev.tagWords = line_tag_words(slots);
+        states[i] = AllocState { nb, 0, 0u, 0u };
+        at[i] = bytes;
+        bytes += (size_t)cap * kLineWords * 4;
+    }
+    const size_t statesAt = bytes, descAt = statesAt + ((n * sizeof(AllocState) + 255) & ~(size_t)255);
+    const size_t segAt = descAt + ((n * sizeof(TableDev) + 255) & ~(size_t)255);
+    SVDAG_HIP(hipMalloc(&hs->arena, segAt + 64 * 5 * 4));
+    uint8_t* base = static_cast<uint8_t*>(hs->arena);
+    hs->states = reinterpret_cast<AllocState*>(base + statesAt);
+    hs->segBuf = reinterpret_cast<uint32_t*>(base + segAt);
+    ts.devTables = reinterpret_cast<TableDev*>(base + descAt);
+    uint32_t most = 1;
+    for (uint32_t i = 0; i < n; ++i) {
+        ts.tables[i].dev.lines = reinterpret_cast<uint32_t*>(base + at[i]);
+        ts.tables[i].dev.alloc = hs->states + i;
+        most = std::max(most, ts.tables[i].slabCap);
+    }
+    SVDAG_HIP(hipMemcpyAsync(hs->states, states.data(), n * sizeof(AllocState), hipMemcpyHostToDevice, hs->stream));
+    SVDAG_TRY(ts.upload(hs->stream));
+    tables_init_lines<<<dim3(grid_for((uint64_t)most * kLineWords, 256, 4096), n), 256, 0, hs->stream>>>(ts.devTables);
+    SVDAG_HIP(hipGetLastError());
+    SVDAG_HIP(hipStreamSynchronize(hs->stream));
+    return SVDAG_OK;
+}
+
 int svdag_hashset_create(uint32_t minWords, uint32_t maxWords, const uint32_t* buckets, const uint32_t* reserve,
                          svdag_hashset** out)
 {
@@ -874,33 +948,21 @@ int svdag_hashset_create(uint32_t minWords, uint32_t maxWords, const uint32_t* b
     }
     SVDAG_TRY(require_device());
     auto* hs = new svdag_hashset();
-    SVDAG_HIP(hipStreamCreateWithFlags(&hs->stream, hipStreamNonBlocking));
-    SVDAG_HIP(hipEventCreate(&hs->ev0));
-    SVDAG_HIP(hipEventCreate(&hs->ev1));
-    SVDAG_HIP(hipEventCreate(&hs->regionStart));
-    SVDAG_HIP(hipEventCreate(&hs->regionEnd));
-    SVDAG_HIP(hipMalloc(&hs->segBuf, 64 * 5 * 4));
     hs->ts.minWords = minWords;
     hs->ts.maxWords = maxWords;
-    hs->ts.tables.resize(maxWords - minWords + 1);
-    for (uint32_t s = minWords; s <= maxWords; ++s) {
-        const uint32_t nb = std::max(1u, buckets[s - minWords]);
-        const uint64_t res = reserve ? reserve[s - minWords] : 0;
-        // Overflow reserve: equal-hash items (bulk multiset inserts) need a
-        // line per `slots` at worst; in a table sized for 75% of its slots
-        // about a fifth of the buckets overflow into a second line.
-        const uint32_t slots = line_slots(s);
-        uint64_t cap = (uint64_t)nb + res / slots + nb / 2 + 64;
-        cap = std::min<uint64_t>(cap, (1ull << (32 - kSlotBits)));
-        int r = table_alloc(hs->ts.tables[s - minWords], s, nb, (uint32_t)cap, hs->stream);
-        if (r != SVDAG_OK) {
-            hs->ts.release();
-            delete hs;
-            return r;
-        }
+    auto make = [&]() -> int {
+        SVDAG_HIP(hipStreamCreateWithFlags(&hs->stream, hipStreamNonBlocking));
+        SVDAG_HIP(hipEventCreate(&hs->ev0));
+        SVDAG_HIP(hipEventCreate(&hs->ev1));
+        SVDAG_HIP(hipEventCreate(&hs->regionStart));
+        SVDAG_HIP(hipEventCreate(&hs->regionEnd));
+        return hashset_tables(hs, buckets, reserve);
+    };
+    const int r = make();
+    if (r != SVDAG_OK) {
+        (void)svdag_hashset_destroy(hs);
+        return r;
     }
-    SVDAG_TRY(hs->ts.upload(hs->stream));
-    SVDAG_HIP(hipStreamSynchronize(hs->stream));
     *out = hs;
     return SVDAG_OK;
 }
@@ -909,17 +971,21 @@ int svdag_hashset_destroy(svdag_hashset* hs)
 {
     if (!hs)
         return SVDAG_OK;
-    (void)hipStreamSynchronize(hs->stream);
-    hs->ts.release();
+    if (hs->stream)
+        (void)hipStreamSynchronize(hs->stream);
     hs->bins.release();
-    (void)hipFree(hs->segBuf);
-    (void)hipEventDestroy(hs->ev0);
-    (void)hipEventDestroy(hs->ev1);
+    if (hs->arena)
+        (void)hipFree(hs->arena);
+    if (hs->ev0)
+        (void)hipEventDestroy(hs->ev0);
+    if (hs->ev1)
+        (void)hipEventDestroy(hs->ev1);
     if (hs->regionStart)
         (void)hipEventDestroy(hs->regionStart);
     if (hs->regionEnd)
         (void)hipEventDestroy(hs->regionEnd);
-    (void)hipStreamDestroy(hs->stream);
+    if (hs->stream)
+        (void)hipStreamDestroy(hs->stream);
     delete hs;
     return SVDAG_OK;
 }
@@ -947,9 +1013,11 @@ static int hashset_bulk(svdag_hashset* hs, const uint32_t* words, const svdag_se
             return hashset_bulk(hs, words, segs, nseg, out, variant % 100, ms, insert);
     }
     if (insert) {
-        for (auto& t : hs->ts.tables) {
-            AllocState a {};
-            SVDAG_TRY(table_read_alloc(t, a, hs->stream));
+        std::vector<AllocState> states(hs->ts.tables.size());
+        SVDAG_HIP(hipMemcpyAsync(states.data(), hs->states, states.size() * sizeof(AllocState), hipMemcpyDeviceToHost,
+                                 hs->stream));
+        SVDAG_HIP(hipStreamSynchronize(hs->stream));
+        for (const AllocState& a : states) {
             if (a.oom) {
                 set_error("slab arena exhausted during bulk insert");
                 return SVDAG_E_OOM;
