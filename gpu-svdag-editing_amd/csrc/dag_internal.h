@@ -361,9 +361,10 @@ int gc_enqueue_stream(svdag_ctx* ctx, uint32_t first, uint32_t count, const std:
                       uint32_t* fail, void** ctrOut, hipStream_t st);
 void gc_stream_take(svdag_ctx* ctx, const void* counters, uint32_t roots);
 size_t gc_counters_bytes();
-// surfDev (optional) receives one surface code per pixel (see dSurf).
+// surfDev (optional) receives one surface code per pixel (see dSurf), hostDev
+// (optional) the hits once more (see direct_host in tracer.hip).
 int launch_trace(svdag_ctx* ctx, const svdag_camera& cam, uint32_t W, uint32_t H, uint32_t root, hipStream_t stream,
-                 svdag_hit* outDev, uint8_t* surfDev = nullptr);
+                 svdag_hit* outDev, uint8_t* surfDev = nullptr, svdag_hit* hostDev = nullptr);
 // Run edits [0, n) in order on ctx->stream (one sync at the end), with the
 // overflow / OOM retry; used by svdag_edit, svdag_edit_batch and the server.
 int run_edits(svdag_ctx* ctx, const EditorDev* eds, uint32_t n, svdag_edit_stats* stats, float* totalMs);

@@ -380,7 +380,11 @@ typedef struct {
     double bounds_min[3];
     double bounds_max[3];
 } svdag_camera;
-/* One hit record per pixel, stored at row (height-1-y) like the reference. */
+/* One hit record per pixel, stored at row (height-1-y) like the reference.
+ * Where the results of this and the other frame passes go to pinned memory
+ * (hits: 16-byte aligned) and gpu_ms is NULL, the kernels store them there
+ * themselves; otherwise they are copied when the pass has ended, and gpu_ms
+ * is the pass without the copy. */
 typedef struct {
     uint32_t x, y, z;          /* hit voxel path (0,0,0 on a miss) */
     uint32_t material;         /* material id, 0xFFFFFFFF on a miss */
