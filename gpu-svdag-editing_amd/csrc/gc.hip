@@ -23,7 +23,7 @@
 // items and marks the buckets that have overflow lines; a pass over those
 // chains unlinks the overflow lines left without items and pushes them on
 // the slab free stack.
-#include "dag_internal.h"
+#include "merge_device.h"
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
@@ -415,10 +415,12 @@ struct ReleaseItem {
     bool chained;
 };
 
-__device__ inline ReleaseItem rc_load(const DagDev& dag, bool load, uint2 e)
+// tabs: the tables' descriptors in LDS; from memory they were a round trip
+// before the item's and another before its children's counts.
+__device__ inline ReleaseItem rc_load(const TableDev* tabs, bool load, uint2 e)
 {
     ReleaseItem r {};
-    const TableDev& t = dag.tables[e.x];
+    const TableDev& t = tabs[e.x];
     const uint32_t s = e.x + 2u;
     const uint32_t* item = load ? table_item_ptr(t, e.y) : nullptr;
     r.roles = load ? t.roles[e.y] : 0u;
@@ -435,17 +437,53 @@ __device__ inline ReleaseItem rc_load(const DagDev& dag, bool load, uint2 e)
     return r;
 }
 
+// A round's output list in memory.
+struct ListOut {
+    uint2* out;
+    uint32_t* count;
+    uint32_t cap;
+    __device__ uint32_t reserve(uint32_t n) const { return atomicAdd(count, n); }
+    __device__ bool put(uint32_t at, uint2 e) const
+    {
+        if (at < cap)
+            out[at] = e;
+        return at < cap;
+    }
+};
+
+// The same for rounds that stay in one block: the first entries in LDS.
+constexpr uint32_t kSmallRelease = 512;
+struct SmallRelease {
+    uint2 list[2][kSmallRelease + 1]; // the last takes what does not fit
+    uint32_t count[kMaxLevels];
+};
+struct BlockOut {
+    SmallRelease& s;
+    uint32_t round; // that the list is the input of
+    uint2* out;
+    uint32_t cap;
+    __device__ uint32_t reserve(uint32_t n) const { return atomicAdd(&s.count[round], n); }
+    __device__ bool put(uint32_t at, uint2 e) const
+    {
+        s.list[round & 1u][min(at, kSmallRelease)] = e;
+        if (at >= kSmallRelease && at < cap)
+            out[at] = e;
+        return at < cap;
+    }
+};
+
 // Releases item e (have) whose words v were read: frees its slot, lists an
 // overflow line's bucket once for the chain pass, and takes one count from
 // each child of each counted role; the children that reach zero go to the
 // output list.  The slot's free and the listing are issued alongside the
 // children's count loads, so each wave waits once per step: the counts, the
 // decrements, the appends.  Every lane of the wave calls it.
-__device__ inline void rc_release_loaded(const DagDev& dag, const GcTables& a, uint32_t rootTable, uint32_t rootPtr,
-                                         bool have, uint2 e, ReleaseItem v, uint2* out, uint32_t* outCount,
-                                         uint32_t cap, uint2* touchedList, GcCounters* ctr)
+template <typename Out>
+__device__ inline void rc_release_loaded(const DagDev& dag, const TableDev* tabs, const GcTables& a, uint32_t rootTable,
+                                         uint32_t rootPtr, bool have, uint2 e, ReleaseItem v, Out out, uint32_t cap,
+                                         uint2* touchedList, GcCounters* ctr)
 {
-    const TableDev& t = dag.tables[e.x];
+    const TableDev& t = tabs[e.x];
     const uint32_t s = e.x + 2u;
     const bool chained = have && v.chained;
     uint32_t tbit = 0, told = 0;
@@ -479,7 +517,7 @@ __device__ inline void rc_release_loaded(const DagDev& dag, const GcTables& a, u
                 const uint32_t ch = v.cw[j];
                 const uint32_t cs = lf ? leaf_handle_size(dag, ch) : node_handle_size(ch);
                 ce[j] = make_uint2(cs - 2u, lf ? leaf_handle_ptr(dag, ch) : node_handle_ptr(ch));
-                cp[j] = &dag.tables[ce[j].x].refs[ce[j].y];
+                cp[j] = &tabs[ce[j].x].refs[ce[j].y];
                 cv[j] = ld_filter(cp[j]);
             }
         }
@@ -523,16 +561,14 @@ __device__ inline void rc_release_loaded(const DagDev& dag, const GcTables& a, u
         uint32_t base0 = 0;
         if (total != 0u) {
             if (__lane_id() == 63u)
-                base0 = atomicAdd(outCount, total);
+                base0 = out.reserve(total);
             base0 = (uint32_t)__shfl((int)base0, 63, 64);
         }
         uint32_t at = base0 + incl - cnt;
 #pragma unroll
         for (uint32_t j = 0; j < 8; ++j) {
             if ((die >> j) & 1u) {
-                if (at < cap)
-                    out[at] = ce[j];
-                else
+                if (!out.put(at, ce[j]))
                     atomicOr(&ctr->overflow, 1u);
                 ++at;
             }
@@ -560,6 +596,9 @@ __global__ void __launch_bounds__(256) rc_release_roots(DagDev dag, GcTables a, 
                                                         uint32_t* outCount, uint32_t cap, uint2* touchedList,
                                                         GcCounters* ctr)
 {
+    __shared__ TableDev sTab[kGcMaxTables];
+    tables_stage(sTab, dag);
+    __syncthreads();
     // A pop past the free stack's end leaves its count below zero; the chain
     // pass pushes onto an empty stack then.
     if (blockIdx.x == 0 && threadIdx.x < dag.numTables && dag.tables[threadIdx.x].alloc->freeCount < 0)
@@ -574,13 +613,14 @@ __global__ void __launch_bounds__(256) rc_release_roots(DagDev dag, GcTables a, 
             const uint32_t hs = leaf ? leaf_handle_size(dag, h) : node_handle_size(h);
             e = make_uint2(hs - 2u, leaf ? leaf_handle_ptr(dag, h) : node_handle_ptr(h));
         }
-        const uint32_t refs = in ? dag.tables[e.x].refs[e.y] : 1u;
-        const ReleaseItem v = rc_load(dag, in, e);
+        const uint32_t refs = in ? sTab[e.x].refs[e.y] : 1u;
+        const ReleaseItem v = rc_load(sTab, in, e);
         const bool dies = in && refs == 0u;
         const unsigned long long m = __ballot(dies);
         if (m != 0ull && __lane_id() == (uint32_t)__ffsll((long long)m) - 1u)
             atomicAdd(&ctr->count[0], (uint32_t)__popcll(m));
-        rc_release_loaded(dag, a, rootTable, rootPtr, dies, e, v, out, outCount, cap, touchedList, ctr);
+        rc_release_loaded(dag, sTab, a, rootTable, rootPtr, dies, e, v, ListOut { out, outCount, cap }, cap,
+                          touchedList, ctr);
     }
 }
 
@@ -599,6 +639,8 @@ __global__ void __launch_bounds__(256) rc_release_batch(DagDev dag, GcTables a, 
                                                         GcCounters* ctr)
 {
     __shared__ uint32_t sCand[256];
+    __shared__ TableDev sTab[kGcMaxTables];
+    tables_stage(sTab, dag);
     const uint32_t t = threadIdx.x;
     const uint32_t stop = *poison;
     const uint32_t cur = *rootDev;
@@ -625,14 +667,14 @@ __global__ void __launch_bounds__(256) rc_release_batch(DagDev dag, GcTables a, 
         const uint32_t hs = leaf ? leaf_handle_size(dag, h) : node_handle_size(h);
         e = make_uint2(hs - 2u, leaf ? leaf_handle_ptr(dag, h) : node_handle_ptr(h));
     }
-    const uint32_t refs = in ? dag.tables[e.x].refs[e.y] : 1u;
-    const ReleaseItem v = rc_load(dag, in, e);
+    const uint32_t refs = in ? sTab[e.x].refs[e.y] : 1u;
+    const ReleaseItem v = rc_load(sTab, in, e);
     const bool dies = in && refs == 0u;
     const unsigned long long mk = __ballot(dies);
     if (mk != 0ull && __lane_id() == (uint32_t)__ffsll((long long)mk) - 1u)
         atomicAdd(&ctr->count[0], (uint32_t)__popcll(mk));
     const uint2 rs = root_slot(dag, cur);
-    rc_release_loaded(dag, a, rs.x, rs.y, dies, e, v, out, outCount, cap, touchedList, ctr);
+    rc_release_loaded(dag, sTab, a, rs.x, rs.y, dies, e, v, ListOut { out, outCount, cap }, cap, touchedList, ctr);
 }
 
 // A later round: frees the items of the input list.  Each thread reads its
@@ -646,6 +688,8 @@ __global__ void __launch_bounds__(256) rc_release(DagDev dag, GcTables a, uint32
                                                   uint2* out, uint32_t* outCount, uint32_t cap, uint2* touchedList,
                                                   GcCounters* ctr)
 {
+    __shared__ TableDev sTab[kGcMaxTables];
+    tables_stage(sTab, dag);
     const uint32_t first = blockIdx.x * blockDim.x;
     const uint32_t i0 = first + threadIdx.x;
     // Once a list overflowed or a count was found off, the marking
@@ -660,14 +704,72 @@ __global__ void __launch_bounds__(256) rc_release(DagDev dag, GcTables a, uint32
     }
     if (stop)
         return;
+    __syncthreads();
     const uint32_t n = min(cnt, cap);
     for (uint32_t base = first; base < n; base += gridDim.x * blockDim.x) {
         const uint32_t i = base + threadIdx.x;
         const bool have = i < n;
         const uint2 e = have ? (base == first ? spec : in[i]) : make_uint2(0u, 0u);
-        const ReleaseItem v = rc_load(dag, have, e);
-        rc_release_loaded(dag, a, rootTable, rootPtr, have, e, v, out, outCount, cap, touchedList, ctr);
+        const ReleaseItem v = rc_load(sTab, have, e);
+        rc_release_loaded(dag, sTab, a, rootTable, rootPtr, have, e, v, ListOut { out, outCount, cap }, cap,
+                          touchedList, ctr);
     }
+}
+
+// Rounds [1, end) in one block: the rounds below the roots hold a few items
+// each, and a launch for every one of them was its start, its chain of round
+// trips and the gap behind it.  Here a round is the item, its children's
+// counts and the decrements; its lists and their lengths are in LDS.  Round
+// 1's list is w1's, odd rounds read w1 past kSmallRelease entries, even ones
+// w0; the last output list is left in memory for the launches behind.
+// Before and after (a launch a round; 7 us of kernel and 2 of gap each):
+// two depth-10 edits with their collection 590 -> 540 us, 16 depth-15 edits
+// in one batch with one 1107 -> 1028, a 256^3 grid built and collected twice
+// 2.52 -> 2.31 ms, 16 batches of an edit stream 11.1 -> 10.5 ms.
+__global__ void __launch_bounds__(kSmallRelease) rc_release_small(DagDev dag, GcTables a, uint32_t rootTable,
+                                                                  uint32_t rootPtr, const uint32_t* rootDev, uint2* w0,
+                                                                  uint2* w1, uint32_t end, uint32_t cap,
+                                                                  uint2* touchedList, GcCounters* ctr)
+{
+    __shared__ TableDev sTab[kGcMaxTables];
+    __shared__ SmallRelease s;
+    tables_stage(sTab, dag);
+    if (rootDev) {
+        const uint2 rs = root_slot(dag, *rootDev);
+        rootTable = rs.x;
+        rootPtr = rs.y;
+    }
+    if (threadIdx.x < kSmallRelease && threadIdx.x < cap)
+        s.list[1][threadIdx.x] = w1[threadIdx.x];
+    if (threadIdx.x < kMaxLevels)
+        s.count[threadIdx.x] = threadIdx.x == 1u ? ctr->count[1] : 0u;
+    __syncthreads();
+    for (uint32_t r = 1; r < end; ++r) {
+        // As in rc_release: nothing more once a list overflowed or a count
+        // was off.
+        const uint32_t stop = __hip_atomic_load(&ctr->overflow, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const uint32_t n = min(s.count[r], cap);
+        const uint2* in = (r & 1u) ? w1 : w0;
+        const BlockOut out { s, r + 1u, (r & 1u) ? w0 : w1, cap };
+        uint2 e = s.list[r & 1u][threadIdx.x];
+        for (uint32_t base = 0; base < n; base += kSmallRelease) {
+            const bool have = base + threadIdx.x < n && !stop;
+            // A wave past the list's end has nothing to read or append.
+            if (__ballot(have) == 0ull)
+                break;
+            const ReleaseItem v = rc_load(sTab, have, e);
+            rc_release_loaded(dag, sTab, a, rootTable, rootPtr, have, e, v, out, cap, touchedList, ctr);
+            const uint32_t next = base + kSmallRelease + threadIdx.x;
+            if (next < n)
+                e = in[next];
+        }
+        __syncthreads();
+    }
+    const uint32_t left = min(min(s.count[end], cap), kSmallRelease);
+    if (threadIdx.x < left)
+        ((end & 1u) ? w1 : w0)[threadIdx.x] = s.list[end & 1u][threadIdx.x];
+    if (threadIdx.x > 1u && threadIdx.x <= end)
+        ctr->count[threadIdx.x] = s.count[threadIdx.x];
 }
 
 // The listed buckets of table blockIdx.y: unlink the overflow lines left
@@ -943,6 +1045,49 @@ int gc_stream_prepare(svdag_ctx* ctx)
     return gc_fronts(ctx, std::max<uint64_t>(ctx->gcCap, 1ull << 22));
 }
 
+// Items to expect in round r of a collection that releases `roots` roots:
+// recent collections' items per released root in that round, doubled;
+// negative where there is no history.
+static double release_expected(const svdag_ctx* ctx, uint32_t r, double roots)
+{
+    return r < ctx->gcPerRoot.size() && roots > 0.0 ? 2.0 * ctx->gcPerRoot[r] * roots : -1.0;
+}
+
+// Blocks of a round: the top rounds hold a few items per root, and a launch
+// of 256 blocks for them costs more than their work.  The grid-stride loop
+// covers any count, so the sizing only affects speed.
+static uint32_t release_grid(const svdag_ctx* ctx, uint32_t r, double roots)
+{
+    const double want = release_expected(ctx, r, roots);
+    return want < 0.0 ? 256u : (uint32_t)std::min(256.0, std::max(1.0, std::ceil(want / 256.0)));
+}
+
+// Rounds [1, rounds).  Those that are expected to fit one block's threads
+// run in one launch up to the first that is not; they had one or two blocks
+// of their own launches before, so a list that outgrows what was expected
+// finds as many threads as it did.
+static void release_rounds(svdag_ctx* ctx, const GcTables& a, uint32_t rootTable, uint32_t rootPtr,
+                           const uint32_t* rootDev, uint2* const w[2], uint32_t cap, uint32_t rounds, double roots,
+                           GcCounters* ctr, hipStream_t st)
+{
+    uint32_t r = 1;
+    while (r < rounds) {
+        const double want = release_expected(ctx, r, roots);
+        if (want < 0.0 || want > (double)kSmallRelease)
+            break;
+        ++r;
+    }
+    if (r > 2u)
+        rc_release_small<<<1, kSmallRelease, 0, st>>>(ctx->dag, a, rootTable, rootPtr, rootDev, w[0], w[1], r, cap,
+                                                      ctx->dGcTouchedList, ctr);
+    else
+        r = 1;
+    for (; r < rounds; ++r)
+        rc_release<<<release_grid(ctx, r, roots), 256, 0, st>>>(ctx->dag, a, rootTable, rootPtr, rootDev, w[r & 1],
+                                                                &ctr->count[r], w[(r + 1) & 1], &ctr->count[r + 1],
+                                                                cap, ctx->dGcTouchedList, ctr);
+}
+
 // Enqueues the counting collection behind edits [first, first + count) of
 // an edit stream (rc_release_batch): held are the roots the host held before
 // the stream, for its first collection (empty for later ones), and
@@ -964,17 +1109,9 @@ int gc_enqueue_stream(svdag_ctx* ctx, uint32_t first, uint32_t count, const std:
     uint2* w[2] = { reinterpret_cast<uint2*>(ctx->gcFront[0]), reinterpret_cast<uint2*>(ctx->gcFront[1]) };
     const uint32_t rounds = dag.leafLevel + 2u;
     const double roots = (double)(count + held.size());
-    auto grid = [&](uint32_t r) {
-        if (r >= ctx->gcPerRoot.size())
-            return 256u;
-        const double want = 2.0 * ctx->gcPerRoot[r] * roots;
-        return (uint32_t)std::min(256.0, std::max(1.0, std::ceil(want / 256.0)));
-    };
     rc_release_batch<<<1, 256, 0, st>>>(dag, a, ctx->dStatusArr, first, count, inl, (uint32_t)held.size(), ctx->dRoot,
                                         ctx->ws.poison, w[1], &ctr->count[1], cap2, ctx->dGcTouchedList, ctr);
-    for (uint32_t r = 1; r < rounds; ++r)
-        rc_release<<<grid(r), 256, 0, st>>>(dag, a, ~0u, ~0u, ctx->dRoot, w[r & 1], &ctr->count[r], w[(r + 1) & 1],
-                                             &ctr->count[r + 1], cap2, ctx->dGcTouchedList, ctr);
+    release_rounds(ctx, a, ~0u, ~0u, ctx->dRoot, w, cap2, rounds, roots, ctr, st);
     rc_chains<<<dim3(256, (uint32_t)nt), 256, 0, st>>>(dag, a, ctx->dGcTouchedList, cap2, rounds, ctr, next, fail);
     SVDAG_HIP(hipGetLastError());
     return SVDAG_OK;
@@ -1044,22 +1181,9 @@ static int gc_release(svdag_ctx* ctx, svdag_gc_stats* stats, bool& done, bool wa
         SVDAG_HIP(hipMemcpyAsync(ctx->dGcCand, cand.data(), cand.size() * 4, hipMemcpyHostToDevice, st));
         candDev = ctx->dGcCand;
     }
-    // Each round's grid from recent collections' items per released root in
-    // that round, times this collection's released roots, doubled: the
-    // top rounds hold a few items per root, and a launch of 256 blocks for
-    // them costs more than their work.  The grid-stride loop covers any
-    // count, so the sizing only affects speed.
-    auto grid = [&](uint32_t r) {
-        if (r >= ctx->gcPerRoot.size() || cand.empty())
-            return 256u;
-        const double want = 2.0 * ctx->gcPerRoot[r] * (double)cand.size();
-        return (uint32_t)std::min(256.0, std::max(1.0, std::ceil(want / 256.0)));
-    };
-    rc_release_roots<<<grid(0), 256, 0, st>>>(dag, a, rootTable, rootPtr, candDev, inl, (uint32_t)cand.size(), w[1],
+    rc_release_roots<<<release_grid(ctx, 0, (double)cand.size()), 256, 0, st>>>(dag, a, rootTable, rootPtr, candDev, inl, (uint32_t)cand.size(), w[1],
                                               &ctr->count[1], cap2, ctx->dGcTouchedList, ctr);
-    for (uint32_t r = 1; r < rounds; ++r)
-        rc_release<<<grid(r), 256, 0, st>>>(dag, a, rootTable, rootPtr, nullptr, w[r & 1], &ctr->count[r],
-                                             w[(r + 1) & 1], &ctr->count[r + 1], cap2, ctx->dGcTouchedList, ctr);
+    release_rounds(ctx, a, rootTable, rootPtr, nullptr, w, cap2, rounds, (double)cand.size(), ctr, st);
     rc_chains<<<dim3(256, (uint32_t)nt), 256, 0, st>>>(dag, a, ctx->dGcTouchedList, cap2, rounds, ctr, next, nullptr);
     SVDAG_HIP(hipEventRecord(ctx->ev1, st));
     if (!wait) {

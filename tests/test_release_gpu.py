@@ -1,0 +1,45 @@
+"""The rounds of a counting collection that stay in one block: lists that fit
+its LDS, lists that outgrow what the collections before let expect (512
+entries and more), the shallowest trees.  A marking collection behind it finds
+nothing left, and the scene reads as the oracle's."""
+import numpy as np
+import pytest
+
+import oracle_py
+import svdag_py
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("levels,bits,small,large", [
+    (4, 4, 2.0, 6.0), (5, 0, 2.0, 12.0), (9, 8, 1.5, 60.0), (11, 4, 3.0, 200.0), (14, 8, 0.6, 60.0)])
+def test_rounds_in_one_block(levels, bits, small, large):
+    g = svdag_py.MyGPUHashDAG(levels, bits)
+    o = oracle_py.OracleDag(levels, bits)
+    s = float(1 << levels)
+    rng = np.random.default_rng(levels)
+    mats = 3 if bits else 1
+
+    def edit(kind, c, r):
+        m = int(rng.integers(0, mats)) if kind in (svdag_py.SPHERE_ADD, svdag_py.BOX_ADD) else 0
+        g.edit(kind, m, tuple(c), r)
+        o.edit(kind, m, tuple(c), r)
+
+    c = np.array([s / 2, s / 2, s / 2])
+    edit(svdag_py.SPHERE_ADD, c, large)
+    freed = []
+    # small edits first, so that little is expected of the large one's rounds
+    for k, r in enumerate([small, small, small * 1.3, large, small, large * 0.9]):
+        print(f"[case] release levels={levels} bits={bits} r={r}", flush=True)
+        kind = svdag_py.SPHERE_REMOVE if k % 2 else svdag_py.BOX_ADD
+        edit(kind, c + rng.uniform(-1, 1, 3) * large / 3, r)
+        st = g.garbage_collect()
+        freed.append(int(st.items_freed))
+        assert st.marked == 0
+        check = g.garbage_collect(mark=True)
+        assert check.items_freed == 0 and check.items_live == st.items_live
+    assert max(freed) > 0
+    if levels >= 9:  # more than two of the block's lists
+        assert max(freed) > 2 * 512
+    pts = rng.integers(0, 1 << levels, (4000, 3)).astype(np.uint32)
+    assert np.array_equal(g.query(pts), o.query(pts))
+    g.close()
