@@ -13,7 +13,7 @@
 //   paint   my_gpu_dag_editors.h:498-536   (Fill only over flagged full nodes)
 //   copy    my_gpu_dag_editors.h:127-253   (translation; up to 8 source parents;
 //           quarter turns about +Y have no reference counterpart; done in
-//           integer voxel arithmetic: decide_copy_rot / rot_source)
+//           integer voxel arithmetic: decide_copy / rot_source)
 // The terrain tool (kind 6) has no reference counterpart: it classifies nodes
 // against a min/max height pyramid so that a heightfield builds through the
 // same pipeline as an edit.

