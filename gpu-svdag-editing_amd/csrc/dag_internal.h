@@ -140,16 +140,6 @@ __device__ inline void child_ref_add(const DagDev& dag, uint32_t h, uint8_t role
     if (ld_filter(c) < kStickyRefs)
         atomicAdd(c, 1u);
 }
-// node handle h may be used where its children decode under `role`.
-__device__ inline bool node_has_role(const DagDev& dag, uint32_t h, uint8_t role)
-{
-    return (dag.tables[node_handle_size(h) - 2].roles[node_handle_ptr(h)] & role) != 0;
-}
-// leaf handle h names an item stored as a leaf (no roles).
-__device__ inline bool leaf_is_plain(const DagDev& dag, uint32_t h)
-{
-    return dag.tables[leaf_handle_size(dag, h) - 2].roles[leaf_handle_ptr(dag, h)] == 0;
-}
 // After a group inserted the item held in n (s words) at pointer res of
 // table s - 2: record its role (0 for a leaf) and count its children.
 template <int G, int MW>

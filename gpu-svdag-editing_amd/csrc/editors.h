@@ -258,24 +258,6 @@ __device__ inline Op decide(const EditorDev& e, uint32_t x, uint32_t y, uint32_t
     }
 }
 
-// get_new_value for the stateless tools: true and a material when the voxel
-// ends up set.
-__device__ inline bool new_value(const EditorDev& e, bool hasOld, uint32_t oldMat, uint32_t& mat)
-{
-    switch (e.kind) {
-    case EK_SPHERE_ADD:
-    case EK_BOX_ADD:
-    case EK_PAINT:
-    case EK_TERRAIN:
-        mat = e.material;
-        return true;
-    default:
-        (void)hasOld;
-        (void)oldMat;
-        return false;
-    }
-}
-
 __host__ __device__ inline bool aabb_overlap(const float lmn[3], const float lmx[3], const float rmn[3], const float rmx[3])
 {
     return !(lmn[0] >= rmx[0] || lmn[1] >= rmx[1] || lmn[2] >= rmx[2] || lmx[0] <= rmn[0] || lmx[1] <= rmn[1]

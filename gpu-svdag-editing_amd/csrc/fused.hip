@@ -142,17 +142,6 @@ size_t spine_scratch_bytes()
     return sizeof(SpineScratch);
 }
 
-__device__ inline uint32_t joint_handle(const WsDev& ws, uint32_t w, uint32_t& created)
-{
-    const uint32_t r = ws.rep[w];
-    if (r == kSentinel) {
-        created = 0u;
-        return kSentinel;
-    }
-    created = ws.created[r] & 1u;
-    return ws.handle[r];
-}
-
 __global__ void __launch_bounds__(kParThreads) fused_spine_par(WsDev ws, DagDev dag, const EditorDev* eds, FusedDev f,
                                                                uint32_t* rootPtr, EditStatus* status,
                                                                LevelDesc* levels)

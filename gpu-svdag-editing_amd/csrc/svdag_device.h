@@ -421,8 +421,8 @@ __device__ inline uint32_t table_find_group(const TableDev& t, const Needle<G, M
 // lines leave a chain only in a collection), so an insert that starts there
 // and walks on finds every free slot it would have found from the head
 // after that line -- it only skips lines the find saw full.
-// role != 0: a filter on the item's role byte (DAG tables, see
-// node_has_role): kRoleLeafUse matches items without roles, any other value
+// role != 0: a filter on the item's role byte (DAG tables):
+// kRoleLeafUse matches items without roles, any other value
 // items with one of its bits.
 template <int G, int MW>
 __device__ inline uint32_t table_find_group_hint(const TableDev& t, const Needle<G, MW>& n, uint32_t s, uint32_t h,
