@@ -1087,6 +1087,7 @@ __global__ void __launch_bounds__(kSmallBlock) merge_small(WsDev ws, DagDev dag,
         const uint32_t parity = (uint32_t)L & 1u;
         const bool more = L > (int)last;
         if (me.count > kSmallBlock) {
+            __syncthreads(); // the level below left other threads' results in the workspace
             const bool gate = kMulti || ws.lvl[L + 1].fullCount != 0;
             for (uint32_t i = threadIdx.x; i < me.count; i += kSmallBlock)
                 prepare_item<kMulti>(ws, dag, (uint32_t)L, me.start + i, gate, below);

@@ -90,3 +90,47 @@ def test_levels_around_the_one_block_limit_match_oracle():
     st = g.garbage_collect()
     assert st.marked == 0 and g.garbage_collect(mark=True).items_freed == 0
     g.close()
+
+
+def _corner_scene(levels):
+    """Voxels around the lattice corners that are odd multiples of 16: below
+    each corner up to its sides, above it only from 10 voxels on.  All eight
+    16-voxel cells around a corner hold voxels, but only the lower four of the
+    8-voxel cells do."""
+    side = 1 << levels
+    rng = np.random.default_rng(5)
+    vox = _noise(side, rng, 0.6, [1, 2, 3, 4])
+    y = np.arange(side) % 32  # the corner is at 16
+    vox[:, ~(((y >= 11) & (y < 16)) | ((y >= 26) & (y < 30))), :] = 0xFF
+    return vox
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bits,lanes", [(4, 0), (8, 4)])
+def test_a_large_level_above_a_small_one_matches_oracle(bits, lanes):
+    # 200 small paints (the tool that leaves empty children alone), each with
+    # 8 items on level 4 and 4 on level 5, in one wave split at level 4: one
+    # block takes both levels, the lower one with an item per thread and the
+    # upper one through the workspace, where it reads what the lower one left.
+    levels, edits = 8, 200
+    vox = _corner_scene(levels)
+    g = svdag_py.MyGPUHashDAG(levels, bits, group_size=lanes)
+    o = oracle_py.OracleDag(levels, bits)
+    g.build_voxels(vox)
+    oracle_py.build_dense(o, vox)
+    rng = np.random.default_rng(9)
+    corners = np.stack(np.meshgrid(*[np.arange(16, 1 << levels, 32)] * 3, indexing="ij"), -1).reshape(-1, 3)
+    print(f"[case] large above small bits={bits} lanes={lanes}", flush=True)
+    for rep in range(3):  # results left by one batch would show in the next
+        at = corners[rng.permutation(len(corners))[:edits]]
+        batch = [(svdag_py.PAINT, 5 + rep, tuple(map(float, c)), 1.6 + 0.4 * rep) for c in at]
+        stats, _ = g.edit_batch(batch)
+        items = np.sum([list(s.svo_items) for s in stats], axis=0)
+        # The host's bound of both levels is 8 items an edit (at most 2048).
+        assert items[4] > 1024 and 0 < items[5] <= 1024 and 8 * edits <= 2048
+        for e in batch:
+            o.edit(*e)
+        assert g.canonical() == o.canonical()
+    st = g.garbage_collect()
+    assert st.marked == 0 and g.garbage_collect(mark=True).items_freed == 0
+    g.close()
