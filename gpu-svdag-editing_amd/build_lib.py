@@ -48,6 +48,15 @@ def _compile(src):
     return obj
 
 
+def build_program(src, out):
+    """A HIP program on the library's device headers, with its flags."""
+    cmd = [_hipcc(), *HIP_FLAGS, src, "-o", out + ".tmp"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"compile failed: {' '.join(cmd)}\n{r.stdout}\n{r.stderr}")
+    os.replace(out + ".tmp", out)
+
+
 def build(verbose=False):
     os.makedirs(OBJ, exist_ok=True)
     os.makedirs(LIBDIR, exist_ok=True)

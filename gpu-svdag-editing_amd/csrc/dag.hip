@@ -962,27 +962,8 @@ __device__ inline void insert_block(const WsDev& ws, const DagDev& dag, const Ta
         if (b != 0ull && (threadIdx.x & 63u) == 0u)
             atomicAdd(&sInserted, (uint32_t)__popcll(b));
         __syncthreads();
-        if constexpr (!kLeaf) {
-            // Every count the thread updates is loaded before the first update.
-            constexpr uint32_t kPer = kSlots / kBlock;
-            uint32_t* cnt[kPer];
-            uint32_t seen[kPer], add[kPer];
-#pragma unroll
-            for (uint32_t k = 0; k < kPer; ++k) {
-                const uint32_t q = k * kBlock + threadIdx.x;
-                const uint32_t c = q <= slotMask ? sRefs.child[q] : kSentinel;
-                seen[k] = kStickyRefs;
-                if (c != kSentinel) {
-                    cnt[k] = child_count(dag, sTab, c, role);
-                    add[k] = sRefs.add[q];
-                    seen[k] = ld_filter(cnt[k]);
-                }
-            }
-#pragma unroll
-            for (uint32_t k = 0; k < kPer; ++k)
-                if (seen[k] < kStickyRefs)
-                    atomicAdd(cnt[k], add[k]);
-        }
+        if constexpr (!kLeaf)
+            block_refs_flush<kBlock>(sRefs, slotMask, dag, sTab, role);
     }
 }
 

@@ -60,6 +60,34 @@ __device__ inline void block_ref_add(BlockRefs<kSlots>& refs, uint32_t slotMask,
         atomicAdd(cnt, 1u);
 }
 
+// The block's sums (after a barrier) to the tables: one update per child, none
+// for a count at its ceiling -- it is never taken back, so it would grow with
+// every item that shares the child until it wrapped.  Every count the thread
+// updates is loaded before the first update.
+template <uint32_t kBlock, uint32_t kSlots>
+__device__ inline void block_refs_flush(const BlockRefs<kSlots>& refs, uint32_t slotMask, const DagDev& dag,
+                                        const TableDev* sTab, uint8_t role)
+{
+    constexpr uint32_t kPer = kSlots / kBlock;
+    uint32_t* cnt[kPer];
+    uint32_t seen[kPer], add[kPer];
+#pragma unroll
+    for (uint32_t k = 0; k < kPer; ++k) {
+        const uint32_t q = k * kBlock + threadIdx.x;
+        const uint32_t c = q <= slotMask ? refs.child[q] : kSentinel;
+        seen[k] = kStickyRefs;
+        if (c != kSentinel) {
+            cnt[k] = child_count(dag, sTab, c, role);
+            add[k] = refs.add[q];
+            seen[k] = ld_filter(cnt[k]);
+        }
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < kPer; ++k)
+        if (seen[k] < kStickyRefs)
+            atomicAdd(cnt[k], add[k]);
+}
+
 // ---------------------------------------------------------------- small levels
 // Levels of at most kSmallBlock items run in one block, one thread per item,
 // the item's words in registers from its record to its insert: what the
@@ -170,11 +198,7 @@ __device__ inline void small_find_insert(const DagDev& dag, const TableDev* sTab
         sh.created[parity][slot] = inserts ? 1u : 0u;
     }
     __syncthreads();
-    // One update per child, not waited for.  A count past its ceiling only
-    // grows, which leaves it past its ceiling.
-    for (uint32_t q = threadIdx.x; q < kRefSlots; q += kSmallBlock)
-        if (refs.child[q] != kSentinel)
-            atomicAdd(child_count(dag, sTab, refs.child[q], role), refs.add[q]);
+    block_refs_flush<kSmallBlock>(refs, kRefSlots - 1u, dag, sTab, role);
 }
 
 } // namespace svdag
