@@ -689,12 +689,15 @@ __global__ void __launch_bounds__(256) rc_release(DagDev dag, GcTables a, uint32
                                                   GcCounters* ctr)
 {
     __shared__ TableDev sTab[kGcMaxTables];
+    __shared__ uint32_t sStop;
     tables_stage(sTab, dag);
     const uint32_t first = blockIdx.x * blockDim.x;
     const uint32_t i0 = first + threadIdx.x;
     // Once a list overflowed or a count was found off, the marking
-    // collection takes over: release nothing more.
-    const uint32_t stop = ctr->overflow;
+    // collection takes over: release nothing more.  One read per block:
+    // other blocks of this round may set the flag meanwhile.
+    if (threadIdx.x == 0)
+        sStop = ctr->overflow;
     const uint32_t cnt = *inCount;
     const uint2 spec = i0 < cap ? in[i0] : make_uint2(0u, 0u);
     if (rootDev) {
@@ -702,9 +705,9 @@ __global__ void __launch_bounds__(256) rc_release(DagDev dag, GcTables a, uint32
         rootTable = rs.x;
         rootPtr = rs.y;
     }
-    if (stop)
-        return;
     __syncthreads();
+    if (sStop)
+        return;
     const uint32_t n = min(cnt, cap);
     for (uint32_t base = first; base < n; base += gridDim.x * blockDim.x) {
         const uint32_t i = base + threadIdx.x;

@@ -43,3 +43,26 @@ def test_rounds_in_one_block(levels, bits, small, large):
     pts = rng.integers(0, 1 << levels, (4000, 3)).astype(np.uint32)
     assert np.array_equal(g.query(pts), o.query(pts))
     g.close()
+
+
+@pytest.mark.gpu
+def test_a_round_past_the_list_leaves_the_rest_to_marking():
+    # More than 2^21 leaves (the least a round's list holds) die at once: the
+    # blocks of the round that overflows the list stop, and the collection
+    # marks instead.
+    levels = 10
+    rng = np.random.default_rng(3)
+    noise = np.where(rng.random((512,) * 3, np.float32) < 0.5, np.uint8(0), np.uint8(0xFF))
+    g = svdag_py.MyGPUHashDAG(levels, 0, expected_items=1 << 22)
+    print("[case] release of more leaves than the list holds", flush=True)
+    g.build_voxels(noise)
+    g.edit(svdag_py.COPY, 0, (760.0, 760.0, 760.0), 60.0, (301.0, 303.0, 202.0), (760.0, 760.0, 760.0))
+    g.build_voxels(noise[:64, :64, :64])
+    st = g.garbage_collect()
+    assert st.marked == 1 and st.items_freed > 1 << 21
+    assert g.garbage_collect(mark=True).items_freed == 0
+    want = svdag_py.MyGPUHashDAG(levels, 0)
+    want.build_voxels(noise[:64, :64, :64])
+    assert g.canonical() == want.canonical()
+    want.close()
+    g.close()
