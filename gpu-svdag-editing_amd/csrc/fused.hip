@@ -154,6 +154,7 @@ __global__ void __launch_bounds__(kParThreads) fused_spine_par(WsDev ws, DagDev 
     __shared__ unsigned long long sPosEdits[kParItems];
     __shared__ uint32_t sFullCnt[2][kParEdits], sDropped[kParEdits]; // full items by level parity
     __shared__ uint32_t sOk, sBad;
+    __shared__ uint32_t sStop[2]; // top-down, by level parity: a level sets its flag while waves still read the last one's
     __shared__ TableDev sTab[kRefTables];
     __shared__ SmallShared<kParItems> sh;
     const uint32_t t = threadIdx.x;
@@ -165,7 +166,7 @@ __global__ void __launch_bounds__(kParThreads) fused_spine_par(WsDev ws, DagDev 
     const EditStatus joint = *ws.status;
     if (t == 0) {
         sOk = K >= 1 && K <= kParEdits && S >= 1 && S <= leafLevel && !joint.overflow && !joint.oom;
-        sBad = 0u;
+        sBad = sStop[0] = sStop[1] = 0u;
         sh.oom = 0u;
         sh.inserted = 0u;
     }
@@ -228,7 +229,7 @@ __global__ void __launch_bounds__(kParThreads) fused_spine_par(WsDev ws, DagDev 
                                           (item.z << 1) | (c & 1u), dag.levels - (l + 1), st, fm);
                 sub = op == OP_SUBDIVIDE;
                 if (!(sub || op == OP_KEEP || (paint && op == OP_EMPTY && st == NS_EMPTY)))
-                    atomicOr(&sBad, 1u); // a fill above S: the sequential spine takes the wave
+                    atomicOr(&sStop[par], 1u); // a fill above S: the sequential spine takes the wave
                 dep = paint && op != OP_KEEP;
             }
             const uint32_t subm = group_ballot<8>(sub, t & 56u), depm = group_ballot<8>(dep, t & 56u);
@@ -271,7 +272,7 @@ __global__ void __launch_bounds__(kParThreads) fused_spine_par(WsDev ws, DagDev 
                     const bool inRange = dx < sd.n[0] && dy < sd.n[1] && dz < sd.n[2];
                     ref = inRange ? f.seedWork[(wv.x + pk) * 8 + ((dx << 2) | (dy << 1) | dz)] : kSentinel;
                     if (ref == kSentinel)
-                        atomicOr(&sBad, 1u);
+                        atomicOr(&sStop[par], 1u);
                 }
                 sc.item[pk][l][pi].ref[c] = ref;
             }
@@ -279,11 +280,11 @@ __global__ void __launch_bounds__(kParThreads) fused_spine_par(WsDev ws, DagDev 
                 sCnt[par ^ 1u][pk] = total < kSpineItems ? total : kSpineItems;
                 sc.cnt[pk][l + 1] = total < kSpineItems ? total : kSpineItems;
                 if (total > kSpineItems)
-                    atomicOr(&sBad, 1u);
+                    atomicOr(&sStop[par], 1u);
             }
         }
         __syncthreads();
-        if (sBad)
+        if (sStop[par])
             return; // nothing written outside the scratch: the sequential spine takes the wave
     }
     const uint32_t k = t >> 3, i = t & 7u; // one (edit, item) pair per thread from here on
