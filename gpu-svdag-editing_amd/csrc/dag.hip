@@ -1931,6 +1931,7 @@ int svdag_create(const svdag_config* cfgIn, svdag_ctx** out)
     SVDAG_TRY(ctx_refresh_tables(ctx));
     SVDAG_HIP(hipMalloc(&ctx->dFullyFilled, (size_t)d.levels * d.numMaterials * 4));
     d.fullyFilled = ctx->dFullyFilled;
+    d.solidFlag = kFullFlag;
     SVDAG_HIP(hipMalloc(&ctx->dStored, sizeof(unsigned long long)));
     SVDAG_HIP(hipMemsetAsync(ctx->dStored, 0, sizeof(unsigned long long), ctx->stream));
     d.stored = ctx->dStored;

@@ -446,6 +446,7 @@ int import_dump(svdag_ctx* ctx, const uint32_t* d, size_t len)
     size_t p = 0;
     auto need = [&](size_t k) { return p + k <= len; };
     std::vector<uint32_t> below; // handles of the level below, by canonical id
+    std::vector<uint8_t> solidBelow, solid; // which items have only set voxels
     for (int L = (int)dag.leafLevel; L >= 0; --L) {
         if (!need(2) || d[p] != (uint32_t)L) {
             set_error("import: level " + std::to_string(L) + " missing or out of order");
@@ -456,6 +457,8 @@ int import_dump(svdag_ctx* ctx, const uint32_t* d, size_t len)
         const bool leaf = (uint32_t)L == dag.leafLevel;
         std::vector<std::vector<uint32_t>> items;
         items.reserve(count);
+        solid.clear();
+        bool flagsHold = true;
         for (uint32_t i = 0; i < count; ++i) {
             if (!need(1)) {
                 set_error("import: truncated");
@@ -473,24 +476,35 @@ int import_dump(svdag_ctx* ctx, const uint32_t* d, size_t len)
                     set_error("import: leaf size does not match its mask");
                     return SVDAG_E_INVALID;
                 }
+                solid.push_back(w[0] == 0xFFFFFFFFu && w[1] == 0xFFFFFFFFu);
             } else {
                 if ((w[0] & 0xFFu) == 0 || sz != node_size_from_header(w[0]) || header_payload(w[0], dag.M) != 0) {
                     set_error("import: node header does not match its size");
                     return SVDAG_E_INVALID;
                 }
+                bool filled = (w[0] & 0xFFu) == 0xFFu;
                 for (uint32_t j = 1; j < sz; ++j) {
                     if (w[j] >= below.size()) {
                         set_error("import: child id out of range");
                         return SVDAG_E_INVALID;
                     }
+                    filled = filled && solidBelow[w[j]];
                     w[j] = below[w[j]];
                 }
+                solid.push_back(filled);
+                flagsHold = flagsHold && (filled || !(w[0] & kFullFlag));
             }
             items.push_back(std::move(w));
+        }
+        if (!flagsHold) {
+            // Frames traced beside this call read the descriptor.
+            FrameQuiesce q(ctx);
+            ctx->dag.solidFlag = 0u;
         }
         std::vector<uint32_t> handles;
         SVDAG_TRY(insert_level(ctx, items, leaf, handles));
         below.swap(handles);
+        solidBelow.swap(solid);
     }
     if (!need(1)) {
         set_error("import: root id missing");

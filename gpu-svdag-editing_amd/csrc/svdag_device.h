@@ -757,7 +757,12 @@ struct DagDev {
     uint32_t leafSizeBits;    // bit_width(maxLeaf - minLeaf)
     uint32_t numTables;
     unsigned long long* stored; // items stored in the tables (inserts minus frees)
+    // The header's full flag (kFullFlag) while every stored node that carries
+    // it has only set voxels below, as a merge makes them; 0 once an import
+    // brought one that has not.  What a kernel may end an occlusion ray on.
+    uint32_t solidFlag;
 };
+constexpr uint32_t kFullFlag = 0x100u;
 
 constexpr uint32_t kNodeSizeBits = 3; // bit_width(9 - 2)
 

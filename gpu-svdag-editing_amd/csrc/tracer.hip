@@ -246,7 +246,7 @@ __device__ inline bool walk(const DagDev& dag, const TraceShared& sh, uint32_t r
             } else {
                 node = item;
                 child = w0 & 0xFFu;
-                if (kAny && (w0 & 0x100u))
+                if (kAny && (w0 & dag.solidFlag))
                     return true;
             }
         } else {

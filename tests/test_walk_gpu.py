@@ -53,3 +53,40 @@ def test_walk_matches_oracle(levels, bits, w, h, view):
         osun, oao = o.shade(*args, bias=0.25, ao_samples=2, ao_length=length, seed=5)
         assert np.array_equal(sun, osun) and np.array_equal(ao, oao)
     g.close()
+
+
+@pytest.mark.gpu
+def test_imported_full_flags_do_not_end_occlusion_rays():
+    # An imported node may carry the full flag over children that are not all
+    # filled; rays pass through its empty parts all the same.
+    levels, bits, w, h = 8, 4, 96, 64
+    g, _, s, r = _scene(levels, bits)
+    _, _, dump = g.canonical(dump=True)
+    forged, p, changed = dump.copy(), 0, 0
+    for level in range(levels - 2, -1, -1):
+        count, p = int(dump[p + 1]), p + 2
+        for _ in range(count):
+            if level < levels - 2 and dump[p + 1] & 0xFF != 0xFF:
+                forged[p + 1] |= 0x100
+                changed += 1
+            p += 1 + int(dump[p])
+    assert changed > 100
+    f = svdag_py.MyGPUHashDAG(levels, bits)
+    f.import_canonical(forged)
+    c = np.array([s / 2, s / 2, s / 2])
+    pos = c + r * np.array([2.5, 2.1, 1.7])
+    args = (tuple(pos), svdag_py.look_at(pos, c), 50.0, (0.0,) * 3, (s,) * 3, w, h)
+    palette = np.linspace(0.1, 0.9, 3 * 16).reshape(16, 3)
+    out = []
+    for d in (g, f):
+        hits, _ = d.trace(*args)
+        sun, _ = d.trace_shadows(0.25)
+        ao, _ = d.trace_ambient_occlusion(4, 0.25, 30.0, 5)
+        d.trace_colors(palette)
+        path, _, _ = d.trace_path_tracing(palette, samples=2, depth=3)
+        out.append((hits.view(np.uint32), sun, ao, path))
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+    assert (out[0][1] > 0).any() and ((out[0][2] > 0) & (out[0][2] < 1)).any()
+    g.close()
+    f.close()
