@@ -56,11 +56,16 @@ def test_a_round_past_the_list_leaves_the_rest_to_marking():
     g = svdag_py.MyGPUHashDAG(levels, 0, expected_items=1 << 22)
     print("[case] release of more leaves than the list holds", flush=True)
     g.build_voxels(noise)
-    g.edit(svdag_py.COPY, 0, (760.0, 760.0, 760.0), 60.0, (301.0, 303.0, 202.0), (760.0, 760.0, 760.0))
-    g.build_voxels(noise[:64, :64, :64])
-    st = g.garbage_collect()
-    assert st.marked == 1 and st.items_freed > 1 << 21
-    assert g.garbage_collect(mark=True).items_freed == 0
+    for copy in (False, True):  # 2^21 leaves fit, the copy's are too many
+        if copy:
+            g.build_voxels(noise)
+            src = (301.0, 303.0, 202.0)
+            assert g.edit(svdag_py.COPY, 0, src, 60.0, src, (760.0, 760.0, 760.0)).applied
+        g.garbage_collect(mark=True)  # counts that hold, whatever grew during the build
+        g.build_voxels(noise[:64, :64, :64])
+        st = g.garbage_collect()
+        assert st.marked == copy and st.items_freed > 1 << 21
+        assert g.garbage_collect(mark=True).items_freed == 0
     want = svdag_py.MyGPUHashDAG(levels, 0)
     want.build_voxels(noise[:64, :64, :64])
     assert g.canonical() == want.canonical()
