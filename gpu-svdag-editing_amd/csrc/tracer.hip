@@ -106,15 +106,18 @@ __device__ inline uint32_t intersection_mask(uint32_t shift, uint32_t px, uint32
 
 // ------------------------------------------------------------------ the walk
 // Bound: each step's chain (stack or child handle, then the child's header)
-// at the waves that LDS leaves room for, and about 130 VALU operations.
+// at the waves in flight, and about 130 VALU operations.  Waves per CU at
+// depth 15: 21 in trace_kernel and shadow_kernel, where LDS is the limit, 20
+// in ao_kernel (83 registers) and 16 in path_kernel (108).
 //   - One wave per block over an 8x8 tile: a wave's rays stay together, and
 //     a block ends with its own longest ray.
 //   - The stack holds one 8-byte entry per level above the last (node
-//     address, child mask, children left), sized by the DAG's depth: 22 waves
-//     per CU at depth 15.  A bit per level says where children are left, so
-//     going up reads one entry, not one per level.
+//     address, child mask, children left), sized by the DAG's depth.  A bit
+//     per level says where children are left, so going up reads one entry,
+//     not one per level.
 //   - An item's address takes one LDS read after its handle, and lanes at
-//     nodes and lanes at leaves load theirs together.
+//     nodes and lanes at leaves load its first word together (the compiler
+//     leaves the second, which only a leaf has a use for, to the leaf lanes).
 // Measured against the walk with 16x16 tiles and a 20-level stack per block
 // of 256: primary 1920x1080 at depth 15 1.354 -> 0.617 ms; at depth 13 and
 // 1280x720 shadows 0.616 -> 0.284, occlusion at 3 samples 0.548 -> 0.236 ms;
@@ -138,7 +141,7 @@ __device__ inline void trace_stage(TraceShared& sh, const DagDev& dag)
 }
 // How a handle's bits split: size = minWords + (h >> 1 >> sizeShift), the
 // index below.  Nodes and leaves differ only in these numbers, so lanes that
-// reach nodes and lanes that reach leaves decode and load together.
+// reach nodes and lanes that reach leaves decode together.
 struct HandleBits {
     uint32_t sizeShift, indexMask, minWords;
 };
