@@ -1926,7 +1926,7 @@ int svdag_create(const svdag_config* cfgIn, svdag_ctx** out)
         const uint32_t buckets = (uint32_t)std::min<uint64_t>(want, ctx->slabLimit[i] / 2);
         uint64_t cap = buckets + (cfg.arena_slabs ? cfg.arena_slabs : buckets / 2 + 4096);
         cap = std::min<uint64_t>(cap, ctx->slabLimit[i]);
-        SVDAG_TRY(table_alloc(ctx->ts.tables[i], 2 + i, buckets, (uint32_t)cap, ctx->stream, true));
+        SVDAG_TRY(table_alloc(ctx->ts.tables[i], 2 + i, buckets, (uint32_t)cap, ctx->stream));
     }
     SVDAG_TRY(ctx_refresh_tables(ctx));
     SVDAG_HIP(hipMalloc(&ctx->dFullyFilled, (size_t)d.levels * d.numMaterials * 4));
@@ -2688,7 +2688,7 @@ static int set_load_factor(svdag_ctx* ctx, uint32_t loadFactor)
         const uint32_t buckets = (uint32_t)std::min<uint64_t>(want, ctx->slabLimit[i] / 2);
         const uint64_t cap = std::min<uint64_t>((uint64_t)buckets + (per[i] + slots - 1) / slots + buckets / 2 + 4096,
                                                 ctx->slabLimit[i]);
-        const int rc = table_alloc(other[i], 2 + i, buckets, (uint32_t)cap, ctx->stream, true);
+        const int rc = table_alloc(other[i], 2 + i, buckets, (uint32_t)cap, ctx->stream);
         if (rc != SVDAG_OK) {
             freeOther();
             return rc;

@@ -42,8 +42,7 @@ __global__ void tables_init_lines(const TableDev* tables)
     }
 }
 
-int table_alloc(HostTable& t, uint32_t itemWords, uint32_t numBuckets, uint32_t slabCap, hipStream_t stream,
-                bool withRefs)
+int table_alloc(HostTable& t, uint32_t itemWords, uint32_t numBuckets, uint32_t slabCap, hipStream_t stream)
 {
     if (itemWords == 0 || itemWords > kMaxItemWords || numBuckets == 0 || slabCap < numBuckets) {
         set_error("table_alloc: bad size");
@@ -65,12 +64,10 @@ int table_alloc(HostTable& t, uint32_t itemWords, uint32_t numBuckets, uint32_t 
     SVDAG_HIP(hipMalloc(d.lines.slot(), (size_t)slabCap * kLineWords * 4));
     SVDAG_HIP(hipMalloc(d.freeList.slot(), (size_t)slabCap * 4));
     SVDAG_HIP(hipMalloc(d.alloc.slot(), sizeof(AllocState)));
-    if (withRefs) {
-        SVDAG_HIP(hipMalloc(d.refs.slot(), (size_t)slabCap * kMaxSlots * 4));
-        SVDAG_HIP(hipMalloc(d.roles.slot(), (size_t)slabCap * kMaxSlots));
-        SVDAG_HIP(hipMemsetAsync(d.refs, 0, (size_t)slabCap * kMaxSlots * 4, stream));
-        SVDAG_HIP(hipMemsetAsync(d.roles, 0, (size_t)slabCap * kMaxSlots, stream));
-    }
+    SVDAG_HIP(hipMalloc(d.refs.slot(), (size_t)slabCap * kMaxSlots * 4));
+    SVDAG_HIP(hipMalloc(d.roles.slot(), (size_t)slabCap * kMaxSlots));
+    SVDAG_HIP(hipMemsetAsync(d.refs, 0, (size_t)slabCap * kMaxSlots * 4, stream));
+    SVDAG_HIP(hipMemsetAsync(d.roles, 0, (size_t)slabCap * kMaxSlots, stream));
     AllocState a { numBuckets, 0, 0u, 0u };
     SVDAG_HIP(hipMemcpyAsync(d.alloc, &a, sizeof(a), hipMemcpyHostToDevice, stream));
     table_init_lines<<<grid_for((uint64_t)slabCap * kLineWords, 256, 8192), 256, 0, stream>>>(d, 0u, slabCap);
@@ -108,25 +105,21 @@ int table_grow(HostTable& t, uint32_t newCap, hipStream_t stream)
     SVDAG_HIP(hipMalloc(&freeList, (size_t)newCap * 4));
     SVDAG_HIP(hipMemcpyAsync(lines, d.lines, (size_t)old * kLineWords * 4, hipMemcpyDeviceToDevice, stream));
     SVDAG_HIP(hipMemcpyAsync(freeList, d.freeList, (size_t)old * 4, hipMemcpyDeviceToDevice, stream));
-    if (d.refs) {
-        SVDAG_HIP(hipMalloc(&refs, (size_t)newCap * kMaxSlots * 4));
-        SVDAG_HIP(hipMalloc(&roles, (size_t)newCap * kMaxSlots));
-        SVDAG_HIP(hipMemcpyAsync(refs, d.refs, (size_t)old * kMaxSlots * 4, hipMemcpyDeviceToDevice, stream));
-        SVDAG_HIP(hipMemcpyAsync(roles, d.roles, (size_t)old * kMaxSlots, hipMemcpyDeviceToDevice, stream));
-        SVDAG_HIP(hipMemsetAsync(refs + (size_t)old * kMaxSlots, 0, (size_t)(newCap - old) * kMaxSlots * 4, stream));
-        SVDAG_HIP(hipMemsetAsync(roles + (size_t)old * kMaxSlots, 0, (size_t)(newCap - old) * kMaxSlots, stream));
-    }
+    SVDAG_HIP(hipMalloc(&refs, (size_t)newCap * kMaxSlots * 4));
+    SVDAG_HIP(hipMalloc(&roles, (size_t)newCap * kMaxSlots));
+    SVDAG_HIP(hipMemcpyAsync(refs, d.refs, (size_t)old * kMaxSlots * 4, hipMemcpyDeviceToDevice, stream));
+    SVDAG_HIP(hipMemcpyAsync(roles, d.roles, (size_t)old * kMaxSlots, hipMemcpyDeviceToDevice, stream));
+    SVDAG_HIP(hipMemsetAsync(refs + (size_t)old * kMaxSlots, 0, (size_t)(newCap - old) * kMaxSlots * 4, stream));
+    SVDAG_HIP(hipMemsetAsync(roles + (size_t)old * kMaxSlots, 0, (size_t)(newCap - old) * kMaxSlots, stream));
     SVDAG_HIP(hipStreamSynchronize(stream));
     (void)hipFree(d.lines);
     (void)hipFree(d.freeList);
-    if (d.refs) {
-        (void)hipFree(d.refs);
-        (void)hipFree(d.roles);
-        d.refs = refs;
-        d.roles = roles;
-    }
+    (void)hipFree(d.refs);
+    (void)hipFree(d.roles);
     d.lines = lines;
     d.freeList = freeList;
+    d.refs = refs;
+    d.roles = roles;
     d.slabCap = newCap;
     t.slabCap = newCap;
     table_init_lines<<<grid_for((uint64_t)(newCap - old) * kLineWords, 256, 8192), 256, 0, stream>>>(d, old, newCap);

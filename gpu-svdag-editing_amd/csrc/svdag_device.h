@@ -127,7 +127,8 @@ struct TableDev {
     DevPtr<uint32_t> lines;     // [slabCap][32]: tags, next, items
     DevPtr<uint32_t> freeList;  // [slabCap] free stack of slab ids
     DevPtr<AllocState> alloc;
-    DevPtr<uint32_t> refs;      // DAG tables: [slabCap][16] stored references to each slot's item
+    DevPtr<uint32_t> refs;      // DAG tables: [slabCap][16] stored references to each slot's item;
+                                // null: a hash set's table, which has no free list either
     DevPtr<uint8_t> roles;      // DAG tables: [slabCap][16] kRoleParentOf* bits of each slot's item
     uint32_t itemWords;
     uint32_t numBuckets;
