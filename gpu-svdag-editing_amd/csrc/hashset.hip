@@ -812,10 +812,11 @@ int require_device()
 
 struct svdag_hashset {
     TableSet ts;
-    // One allocation holds every table (see hashset_tables): 17 tables of their
-    // own lines, free lists and states cost 51 allocations and as many
-    // synchronising frees, 4.4 of the 6.0 ms that filling, probing and releasing
-    // 3 M items of 2-18 words took.
+    // One allocation holds every table (see hashset_tables): making and
+    // releasing 17 tables with lines, free lists and states of their own took
+    // 51 allocations and 4.4 ms (3 M items of 2-18 words), 0.55 so.  In a
+    // process that has allocated and freed about the card's memory the driver
+    // takes longer to release the 0.5 GB: 7.9 then and 9.7 ms now.
     void* arena = nullptr;
     AllocState* states = nullptr; // [tables], in the arena
     hipStream_t stream = nullptr;
