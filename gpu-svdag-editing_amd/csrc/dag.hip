@@ -754,8 +754,10 @@ struct DedupShared {
 // This block's part (of `blocks`) of a level.
 template <bool kLeaf, int MW, uint32_t kBlock>
 __device__ inline void dedup_find_block(const WsDev& ws, const DagDev& dag, const TableDev* sTab, const LevelDesc& me,
-                                        uint32_t lg, uint32_t block, uint32_t blocks, DedupShared<kBlock>& sh)
+                                        uint32_t L, uint32_t lg, uint32_t block, uint32_t blocks,
+                                        DedupShared<kBlock>& sh)
 {
+    const uint8_t role = kLeaf ? kRoleLeafUse : node_role(dag, L);
     uint32_t (&sFirst)[2 * kBlock] = sh.first;
     uint32_t (&sHash)[kBlock] = sh.hash;
     uint32_t (&sRep)[kBlock] = sh.rep;
@@ -769,8 +771,9 @@ __device__ inline void dedup_find_block(const WsDev& ws, const DagDev& dag, cons
         // unchanged leaf: rep and handle were set by svo_leaf_level
         bool active = works && i < me.count && !(kLeaf && ws.created[w] == 2u);
         uint32_t n[MW];
-        uint32_t s = 0, h = 0;
+        uint32_t s = 0, h = 0, old = kSentinel;
         if (active) {
+            old = ws.work[w].w;
             lane_rec_load<MW>(n, kLeaf ? ws.leaves + (size_t)i * MW : ws.nodes + (size_t)w * kNodeStride);
             const bool empty = kLeaf ? (n[0] == 0u && n[1] == 0u) : ((n[0] & 0xFFu) == 0u);
             if (empty) {
@@ -839,11 +842,26 @@ __device__ inline void dedup_find_block(const WsDev& ws, const DagDev& dag, cons
             ws.rep[w] = rep;
             if (rep == w) {
                 // A node with a child this merge inserted is new: no find.
-                uint32_t r = kNotFound, hint = kNoSlab;
-                LineHead head;
-                if (kLeaf || n[MW - 1] == 0u)
-                    r = lane_find_hint<MW>(sTab[s - 2], n, s, h, hint, head);
-                ws.handle[w] = (r == kNotFound) ? kNotFound : (kLeaf ? leaf_handle(dag, r, s) : node_handle(r, s));
+                uint32_t r = kNotFound, hint = kNoSlab, found = kNotFound;
+                auto handle = [&] { return kLeaf ? leaf_handle(dag, r, s) : node_handle(r, s); };
+                if (kLeaf || n[MW - 1] == 0u) {
+                    const TableDev& t = sTab[s - 2];
+                    LineHead head;
+                    r = lane_find_hint<MW>(t, n, s, h, hint, head);
+                    // A found item of another role counts as a miss (the
+                    // reference-count rule in dag_internal.h); an equal one of
+                    // the right role may follow in the chain.  The item that
+                    // the DAG holds at this position has the position's role:
+                    // no role load.
+                    if (r != kNotFound && handle() != old) {
+                        const uint8_t roles = t.roles[r];
+                        if (kLeaf ? roles != 0u : (roles & role) == 0u)
+                            r = lane_find_hint<MW>(t, n, s, h, hint, head, role);
+                    }
+                    if (r != kNotFound)
+                        found = handle();
+                }
+                ws.handle[w] = found;
                 ws.created[w] = 0;
                 ws.hint[w] = hint;
             }
@@ -864,13 +882,15 @@ __global__ void __launch_bounds__(kMergeBlock) merge_dedup_find(WsDev ws, DagDev
     if (blockIdx.x * (kMergeBlock >> lg) >= me.count)
         return;
     tables_stage(sTab, dag);
-    dedup_find_block<kLeaf, MW, kMergeBlock>(ws, dag, sTab, me, lg, blockIdx.x, gridDim.x, sh);
+    dedup_find_block<kLeaf, MW, kMergeBlock>(ws, dag, sTab, me, L, lg, blockIdx.x, gridDim.x, sh);
 }
 
 // Insert the representatives the DAG did not hold (insertUniqueInHashTableAsWarp,
 // my_gpu_hash_dag_edits.cu:248-280).  All contents are distinct, so inserts
-// never race on equal items, and no find runs beside them except the one for
-// an equal item of another role.  Returns true when an item was inserted.
+// never race on equal items, and no find runs beside them: an insert claims a
+// slot's tag before it writes the item, and until then the slot holds the
+// words of whatever a collection freed there.  Returns true when an item was
+// inserted.
 //
 // Bound: dependent trips again (record, line, CAS, counts).  One lane per
 // item, as in the find: the leaf level of a 16-edit wave at depth 15 inserts
@@ -885,42 +905,15 @@ __device__ inline bool insert_item(const WsDev& ws, const DagDev& dag, const Tab
                                    uint32_t i, uint8_t role, BlockRefs<kSlots>& refs, uint32_t slotMask)
 {
     const uint32_t w = me.start + i;
-    const uint32_t rep = ws.rep[w], found = ws.handle[w];
-    uint32_t hint = ws.hint[w];
-    const uint32_t old = ws.work[w].w;
-    const uint8_t created = kLeaf ? ws.created[w] : 0u;
+    const uint32_t rep = ws.rep[w], found = ws.handle[w], hint = ws.hint[w];
     // The record is read along with what decides whether it is needed.
     uint32_t n[MW];
     lane_rec_load<MW>(n, kLeaf ? ws.leaves + (size_t)i * MW : ws.nodes + (size_t)w * kNodeStride);
-    if (rep != w)
+    if (rep != w || found != kNotFound)
         return false;
-    // A found node that lacks the role it is needed in counts as a miss
-    // (the reference-count rule in dag_internal.h).  A leaf the edit
-    // left unchanged (created 2) is the DAG's own leaf there: plain.
-    // The item the DAG holds at this position already has this position's
-    // role (unchanged leaves are that case too): no role load.
-    if (found != kNotFound) {
-        if (found == old)
-            return false;
-        if (kLeaf) {
-            if (created == 2u || sTab[leaf_handle_size(dag, found) - 2].roles[leaf_handle_ptr(dag, found)] == 0u)
-                return false;
-        } else if (sTab[node_handle_size(found) - 2].roles[node_handle_ptr(found)] & role) {
-            return false;
-        }
-    }
     const uint32_t s = kLeaf ? leaf_size_from_words(n[0], n[1], dag.M) : node_size_from_header(n[0]);
     const uint32_t h = lane_hash<MW>(n, s);
     const TableDev& t = sTab[s - 2];
-    if (found != kNotFound) {
-        // An equal item stored with the right role may follow in the chain.
-        LineHead head;
-        const uint32_t again = lane_find_hint<MW>(t, n, s, h, hint, head, kLeaf ? kRoleLeafUse : role);
-        if (again != kNotFound) {
-            ws.handle[w] = kLeaf ? leaf_handle(dag, again, s) : node_handle(again, s);
-            return false;
-        }
-    }
     const uint32_t r = lane_insert<MW>(t, n, s, h, hint);
     if (r == kNotFound) {
         atomicOr(&ws.status->oom, 1u);
@@ -1077,7 +1070,7 @@ __global__ void __launch_bounds__(kSmallBlock) merge_small(WsDev ws, DagDev dag,
                 (&sFull[0][0])[q] = 0u;
             __syncthreads();
             DedupShared<kSmallBlock>& ds = *reinterpret_cast<DedupShared<kSmallBlock>*>(&sh.word[0][0]);
-            dedup_find_block<false, (int)kNodeStride, kSmallBlock>(ws, dag, sTab, me, 0u, 0u, 1u, ds);
+            dedup_find_block<false, (int)kNodeStride, kSmallBlock>(ws, dag, sTab, me, (uint32_t)L, 0u, 0u, 1u, ds);
             __syncthreads();
             insert_block<false, (int)kNodeStride, kSmallBlock>(ws, dag, sTab, me, (uint32_t)L, 0u, 0u, 1u,
                                                                sh.refs[parity], sh.inserted);

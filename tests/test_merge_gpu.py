@@ -134,3 +134,47 @@ def test_a_large_level_above_a_small_one_matches_oracle(bits, lanes):
     st = g.garbage_collect()
     assert st.marked == 0 and g.garbage_collect(mark=True).items_freed == 0
     g.close()
+
+
+@pytest.mark.gpu
+def test_leaves_with_the_words_of_stored_nodes_get_their_own_items():
+    # At no material bits a leaf's two words can be those of a node with one
+    # child; a merge finds the node, which has another role, and must store
+    # the leaf beside it, once.
+    levels, side = 8, 64
+    rng = np.random.default_rng(4)
+    vox = np.full((side,) * 3, 0xFF, np.uint8)
+    for at in rng.choice(512, 60, replace=False):  # one leaf in a cell of 8: nodes of one child
+        x, y, z = (8 * v for v in (at // 64, at // 8 % 8, at % 8))
+        vox[x:x + 4, y:y + 4, z:z + 4][rng.random((4, 4, 4)) < 0.4] = 0
+    g = svdag_py.MyGPUHashDAG(levels, 0)
+    g.build_voxels(vox)
+    rec, p, twins = g.export_records(), 4, []
+    while p < len(rec):
+        size = int(rec[p + 2])
+        if rec[p] == levels - 3 and size == 2:
+            twins.append(int(rec[p + 3]) | int(rec[p + 4]) << 32)
+        p += 3 + size
+    assert len(twins) > 30
+    both = np.full((2 * side,) * 3, 0xFF, np.uint8)
+    both[:side, :side, :side] = vox
+    for k, bits in enumerate(twins * 2):  # each twice, as a leaf of the other half
+        x, y, z = side + 8 * (k % 8), side + 8 * (k // 8 % 8), side + 8 * (k // 64)
+        for b in range(64):
+            if bits >> b & 1:
+                both[x + (b >> 5 & 1) * 2 + (b >> 2 & 1), y + (b >> 4 & 1) * 2 + (b >> 1 & 1),
+                     z + (b >> 3 & 1) * 2 + (b & 1)] = 0
+    print("[case] leaves equal to nodes", flush=True)
+    o = oracle_py.OracleDag(levels, 0)
+    full = np.full((1 << levels,) * 3, 0xFF, np.uint8)
+    full[:2 * side, :2 * side, :2 * side] = both
+    oracle_py.build_dense(o, full)
+    for again in range(2):
+        g.build_voxels(both)
+        assert g.canonical() == o.canonical()
+        st = g.garbage_collect()
+        marked = g.garbage_collect(mark=True)
+        assert marked.items_freed == 0 and marked.items_live == st.items_live
+        live = st.items_live if not again else live
+        assert st.items_live == live
+    g.close()
