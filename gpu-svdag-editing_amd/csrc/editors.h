@@ -258,13 +258,6 @@ __device__ inline Op decide(const EditorDev& e, uint32_t x, uint32_t y, uint32_t
     }
 }
 
-__host__ __device__ inline bool aabb_overlap(const float lmn[3], const float lmx[3], const float rmn[3], const float rmx[3])
-{
-    return !(lmn[0] >= rmx[0] || lmn[1] >= rmx[1] || lmn[2] >= rmx[2] || lmx[0] <= rmn[0] || lmx[1] <= rmn[1]
-             || lmx[2] <= rmn[2] || rmn[0] >= lmx[0] || rmn[1] >= lmx[1] || rmn[2] >= lmx[2] || rmx[0] <= lmn[0]
-             || rmx[1] <= lmn[1] || rmx[2] <= lmn[2]);
-}
-
 // Rotated copy: source voxel of destination voxel v, k quarter turns of
 // R(x, y, z) = (-z - 1, y, x) (the turn about +Y that carries voxel cells
 // onto voxel cells) about the pivots, clamped at 0 per axis like the
@@ -358,7 +351,7 @@ __device__ inline Op decide_copy(const EditorDev& e, uint32_t x, uint32_t y, uin
                 bool ok;
                 if (e.rot) {
                     ok = (int64_t)cp >= clo[a] && (int64_t)cp <= chi[a];
-                } else { // one axis of aabb_overlap(child box, [smn, smx))
+                } else { // the child's extent and [smn, smx) on this axis overlap
                     const float cmn = (float)(cp << depth);
                     const float cmx = cmn + (float)(1u << depth);
                     ok = !(cmn >= smx[a] || cmx <= smn[a] || smn[a] >= cmx || smx[a] <= cmn);
